@@ -247,6 +247,8 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.gfr, 30 * nc);
     rc |= dalloc(c, &d.cprob, nc);
     rc |= dalloc(c, &d.gprob, cg);
+    rc |= dalloc(c, &d.gshort, cg);
+    rc |= dalloc(c, &d.cshort, nc);
     rc |= dalloc(c, &d.gorder, cg);
     rc |= dalloc(c, &d.cumL, cg);
     rc |= dalloc(c, &d.cumR, cg);
@@ -258,7 +260,6 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.pmu, np);
     rc |= dalloc(c, &d.pwl, np);
     rc |= dalloc(c, &d.pe, np);
-    rc |= dalloc(c, &d.pe0, np);
     rc |= dalloc(c, &d.pstat, np);
     rc |= dalloc(c, &d.pig, np);
     rc |= dalloc(c, &d.perr, np);

@@ -35,6 +35,17 @@ struct DdmcProb {
     double denom, t1, t2, t3;
 };
 
+// The same for the transport's short step: the event thresholds as 32-bit words compared with
+// a generator word (k_ddmc_probs), half the bytes of the FP64 record per random gather.
+struct ShortProb {              // an unlumped (cell, group): scatter above w3
+    double denom;
+    uint32_t w3, pad;
+};
+struct ShortCell {              // a cell's lumped step, and its divv
+    double denom, divv;
+    uint32_t w1, w2, w3, pad;
+};
+
 // Everything the kernels read or write, passed to kernels by value.
 struct Dev {
     int nx, ng, nep, nepg, nion, nel;
@@ -91,13 +102,15 @@ struct Dev {
     CellDDMC *cell;             // nc
     DdmcProb *cprob;            // nc     lumped-group step of each cell
     DdmcProb *gprob;            // nc*ng  unlumped step of each (cell, group), group-fastest
+    ShortProb *gshort;          // nc*ng  the short step's form of gprob
+    ShortCell *cshort;          // nc     and of cprob
     int *gorder;                // nc*ng  lumped groups ascending, then unlumped ascending
     double *cumL, *cumR, *cumD, *cumS;   // nc*ng cumulative lumped sampling weights
     uint32_t *btab;             // 5*nc*BT_K bucket maps of the cumL/R/D/S rows and emitgroup
     // particles (SoA)
     int64_t npart;
     const int64_t *pstart;      // nc+1
-    double *px, *pmu, *pwl, *pe, *pe0;
+    double *px, *pmu, *pwl, *pe;
     uint8_t *pstat;
     int *pig, *pix, *perr;
     int64_t *pnstep;

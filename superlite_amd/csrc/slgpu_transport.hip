@@ -98,14 +98,13 @@ __global__ __launch_bounds__(256) void k_sources(Dev d, uint32_t iteration)
     d.px[p] = x0;
     d.pmu[p] = mu;
     d.pe[p] = ep0;
-    d.pe0[p] = ep0;
     d.pwl[p] = wl0;
     if (guard >= (1 << 20)) atomicOr(d.flags, 1);
 }
 
 // ---------------------------------------------------------------------------
 struct Ptcl {
-    double x, mu, e, e0, wl, vx;
+    double x, mu, e, wl, vx;
     int ix, ig, itype, stat, idist;
     // for a DDMC particle: NF_VALID | BT_LUMP of its current (group, cell) when the step that
     // put it there knew them, so its next step needs no opacity load to pick its thresholds
@@ -119,6 +118,7 @@ constexpr uint32_t NF_VALID = 1u;
 enum { PEND_SCAT = 1, PEND_LEFT = 2, PEND_RIGHT = 3, PEND_DOP = 4 };
 constexpr uint32_t NF_PEND = 7u << 1;
 constexpr uint32_t NF_R2FREE = 1u << 4;
+constexpr uint32_t NF_FULL = 1u << 5;      // this DDMC step needs diffusion11, not the short step
 
 // TRANSPORT1/transport11.f90:86-489 (trn_noampfact = .true.)
 // Arithmetic of the precision form.  SLGPU_MIXED evaluates the sampled path lengths and
@@ -197,7 +197,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
 {
     const int ng = d.ng, nx = d.nx;
     int ix = p.ix, ig = p.ig;
-    double x = p.x, mu = p.mu, e = p.e, e0 = p.e0, wl = p.wl, vx = p.vx;
+    double x = p.x, mu = p.mu, e = p.e, wl = p.wl, vx = p.vx;
     int ic = ix;
     double r1, r2, db, dcol, dthm, ddop, dd;
     int ixnext;
@@ -290,13 +290,11 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
         const double help = elabfact / (1.0 - mu * vx * CINV);
         evelo = evelo + e * (1.0 - help);
         e = e * help;
-        e0 = e0 * help;
     } else if (dd == dcol) {
         r1 = s.draw();                 // unused draw (transport11.f90:313)
         const double help = elabfact / (1.0 - mu * vx * CINV);
         evelo = evelo + e * (1.0 - help);
         e = e * help;
-        e0 = e0 * help;
         if (ng != 1) {
             r1 = s.draw();
             int fl;
@@ -310,7 +308,6 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
         if (p.itype == 2) {
             evelo = evelo + e * vx * mu * CINV;
             e = e * (1.0 - vx * mu * CINV);
-            e0 = e0 * (1.0 - vx * mu * CINV);
         } else {
             r1 = s.draw();
             wl = 1.0 / ((1.0 - r1) * WLI(ig) + r1 * WLI(ig + 1));
@@ -337,7 +334,6 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
                 p.nflag = NF_VALID | lump_flag(d, CAPT(ig, l), DXX(ix + 1), l);
                 evelo = evelo + e * (1.0 - elabfact);
                 e = e * elabfact;
-                e0 = e0 * elabfact;
                 wl = wl / elabfact;
                 ix = ix + 1;
             } else {
@@ -364,7 +360,6 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
                 evelo = evelo - e * 2.0 * (0.55 * h - 1.25 * fabs(mu)) * vx * CINV;
                 eamp = e * 2.0 * 0.55 * (h - 2.0 > 0.0 ? h - 2.0 : 0.0) * vx * CINV;
                 h = h < 2.0 ? h : 2.0;
-                e0 = e0 * (1.0 + 2.0 * (0.55 * h - 1.25 * fabs(mu)) * vx * CINV);
                 e = e * (1.0 + 2.0 * (0.55 * h - 1.25 * fabs(mu)) * vx * CINV);
             }
             double help = (CAPT(ig, l) + SIGT(l)) * DXX(ix - 1);
@@ -375,7 +370,6 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
                 p.nflag = NF_VALID | lump_flag(d, CAPT(ig, l), DXX(ix - 1), l);
                 evelo = evelo + e * (1.0 - elabfact);
                 e = e * elabfact;
-                e0 = e0 * elabfact;
                 wl = wl / elabfact;
                 ix = ix - 1;
             } else {
@@ -412,14 +406,13 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
             p.nflag = NF_VALID | lump_flag(d, CAPT(ig, ic), DXX(ix), ic);
             evelo = evelo + e * vx * mu * CINV;
             e = e * elabfact;
-            e0 = e0 * elabfact;
             wl = wl / elabfact;
         }
     } else {
         ret = 17;
     }
 done:
-    p.x = x; p.mu = mu; p.e = e; p.e0 = e0; p.wl = wl; p.vx = vx;
+    p.x = x; p.mu = mu; p.e = e; p.wl = wl; p.vx = vx;
     p.ix = ix; p.ig = ig;
     return ret;
 }
@@ -482,6 +475,16 @@ __device__ __forceinline__ DdmcProb ddmc_prob(double opl, double opr, double emi
 // The per-event constants of diffusion11.f90:95-152 and 204-239 depend only on the cell
 // and, for an unlumped group, on the group; they are evaluated once per iteration here,
 // one thread per (group, cell), and the step loads them.
+// The short step's form of the thresholds.  The event draw is (m + 0.5) 2^-42 with a 42-bit m
+// whose upper 32 bits are a generator word w.  With T = floor(t 2^32), w < T gives draw < t and
+// w > T gives draw > t, exactly; w == T leaves the step to the full FP64 test.  A denominator
+// that is not a number (no threshold means anything then) sends every step there.
+__device__ __forceinline__ uint32_t word_threshold(double t)
+{
+    if (!(t > 0.0)) return 0u;
+    return t >= 1.0 ? 0xFFFFFFFFu : (uint32_t)(t * 4294967296.0);
+}
+
 __global__ __launch_bounds__(256) void k_ddmc_probs(Dev d)
 {
     const int ng = d.ng;
@@ -502,8 +505,25 @@ __global__ __launch_bounds__(256) void k_ddmc_probs(Dev d)
         doplump = 0.0;
     const double opl = (ix == 1) ? 0.0 : resleak_t(d, ix, ig, -1);
     const double opr = resleak_t(d, ix, ig, +1);
-    d.gprob[(size_t)(ic - 1) * ng + ig - 1] = ddmc_prob(opl, opr, emitlump, cp, doplump);
-    if (ig == 1) d.cprob[ic - 1] = ddmc_prob(OPL(1, ic), OPL(2, ic), cc.emitlump, cc.caplump, cc.doplump);
+    const DdmcProb q = ddmc_prob(opl, opr, emitlump, cp, doplump);
+    d.gprob[(size_t)(ic - 1) * ng + ig - 1] = q;
+    ShortProb sp;
+    sp.denom = q.t3 == q.t3 ? q.denom : q.t3;
+    sp.w3 = word_threshold(q.t3);
+    sp.pad = 0;
+    d.gshort[(size_t)(ic - 1) * ng + ig - 1] = sp;
+    if (ig == 1) {
+        const DdmcProb c = ddmc_prob(OPL(1, ic), OPL(2, ic), cc.emitlump, cc.caplump, cc.doplump);
+        d.cprob[ic - 1] = c;
+        ShortCell sc;
+        sc.denom = c.t3 == c.t3 ? c.denom : c.t3;
+        sc.divv = DIVV(ic);
+        sc.w1 = word_threshold(c.t1);
+        sc.w2 = word_threshold(c.t2);
+        sc.w3 = word_threshold(c.t3);
+        sc.pad = 0;
+        d.cshort[ic - 1] = sc;
+    }
 }
 
 void launch_ddmc_probs(slgpu_ctx *c)
@@ -526,7 +546,7 @@ __device__ int diffusion11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
     const int ng = d.ng, nx = d.nx;
     int ix = p.ix, ig = p.ig;
     const int ic = ix;
-    double x = p.x, mu = p.mu, e = p.e, e0 = p.e0, wl = p.wl, vx = p.vx;
+    double x = p.x, mu = p.mu, e = p.e, wl = p.wl, vx = p.vx;
     double r1;
     erd = 0.0; jrd = 0.0;
     const double dist = DXX(ix);
@@ -608,7 +628,6 @@ __device__ int diffusion11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
             evelo = evelo + e * (1.0 - help);
             wl = wl / help;
             e = e * help;
-            e0 = e0 * help;
             adiabatic = false;
         } else {
             // destination group and the cell whose optical depth decides IMC conversion
@@ -648,10 +667,9 @@ __device__ int diffusion11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
             const double f = p_adiabatic<M>(DIVV(ix), ddmct);
             evelo = evelo + e * (1.0 - f);
             e = e * f;
-            e0 = e0 * f;
         }
     }
-    p.x = x; p.mu = mu; p.e = e; p.e0 = e0; p.wl = wl; p.vx = vx;
+    p.x = x; p.mu = mu; p.e = e; p.wl = wl; p.vx = vx;
     p.ix = ix; p.ig = ig;
     return ret;
 }
@@ -676,7 +694,7 @@ __device__ void imc_entry(const Dev &d, Ptcl &p, const StepRng &s, uint32_t step
         return u;
     };
     const int ix = p.ix, ig = p.ig;
-    double x, mu, vx, e = p.e, e0 = p.e0, wl = p.wl;
+    double x, mu, vx, e = p.e, wl = p.wl;
     const bool face = kind == PEND_LEFT || kind == PEND_RIGHT;
     if (kind == PEND_SCAT) {
         const double r1 = next();
@@ -701,40 +719,28 @@ __device__ void imc_entry(const Dev &d, Ptcl &p, const StepRng &s, uint32_t step
     const double help = 1.0 / (1.0 - vx * mu * CINV);
     evelo = evelo + e * (1.0 - help);
     e = e * help;
-    e0 = e0 * help;
     wl = wl * (1.0 - vx * mu * CINV);
     evelo = evelo + e * (1.0 - f);
     e = e * f;
-    e0 = e0 * f;
-    p.x = x; p.mu = mu; p.vx = vx; p.e = e; p.e0 = e0; p.wl = wl;
+    p.x = x; p.mu = mu; p.vx = vx; p.e = e; p.wl = wl;
     p.nflag = NF_VALID | (p.nflag & BT_LUMP);
 }
 
 // Block totals in LDS, indexed like Dev::tot and Dev::ct.  Whatever changes once per
-// particle (its start, its end, the rare warnings and amplification energies) is added
-// here at once; only the per-step sums stay in registers (evelo, nddmc, nswap), which
-// keeps the persistent lane state small enough to avoid spilling.  The IMC step count is
-// the particles' total steps minus the DDMC steps.
+// particle or pass (its start, its end, conversions, the rare warnings and amplification
+// energies) is added here at once; only evelo, summed per step, stays in a register, which
+// keeps the persistent lane state small.  The DDMC step count is the particles' total steps
+// minus the IMC steps.
 struct BlockTotals {
     double tot[7];                 // eout, evelo, -, estart, edead, esrc, eamp
-    unsigned long long ct[9];      // nact, total steps (then nimc), nddmc, nmax, nswap,
+    unsigned long long ct[9];      // nact, nimc, total steps (then nddmc), nmax, nswap,
                                    // nflux, ndead, nerr, nwarn
 };
 
-__device__ __forceinline__ void flush_totals(const Dev &d, BlockTotals &b, double evelo,
-                                             uint32_t nddmc, uint32_t nswap)
+__device__ __forceinline__ void flush_totals(const Dev &d, BlockTotals &b, double evelo)
 {
     const double ev = wave_sum(evelo);
-    unsigned long long nd = nddmc, ns = nswap;
-    for (int off = 32; off > 0; off >>= 1) {
-        nd += __shfl_xor(nd, off, 64);
-        ns += __shfl_xor(ns, off, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        if (ev != 0.0) atomicAdd(&b.tot[1], ev);
-        atomicAdd(&b.ct[2], nd);
-        atomicAdd(&b.ct[4], ns);
-    }
+    if ((threadIdx.x & 63) == 0 && ev != 0.0) atomicAdd(&b.tot[1], ev);
     __syncthreads();
     if (threadIdx.x < 7) {
         const double v = b.tot[threadIdx.x];
@@ -742,63 +748,179 @@ __device__ __forceinline__ void flush_totals(const Dev &d, BlockTotals &b, doubl
     } else if (threadIdx.x >= 64 && threadIdx.x < 64 + 9) {
         const int q = threadIdx.x - 64;
         unsigned long long v = b.ct[q];
-        if (q == 1) v -= b.ct[2];                                // IMC steps
+        if (q == 2) v -= b.ct[1];                                // DDMC steps
         if (q == 3) atomicMax(&d.ct[3], v);
         else if (v) atomicAdd(&d.ct[q], v);
     }
 }
 
-// particle_advance.f90:140-294 as a persistent kernel: each lane takes the next particle
-// from a global counter, runs it event by event to escape or death (145-202 on start,
-// 271-292 at the end), then takes another, so lanes stay busy until the pool is empty.
-// Lanes that leave the loop drop out of the votes; a pass always runs the type of at
-// least one remaining lane, so every particle advances.
 // Occupancy target per precision (waves per SIMD), measured on c2: the precision form runs
 // best at 4 (VGPRs capped at 128), the FP64 form at 3 (capped at 168); the compiler's own
 // choice (2 and 3) is 6-11% slower.
-// A wave runs an IMC pass when n_imc * SLGPU_VOTE_IMC >= n_ddmc * SLGPU_VOTE_DDMC.  IMC
-// lanes wait out DDMC passes, so letting them go once they are a third of the live lanes
-// (2:1) beat a plain majority by 3-4% on c2 (1:2 and 4:1 were slower).
-#ifndef SLGPU_VOTE_IMC
-#define SLGPU_VOTE_IMC 2
-#endif
-#ifndef SLGPU_VOTE_DDMC
-#define SLGPU_VOTE_DDMC 1
-#endif
 #ifndef SLGPU_WAVES_MIXED
 #define SLGPU_WAVES_MIXED 4
 #endif
 #ifndef SLGPU_WAVES_FP64
 #define SLGPU_WAVES_FP64 3
 #endif
+// A wave runs short DDMC steps while at least this many eighths of its lanes take them: 2, 3
+// and 4 are within 4% of each other on c2 and c1, 5 and 6 are 10-40% slower (the lanes that
+// wait for a full or an IMC pass wait too long for company of their own kind).
+#ifndef SLGPU_RUN_EIGHTHS
+#define SLGPU_RUN_EIGHTHS 3
+#endif
+
+// What a lane's particle carries that the short step does not touch waits in LDS between
+// its full and IMC passes.
+struct Cold {
+    double x[256], mu[256], wl[256], vx[256];
+    double pend_f[256], pend_r2[256];          // a recorded conversion
+};
+
+__device__ __forceinline__ void cold_load(Ptcl &p, const Cold &s)
+{
+    const int t = threadIdx.x;
+    p.x = s.x[t]; p.mu = s.mu[t]; p.wl = s.wl[t]; p.vx = s.vx[t];
+}
+__device__ __forceinline__ void cold_store(const Ptcl &p, Cold &s)
+{
+    const int t = threadIdx.x;
+    s.x[t] = p.x; s.mu[t] = p.mu; s.wl[t] = p.wl; s.vx[t] = p.vx;
+}
+
+// The short DDMC step: one event of diffusion11.f90:243-620 that needs no more than a pure
+// bucket entry: an effective scatter, or a lumped particle's leak or Doppler shift inside the
+// mesh; the group, the cell and the optical-depth flags of the destination all come from the
+// entry.  These are 93% of the DDMC steps of the c2 workload.  A lane runs them back to back.
+// Per step it waits for one round trip to memory: a lumped particle's event follows from the
+// cell's thresholds (held in registers while the cell stays), so its entry comes from the
+// right table at once; an unlumped one requests its threshold and the effective-scatter entry
+// together.  The logarithm and the next step's Philox block are computed while they travel.
+// Any other step is left untouched for diffusion11 (NF_FULL).  The draws, the arithmetic and
+// the order of the sums are diffusion11's.  least: the lanes below which the wave leaves.
+// What bounds it is that round trip (1.1 us for a lane alone, in 160 KB of thresholds and 64 KB
+// of entries per cell and table).  Against a full diffusion11 pass per DDMC step, c2 (400 x 10^4) at 2^20
+// particles went from 3.69 to 2.87 s in the precision form and from 4.69 to 3.75 s in FP64.
+template <bool M>
+__device__ __forceinline__ void short_run(const Dev &d, Ptcl &p, uint32_t pid, uint32_t k0, uint32_t k1,
+                                          int64_t &istep, double &evelo, int &run_ic, double &run_e,
+                                          double *s_tally, double *jrad, Cold &cold, BlockTotals &bt,
+                                          int least)
+{
+    const uint32_t ng = d.ng, nx = d.nx;
+    uint32_t o[4];
+    Philox::block(pid, (uint32_t)(istep + 1), StepRng::PHASE, 0u, k0, k1, o);
+    ShortCell c = d.cshort[p.ix - 1], cn = c;                  // of the particle's cell, of the next
+    uint32_t wlg = 0;                                          // group edge a Doppler shift left wl at
+    bool go = true;
+    uint32_t t, ent, w3;
+    double denom;
+    auto request = [&]() {
+        const uint32_t ic = p.ix, w = o[1];
+        const bool lump = (p.nflag & BT_LUMP) != 0;
+        t = !lump ? TAB_E : (w > c.w3 ? TAB_S : (w < c.w1 ? TAB_D : (w < c.w2 ? TAB_L : TAB_R)));
+        ent = d.btab[((t * nx + (ic - 1)) << BT_BITS) + (o[2] >> (32 - BT_BITS))];
+        denom = c.denom;
+        w3 = c.w3;
+        if (!lump) {
+            const ShortProb q = d.gshort[(ic - 1) * ng + (p.ig - 1)];
+            denom = q.denom;
+            w3 = q.w3;
+        } else if (w == c.w1 || w == c.w2 || w == c.w3 || (t == TAB_L && ic == 1) || (t == TAB_R && ic == nx)) {
+            denom = __builtin_nan("");                         // undecided, or a face of the mesh
+        } else if (t == TAB_L || t == TAB_R) {
+            cn = d.cshort[t == TAB_L ? ic - 2 : ic];
+        }
+    };
+    request();
+    do {
+        const double lrt = p_log<M>(Philox::u42(o[0], o[3] & 0x3FFu));
+        const uint32_t w = o[1];
+        Philox::block(pid, (uint32_t)(istep + 2), StepRng::PHASE, 0u, k0, k1, o);
+        __builtin_amdgcn_sched_barrier(0);
+        if ((ent & BT_PURE) && denom == denom && (t != TAB_E || w > w3)) {
+            const uint32_t ic = p.ix;
+            const double ddmct = fabs(lrt * denom * CINV);
+            const double erd = p.e * ddmct, jrd = PC_C * erd;
+            if (jrd != 0.0) atomicAdd(jrad + ((ic - 1) * ng + (p.ig - 1)), jrd);
+            run_e += erd;
+            uint32_t g = ent & 0x7fffu, kind = PEND_SCAT;
+            if (t == TAB_D) {
+                kind = PEND_DOP;
+                wlg = c.divv >= 0 ? g + 1 : g;
+                g = c.divv >= 0 ? (g + 1 > ng ? ng : g + 1) : (g < 2 ? 1 : g - 1);
+            } else if (t <= TAB_R) {
+                kind = t == TAB_L ? PEND_LEFT : PEND_RIGHT;
+                atomicAdd(&s_tally[ic - 1], run_e);
+                run_e = 0.0;
+                p.ix = t == TAB_L ? ic - 1 : ic + 1;
+                c = cn;
+            }
+            p.ig = g;
+            ++istep;
+            const double f = p_adiabatic<M>(c.divv, ddmct);
+            if (ent & BT_THIN) {                               // conversion, at the next pass
+                p.itype = 1;
+                p.nflag = (kind << 1) | (ent & BT_LUMP);
+                cold.pend_f[threadIdx.x] = f;
+                atomicAdd(&bt.ct[4], 1ull);
+                go = false;
+            } else {
+                p.nflag = NF_VALID | (ent & BT_LUMP);
+                evelo = evelo + p.e * (1.0 - f);
+                p.e = p.e * f;
+            }
+        } else {
+            p.nflag |= NF_FULL;
+            go = false;
+        }
+        // max_steps belongs to the full step; leave when too few of the wave's lanes remain
+        go = go && istep + 1 < d.max_steps;
+        if (__popcll(__ballot(go)) < least) go = false;
+        if (go) request();
+    } while (go);
+    run_ic = p.ix;
+    if (wlg) cold.wl[threadIdx.x] = d.wl[wlg - 1];
+}
+
+// particle_advance.f90:140-294 as a persistent kernel: each lane takes the next particle
+// from a global counter, runs it event by event to escape or death (145-202 on start,
+// 271-292 at the end), then takes another, so lanes stay busy until the pool is empty.
+// Lanes that leave the loop drop out of the votes; a pass always runs the kind of at
+// least one remaining lane, so every particle advances.  lanes: how many lanes of a wave take
+// particles.  A pool smaller than the lanes resident on the chip is spread over all waves: its
+// time is the longest walk's, and a step costs a lane 1.9 us with one neighbour in its wave
+// against 3 us with 31 (8192 particles on c2: 1.34 s in full waves, 0.59 s spread).
 template <bool M>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(M ? SLGPU_WAVES_MIXED : SLGPU_WAVES_FP64, 8)))
-void k_transport(Dev d, uint32_t iteration)
+void k_transport(Dev d, uint32_t iteration, int lanes)
 {
     extern __shared__ double s_tally[];
     const int ng = d.ng, nx = d.nx;
     __shared__ BlockTotals bt;
-    __shared__ double s_pend_f[256], s_pend_r2[256];       // a lane's recorded conversion
+    __shared__ Cold cold;
     for (int k = threadIdx.x; k < nx; k += blockDim.x) s_tally[k] = 0.0;
     if (threadIdx.x < 7) bt.tot[threadIdx.x] = 0.0;
     if (threadIdx.x < 9) bt.ct[threadIdx.x] = 0;
     __syncthreads();
     double evelo = 0.0;
-    uint32_t nddmc = 0, nswap = 0;
     int run_ic = -1;
     double run_e = 0.0;
     double *jrad = d.jrad + (size_t)(blockIdx.x % d.jrad_copies) * nx * ng;
     Ptcl p;
     StepRng s;
     s.key(d.seed, iteration);
-    int64_t ip = -1, istep = 0;
+    uint32_t ip = 0;
+    int64_t istep = 0;
     bool have = false;
     for (;;) {
         if (!have) {
-            ip = (int64_t)atomicAdd(d.queue, 1ull);
-            if (ip >= d.npart) break;
-            p.x = d.px[ip]; p.mu = d.pmu[ip]; p.e = d.pe[ip]; p.e0 = d.pe0[ip]; p.wl = d.pwl[ip];
+            if ((int)(threadIdx.x & 63) >= lanes) break;
+            const int64_t next = (int64_t)atomicAdd(d.queue, 1ull);
+            if (next >= d.npart) break;
+            ip = (uint32_t)next;
+            p.x = d.px[ip]; p.mu = d.pmu[ip]; p.e = d.pe[ip]; p.wl = d.pwl[ip];
             atomicAdd(&bt.tot[5], p.e);
             atomicAdd(&bt.ct[0], 1ull);
             p.ix = binsrch(p.x, d.xarr, nx + 1, false);
@@ -817,40 +939,55 @@ void k_transport(Dev d, uint32_t iteration)
                 const double labfact = 1.0 - p.vx * p.mu / PC_C;
                 p.wl = p.wl * labfact;
                 p.e = p.e / labfact;
-                p.e0 = p.e0 / labfact;
             }
             atomicAdd(&bt.tot[3], p.e);
-            p.stat = 0;
-            p.idist = 0;
             p.nflag = 0;
-            s.init((uint32_t)ip);
+            cold_store(p, cold);
             istep = 0;
             have = true;
         }
-        // One event.  The wave runs one event type per pass, chosen by the vote above the
-        // kernel; lanes of the other type wait a pass, so each pass executes one body.
+        // The wave runs one kind of step per pass: short DDMC steps while they are enough of
+        // its lanes, else one IMC event or one full DDMC event, whichever more lanes wait for.
+        // The other lanes wait a pass, so each pass executes one body.
         const bool imc = p.itype == 1 || d.puretran;
-        const int n_imc = __popcll(__ballot(imc)), n_ddmc = __popcll(__ballot(!imc));
-        if (imc != (n_imc * SLGPU_VOTE_IMC >= n_ddmc * SLGPU_VOTE_DDMC)) continue;
+        const bool quick = !imc && (p.nflag & (NF_VALID | NF_FULL)) == NF_VALID && istep + 1 < d.max_steps;
+        const int n_imc = __popcll(__ballot(imc)), n_quick = __popcll(__ballot(quick));
+        const int live = __popcll(__ballot(1)), n_full = live - n_imc - n_quick;
+        const int least = (SLGPU_RUN_EIGHTHS * live + 7) / 8;
+        if (n_quick >= least) {
+            if (quick) {
+                if (p.ix != run_ic) {
+                    if (run_ic > 0) atomicAdd(&s_tally[run_ic - 1], run_e);
+                    run_ic = p.ix; run_e = 0.0;
+                }
+                short_run<M>(d, p, ip, s.k0, s.k1, istep, evelo, run_ic, run_e, s_tally, jrad, cold, bt, least);
+            }
+            continue;
+        }
+        if (quick || imc != (n_imc >= n_full)) continue;
         istep++;
+        cold_load(p, cold);
+        p.stat = 0;
+        p.idist = 0;
+        s.init(ip);
         if (imc && (p.nflag & NF_PEND))
-            imc_entry<M>(d, p, s, (uint32_t)(istep - 1), evelo, s_pend_f[threadIdx.x], s_pend_r2[threadIdx.x]);
+            imc_entry<M>(d, p, s, (uint32_t)(istep - 1), evelo, cold.pend_f[threadIdx.x], cold.pend_r2[threadIdx.x]);
         s.begin_step((uint32_t)istep);
         const int icold = p.ix, igold = p.ig;
         double erd, jrd;
         int ierr;
         if (imc) {
             double ea;
+            atomicAdd(&bt.ct[1], 1ull);
             ierr = transport11<M>(d, p, s, erd, jrd, ea, evelo);
             if (ea != 0.0) {                                   // particle_advance.f90:216-217
                 atomicAdd(&d.eamp[icold - 1], ea);
                 atomicAdd(&bt.tot[6], ea);
             }
-            if (p.itype != 1) nswap++;
+            if (p.itype != 1) atomicAdd(&bt.ct[4], 1ull);
         } else {
-            nddmc++;
-            ierr = diffusion11<M>(d, p, s, erd, jrd, evelo, s_pend_f[threadIdx.x], s_pend_r2[threadIdx.x]);
-            if (p.itype == 1) nswap++;
+            ierr = diffusion11<M>(d, p, s, erd, jrd, evelo, cold.pend_f[threadIdx.x], cold.pend_r2[threadIdx.x]);
+            if (p.itype == 1) atomicAdd(&bt.ct[4], 1ull);
         }
         // grd_jrad: one FP64 atomic per event into the block's replica (the group changes on
         // almost every step, so merging a particle's events would save no atomics); the
@@ -871,24 +1008,28 @@ void k_transport(Dev d, uint32_t iteration)
         if (ierr > 0) { atomicAdd(&bt.ct[7], 1ull); p.stat = 2; }
         if (p.stat != 0) {
             if (p.nflag & NF_PEND)                             // stopped by max_steps right after
-                imc_entry<M>(d, p, s, (uint32_t)istep, evelo, s_pend_f[threadIdx.x], s_pend_r2[threadIdx.x]);
+                imc_entry<M>(d, p, s, (uint32_t)istep, evelo, cold.pend_f[threadIdx.x], cold.pend_r2[threadIdx.x]);
             atomicMax(&bt.ct[3], (unsigned long long)istep);
-            atomicAdd(&bt.ct[1], (unsigned long long)istep);
+            atomicAdd(&bt.ct[2], (unsigned long long)istep);
             if (p.stat == 2) { atomicAdd(&bt.ct[6], 1ull); atomicAdd(&bt.tot[4], p.e); }
             else { atomicAdd(&bt.ct[5], 1ull); atomicAdd(&bt.tot[0], p.e); }
             d.pstat[ip] = (uint8_t)p.stat;
-            d.px[ip] = p.x; d.pmu[ip] = p.mu; d.pwl[ip] = p.wl; d.pe[ip] = p.e; d.pe0[ip] = p.e0;
+            d.px[ip] = p.x; d.pmu[ip] = p.mu; d.pwl[ip] = p.wl; d.pe[ip] = p.e;
             d.pig[ip] = p.ig; d.pix[ip] = p.ix;
             d.pnstep[ip] = istep;
             d.perr[ip] = ierr > 0 ? ierr : 0;
             have = false;
+        } else {
+            cold_store(p, cold);
+            // inside the innermost face every DDMC step ends the particle (diffusion11.f90:623-626)
+            if (p.itype == 2 && p.x < XA(1)) p.nflag |= NF_FULL;
         }
     }
     if (run_ic > 0) atomicAdd(&s_tally[run_ic - 1], run_e);
     __syncthreads();
     for (int k = threadIdx.x; k < nx; k += blockDim.x)
         if (s_tally[k] != 0.0) atomicAdd(&d.tally[k], s_tally[k]);
-    flush_totals(d, bt, evelo, nddmc, nswap);
+    flush_totals(d, bt, evelo);
 }
 
 // fluxtally.f:30-54 (flux grid == group grid; polar/azimuth bins are single)
@@ -918,15 +1059,16 @@ void launch_transport(slgpu_ctx *c, uint32_t iteration)
     int dev = 0, ncu = 256;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    int64_t blocks = (int64_t)ncu * 8;
-    const int64_t need = (c->d.npart + 255) / 256;
-    if (need < blocks) blocks = need > 0 ? need : 1;
+    const int64_t blocks = (int64_t)ncu * 8;
+    const int64_t resident = (int64_t)ncu * 4 * (c->d.precision == SLGPU_MIXED ? SLGPU_WAVES_MIXED : SLGPU_WAVES_FP64);
+    const int64_t share = (c->d.npart + resident - 1) / resident;
+    const int lanes = share < 1 ? 1 : (share > 64 ? 64 : (int)share);
     if (c->d.precision == SLGPU_MIXED)
         hipLaunchKernelGGL(k_transport<true>, dim3((unsigned)blocks), dim3(256),
-                           c->nx * sizeof(double), c->stream, c->d, iteration);
+                           c->nx * sizeof(double), c->stream, c->d, iteration, lanes);
     else
         hipLaunchKernelGGL(k_transport<false>, dim3((unsigned)blocks), dim3(256),
-                           c->nx * sizeof(double), c->stream, c->d, iteration);
+                           c->nx * sizeof(double), c->stream, c->d, iteration, lanes);
 }
 
 // the transport's group samplers at arbitrary (r, cell), table path or direct search
