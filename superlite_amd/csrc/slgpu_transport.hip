@@ -191,8 +191,31 @@ __device__ __forceinline__ double thomson_aniso_mu(double r1)
     return 1.0 - 2.0 * r1;
 }
 
+// What an IMC pass reads of its cell and group, requested together at the top of the pass:
+// the conversion that most passes begin with and the event then wait for one round trip
+// instead of one at each branch.
+struct ImcIn {
+    double xl, xr, vl, vr, sg, dvdr, c3, wi0, wi1;     // faces, their velocities, sigma_T, WLI(ig), WLI(ig+1)
+    float cp, cpup, cpdn;                              // gas_cap of the group and of its two neighbours
+};
+
+__device__ __forceinline__ void imc_request(const Dev &d, const Ptcl &p, ImcIn &q)
+{
+    const int ng = d.ng, ix = p.ix, ig = p.ig;
+    const float *row = d.cap32 + (size_t)(ix - 1) * ng;
+    q.cp = row[ig - 1];
+    q.cpup = row[ig < ng ? ig : ig - 1];
+    q.cpdn = row[ig > 1 ? ig - 2 : ig - 1];
+    q.wi0 = WLI(ig); q.wi1 = WLI(ig + 1);
+    q.xl = XA(ix); q.xr = XA(ix + 1);
+    q.vl = VXA(ix); q.vr = VXA(ix + 1);
+    q.sg = SIGT(ix);
+    q.dvdr = d.dvdr[ix - 1];
+    q.c3 = d.c3divv[ix - 1];
+}
+
 template <bool M>
-__device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, double &jrd,
+__device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, double &erd, double &jrd,
                            double &eamp, double &evelo)
 {
     const int ng = d.ng, nx = d.nx;
@@ -204,7 +227,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
     erd = 0.0; jrd = 0.0; eamp = 0.0;
     double elabfact = 1.0 - mu * vx * CINV;
     const double elabfactold = elabfact;
-    const double xl = XA(ix), xr = XA(ix + 1);
+    const double xl = q.xl, xr = q.xr;
     const double far = 2.0 * fabs(sqrt(xr * xr - xl * xl));
     if (ix == 1 || mu >= -sqrt(1.0 - (xl / x) * (xl / x))) {
         db = fabs(sqrt(xr * xr - (1.0 - mu * mu) * x * x) - mu * x);
@@ -213,14 +236,17 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
         db = fabs(sqrt(xl * xl - (1.0 - mu * mu) * x * x) + mu * x);
         ixnext = ix - 1;
     }
+    // the neighbour cell, for an event at the face
+    const int nb = ixnext < 1 ? 1 : (ixnext > nx ? nx : ixnext);
+    const double cap_nb = CAPT(ig, nb), sig_nb = SIGT(nb), dx_nb = DXX(nb);
     if (db != db) return 1;
-    const double sg = SIGT(ic), cp = CAPT(ig, ic);
+    const double sg = q.sg, cp = (double)q.cp;
     if (sg > 0.0) { r1 = s.draw(); dthm = p_path<M>(r1, elabfact * sg); }
     else dthm = far;
     if (cp <= 0.0) dcol = far;
     else { r1 = s.draw(); dcol = p_path<M>(r1, elabfact * cp); }
-    const double dvdr = d.dvdr[ix - 1];
-    const double vhelp = VXA(ix) - dvdr * xl;
+    const double dvdr = q.dvdr;
+    const double vhelp = q.vl - dvdr * xl;
     if (fabs(vx - vhelp) / PC_C >= 0.1) {
         // Newton-Raphson Doppler distance (transport11.f90:159-199)
         const double epstol = 1e-3;
@@ -228,7 +254,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
         double shelp = db;
         double xhelp = sqrt(x * x + shelp * shelp + 2.0 * shelp * x * mu);
         double muhelp = (mu * x + shelp) / xhelp;
-        double phi = dvdr * mu * x - PC_C * (1 - wl * WLI(ig + 1)) + vhelp * muhelp + dvdr * shelp;
+        double phi = dvdr * mu * x - PC_C * (1 - wl * q.wi1) + vhelp * muhelp + dvdr * shelp;
         double dphi = dvdr + vhelp * (1 - muhelp * muhelp) / xhelp;
         ddop = shelp - phi / dphi;
         while ((fabs(ddop - shelp) > ddop * epstol) && it < 100) {
@@ -237,17 +263,17 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
             xhelp = sqrt(x * x + shelp * shelp + 2.0 * shelp * x * mu);
             muhelp = (mu * x + shelp) / xhelp;
             if (dvdr > 0 && ig < ng)
-                phi = dvdr * mu * x - PC_C * (1 - wl * WLI(ig + 1)) + vhelp * muhelp + dvdr * shelp;
+                phi = dvdr * mu * x - PC_C * (1 - wl * q.wi1) + vhelp * muhelp + dvdr * shelp;
             else if (dvdr < 0 && ig > 1)
-                phi = dvdr * mu * x - PC_C * (1 - wl * WLI(ig)) + vhelp * muhelp + dvdr * shelp;
+                phi = dvdr * mu * x - PC_C * (1 - wl * q.wi0) + vhelp * muhelp + dvdr * shelp;
             else { ddop = far; break; }
             dphi = dvdr + vhelp * (1 - muhelp * muhelp) / xhelp;
             ddop = shelp - phi / dphi;
         }
         if (ddop <= 0.0 || it == 100) ddop = far;
     } else {
-        if (dvdr > 0 && ig < ng) ddop = d.c3divv[ix - 1] * (elabfact - wl * WLI(ig + 1));
-        else if (dvdr < 0 && ig > 1) ddop = d.c3divv[ix - 1] * (elabfact - wl * WLI(ig));
+        if (dvdr > 0 && ig < ng) ddop = q.c3 * (elabfact - wl * q.wi1);
+        else if (dvdr < 0 && ig > 1) ddop = q.c3 * (elabfact - wl * q.wi0);
         else ddop = far;
         if (ddop < 0.0) ddop = far;
     }
@@ -262,7 +288,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
     if (dd < 0.0) return 4;
     const double xold = x;
     x = sqrt(x * x + dd * dd + 2.0 * dd * x * mu);
-    vx = (VXA(ix) * (xr - x) + VXA(ix + 1) * (x - xl)) / DXX(ix);
+    vx = (q.vl * (xr - x) + q.vr * (x - xl)) / (xr - xl);
     if (x == 0.0) mu = 1.0;
     else mu = (xold * mu + dd) / x;
     erd = e * elabfact * elabfact * dd * CINV;
@@ -320,18 +346,18 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
         goto done;
     } else if (dd == db && ixnext > ix) {
         const int l = ix + 1;
-        if ((SIGT(l) + CAPT(ig, l)) * DXX(ix + 1) < d.tauddmc || d.puretran) {
-            x = XA(ix + 1);
-            vx = VXA(ix + 1);
+        if ((sig_nb + cap_nb) * dx_nb < d.tauddmc || d.puretran) {
+            x = xr;
+            vx = q.vr;
             ix = ix + 1;
         } else {
             mu = (mu - vx * CINV) / (1.0 - vx * mu * CINV);
-            double help = (CAPT(ig, l) + SIGT(l)) * DXX(ix + 1);
+            double help = (cap_nb + sig_nb) * dx_nb;
             help = 4.0 / (3.0 * help + 6.0 * PC_DEXT);
             r1 = s.draw();
             if (r1 < help * (1.0 + 1.5 * fabs(mu))) {
                 p.itype = 2;
-                p.nflag = NF_VALID | lump_flag(d, CAPT(ig, l), DXX(ix + 1), l);
+                p.nflag = NF_VALID | lump_flag(d, cap_nb, dx_nb, l);
                 evelo = evelo + e * (1.0 - elabfact);
                 e = e * elabfact;
                 wl = wl / elabfact;
@@ -341,15 +367,15 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
                 r2 = s.draw();
                 mu = -(r1 > r2 ? r1 : r2);
                 mu = (mu + vx * CINV) / (1.0 + vx * mu * CINV);
-                x = XA(ix + 1);
-                vx = VXA(ix + 1);
+                x = xr;
+                vx = q.vr;
             }
         }
     } else if (dd == db) {
         const int l = ix - 1;
-        if ((SIGT(l) + CAPT(ig, l)) * DXX(ix - 1) < d.tauddmc || d.puretran) {
-            x = XA(ix);
-            vx = VXA(ix);
+        if ((sig_nb + cap_nb) * dx_nb < d.tauddmc || d.puretran) {
+            x = xl;
+            vx = q.vl;
             ix = ix - 1;
         } else {
             mu = (mu - vx * CINV) / (1.0 - vx * mu * CINV);
@@ -362,12 +388,12 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
                 h = h < 2.0 ? h : 2.0;
                 e = e * (1.0 + 2.0 * (0.55 * h - 1.25 * fabs(mu)) * vx * CINV);
             }
-            double help = (CAPT(ig, l) + SIGT(l)) * DXX(ix - 1);
+            double help = (cap_nb + sig_nb) * dx_nb;
             help = 4.0 / (3.0 * help + 6.0 * PC_DEXT);
             r1 = s.draw();
             if (r1 < help * (1.0 + 1.5 * fabs(mu))) {
                 p.itype = 2;
-                p.nflag = NF_VALID | lump_flag(d, CAPT(ig, l), DXX(ix - 1), l);
+                p.nflag = NF_VALID | lump_flag(d, cap_nb, dx_nb, l);
                 evelo = evelo + e * (1.0 - elabfact);
                 e = e * elabfact;
                 wl = wl / elabfact;
@@ -377,14 +403,16 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
                 r2 = s.draw();
                 mu = r1 > r2 ? r1 : r2;
                 mu = (mu + vx * CINV) / (1.0 + vx * mu * CINV);
-                x = XA(ix);
-                vx = VXA(ix);
+                x = xl;
+                vx = q.vl;
             }
         }
     } else if (dd == ddop) {
+        double cnew = (double)q.cp;
         if (dvdr > 0) {
             if (ig < ng) {
                 ig = ig + 1;
+                cnew = (double)q.cpup;
                 wl = (WLG(ig) + 1e-6 * (WLG(ig + 1) - WLG(ig))) * elabfactold;
             } else {
                 r1 = s.draw();
@@ -395,15 +423,16 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
             if (ig > 1) {
                 wl = (WLG(ig) + 1e-6 * (WLG(ig - 1) - WLG(ig))) * elabfactold;
                 ig = ig - 1;
+                cnew = (double)q.cpdn;
             } else {
                 r1 = s.draw();
                 wl = 1.0 / (r1 * WLI(1) + (1.0 - r1) * WLI(2));
                 wl = wl * elabfact;
             }
         }
-        if (((SIGT(ic) + CAPT(ig, ic)) * DXX(ix) >= d.tauddmc) && !d.puretran) {
+        if (((sg + cnew) * (xr - xl) >= d.tauddmc) && !d.puretran) {
             p.itype = 2;
-            p.nflag = NF_VALID | lump_flag(d, CAPT(ig, ic), DXX(ix), ic);
+            p.nflag = NF_VALID | lump_flag(d, cnew, xr - xl, ic);
             evelo = evelo + e * vx * mu * CINV;
             e = e * elabfact;
             wl = wl / elabfact;
@@ -448,9 +477,8 @@ __device__ __forceinline__ double resleak_t(const Dev &d, int ix, int g, int sid
 
 // uniform position in the shell with the single-precision 1/3 exponent, clamped (:336-339)
 template <bool M>
-__device__ __forceinline__ double shell_position(const Dev &d, int ix, double r1)
+__device__ __forceinline__ double shell_position(double xl, double xr, double r1)
 {
-    const double xl = XA(ix), xr = XA(ix + 1);
     double x = p_shell_root<M>(r1, xl, xr);
     x = x > xr ? xr : x;
     x = x < xl ? xl : x;
@@ -679,8 +707,8 @@ __device__ int diffusion11(const Dev &d, Ptcl &p, StepRng &s, double &erd, doubl
 // step's adiabatic factor f, in the reference's order.  Its draws are that step's: draw 2 when
 // it was still unused (r2), then draws 3.. (block 1 of the step).
 template <bool M>
-__device__ void imc_entry(const Dev &d, Ptcl &p, const StepRng &s, uint32_t step, double &evelo,
-                          double f, double r2)
+__device__ void imc_entry(const Dev &d, Ptcl &p, const StepRng &s, const ImcIn &q, uint32_t step,
+                          double &evelo, double f, double r2)
 {
     const uint32_t kind = (p.nflag & NF_PEND) >> 1;
     bool r2_free = (p.nflag & NF_R2FREE) != 0;
@@ -693,27 +721,25 @@ __device__ void imc_entry(const Dev &d, Ptcl &p, const StepRng &s, uint32_t step
         ++j;
         return u;
     };
-    const int ix = p.ix, ig = p.ig;
     double x, mu, vx, e = p.e, wl = p.wl;
     const bool face = kind == PEND_LEFT || kind == PEND_RIGHT;
     if (kind == PEND_SCAT) {
         const double r1 = next();
-        wl = 1.0 / ((1.0 - r1) * WLI(ig) + r1 * WLI(ig + 1));
+        wl = 1.0 / ((1.0 - r1) * q.wi0 + r1 * q.wi1);
     } else if (face) {
         const double r1 = next();
-        wl = 1.0 / (r1 * WLI(ig + 1) + (1.0 - r1) * WLI(ig));
+        wl = 1.0 / (r1 * q.wi1 + (1.0 - r1) * q.wi0);
     }
     const double ra = next(), rb = next();
     if (face) {
-        const int xi = kind == PEND_LEFT ? ix + 1 : ix;      // the face crossed into cell ix
-        x = XA(xi);
-        vx = VXA(xi);
+        x = kind == PEND_LEFT ? q.xr : q.xl;                  // the face crossed into cell ix
+        vx = kind == PEND_LEFT ? q.vr : q.vl;
         mu = ra > rb ? ra : rb;
         if (kind == PEND_LEFT) mu = -mu;
     } else {
         mu = 1.0 - 2.0 * ra;
-        x = shell_position<M>(d, ix, rb);
-        vx = (VXA(ix) * (XA(ix + 1) - x) + VXA(ix + 1) * (x - XA(ix))) / DXX(ix);
+        x = shell_position<M>(q.xl, q.xr, rb);
+        vx = (q.vl * (q.xr - x) + q.vr * (x - q.xl)) / (q.xr - q.xl);
     }
     mu = (mu + vx * CINV) / (1.0 + vx * mu * CINV);
     const double help = 1.0 / (1.0 - vx * mu * CINV);
@@ -970,8 +996,10 @@ void k_transport(Dev d, uint32_t iteration, int lanes)
         p.stat = 0;
         p.idist = 0;
         s.init(ip);
+        ImcIn q;
+        if (imc) imc_request(d, p, q);
         if (imc && (p.nflag & NF_PEND))
-            imc_entry<M>(d, p, s, (uint32_t)(istep - 1), evelo, cold.pend_f[threadIdx.x], cold.pend_r2[threadIdx.x]);
+            imc_entry<M>(d, p, s, q, (uint32_t)(istep - 1), evelo, cold.pend_f[threadIdx.x], cold.pend_r2[threadIdx.x]);
         s.begin_step((uint32_t)istep);
         const int icold = p.ix, igold = p.ig;
         double erd, jrd;
@@ -979,7 +1007,7 @@ void k_transport(Dev d, uint32_t iteration, int lanes)
         if (imc) {
             double ea;
             atomicAdd(&bt.ct[1], 1ull);
-            ierr = transport11<M>(d, p, s, erd, jrd, ea, evelo);
+            ierr = transport11<M>(d, p, s, q, erd, jrd, ea, evelo);
             if (ea != 0.0) {                                   // particle_advance.f90:216-217
                 atomicAdd(&d.eamp[icold - 1], ea);
                 atomicAdd(&bt.tot[6], ea);
@@ -1007,8 +1035,10 @@ void k_transport(Dev d, uint32_t iteration, int lanes)
         if (ierr == 0 && p.stat == 0 && istep >= d.max_steps) ierr = 200;
         if (ierr > 0) { atomicAdd(&bt.ct[7], 1ull); p.stat = 2; }
         if (p.stat != 0) {
-            if (p.nflag & NF_PEND)                             // stopped by max_steps right after
-                imc_entry<M>(d, p, s, (uint32_t)istep, evelo, cold.pend_f[threadIdx.x], cold.pend_r2[threadIdx.x]);
+            if (p.nflag & NF_PEND) {                           // stopped by max_steps right after
+                imc_request(d, p, q);
+                imc_entry<M>(d, p, s, q, (uint32_t)istep, evelo, cold.pend_f[threadIdx.x], cold.pend_r2[threadIdx.x]);
+            }
             atomicMax(&bt.ct[3], (unsigned long long)istep);
             atomicAdd(&bt.ct[2], (unsigned long long)istep);
             if (p.stat == 2) { atomicAdd(&bt.ct[6], 1ull); atomicAdd(&bt.tot[4], p.e); }
