@@ -213,7 +213,6 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.ffB, (size_t)nc * FF_NU);
     rc |= dalloc(c, &d.ffclamp, nc);
     rc |= dalloc(c, &d.ffC, (size_t)nc * FF_NU);
-    rc |= dalloc(c, &d.ffW, (size_t)nc * FF_NU);
     rc |= dalloc(c, &d.sig, nc);
     rc |= dalloc(c, &d.tempinv, nc);
     rc |= dalloc(c, &d.temp, nc);
@@ -241,10 +240,8 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.vol_in, nc);
     rc |= dalloc(c, &d.nelec_in, nc);
     rc |= dalloc(c, &d.gcapT, cg);
-    rc |= dalloc(c, &d.gcell, 4 * nc);
     rc |= dalloc(c, &d.gmpart, (size_t)2 * ((ng + 63) / 64) * nc);
     rc |= dalloc(c, &d.ctpart, (size_t)2 * ((ng + 1023) / 1024) * nc);
-    rc |= dalloc(c, &d.gfr, 30 * nc);
     rc |= dalloc(c, &d.cprob, nc);
     rc |= dalloc(c, &d.gprob, cg);
     rc |= dalloc(c, &d.gshort, cg);
@@ -353,6 +350,7 @@ int slgpu_set_grid(slgpu_ctx *c, const double *xarr, const double *vxarr, const 
 }
 
 static int upload_lines(slgpu_ctx *c);
+static int build_lines64(slgpu_ctx *c);
 static int build_bfxs(slgpu_ctx *c);
 
 int slgpu_set_groups(slgpu_ctx *c, const double *wl)
@@ -396,18 +394,23 @@ int slgpu_set_ions(slgpu_ctx *c, int nion, const int *ion_iz, const int *ion_ii)
     dfree(c, c->d.ginvT);
     dfree(c, c->d.goc);
     dfree(c, (void *)c->d.bfxs);
+    dfree(c, c->d.bfmask);
     const size_t nc = c->nx;
     int rc = 0;
     rc |= dalloc(c, &c->d.ocg, (size_t)std::max(nion, 1) * nc);
     rc |= dalloc(c, &c->d.ginvT, (size_t)std::max(nion, 1) * nc);
-    rc |= dalloc(c, &c->d.goc, (size_t)std::max(nion, 1) * nc);
+    rc |= dalloc(c, &c->d.goc, vjp_acc_doubles(nion, nc));
     rc |= dalloc(c, &c->d.ocT, (size_t)(nion + 30) * nc);     // tail: ff coordinates per element
     rc |= dalloc(c, (double **)&c->d.bfxs, (size_t)std::max(nion, 1) * c->ng);
+    rc |= dalloc(c, &c->d.bfmask, (size_t)(std::max(nion, 1) + 31) / 32 * c->ng);
     rc |= dalloc(c, &c->d.ion_z, std::max(nion, 1));
     rc |= dalloc(c, &c->d.ion_i, std::max(nion, 1));
     rc |= dalloc(c, &c->eos_oc, (size_t)std::max(nion, 1) * nc);
     rc |= dalloc(c, &c->eos_ginv, (size_t)std::max(nion, 1) * nc);
     if (rc) return rc;
+    c->d.ffW = c->d.goc + (size_t)GACC_COPIES * std::max(nion, 1) * nc;
+    c->d.gcell = c->d.ffW + (size_t)GACC_COPIES * FF_NU * nc;
+    c->d.gfr = c->d.gcell + 2 * nc;
     if (nion > 0) {
         HIPCHK(hipMemcpyAsync(c->d.ion_z, ion_iz, nion * sizeof(int), hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipMemcpyAsync(c->d.ion_i, ion_ii, nion * sizeof(int), hipMemcpyHostToDevice, c->stream));
@@ -481,6 +484,9 @@ static int upload_lines(slgpu_ctx *c)
     dfree(c, (void *)c->d.lines);
     dfree(c, (void *)c->d.lines_ion);
     dfree(c, (void *)c->d.gstart);
+    dfree(c, c->d.lines64);
+    c->d.lines64 = nullptr;
+    c->d.line_step = 0.0;
     int rc = 0;
     rc |= dalloc(c, (LineRec **)&c->d.lines, recs.size());
     rc |= dalloc(c, (LineRec **)&c->d.lines_ion, recs.size());
@@ -494,7 +500,33 @@ static int upload_lines(slgpu_ctx *c)
     }
     HIPCHK(hipMemcpyAsync((void *)c->d.gstart, gstart.data(), (ng + 2) * sizeof(int),
                           hipMemcpyHostToDevice, c->stream));
+    // largest lower level, and whether every line suits the exponential tables
+    double top = 0.0;
+    bool plain = true;
+    for (const LineRec &q : recs) {
+        plain = plain && q.chilw >= 0.0f && std::isfinite(q.chilw) && std::isfinite(q.gxs);
+        top = std::max(top, (double)q.chilw);
+    }
+    c->line_top = plain && !recs.empty() ? std::max(top, 1.0) : 0.0;
+    if (c->cfg.precision == SLGPU_FP64) rc = build_lines64(c);
     HIPCHK(hipStreamSynchronize(c->stream));
+    return rc;
+}
+
+// The FP64 line sums' records and tables (FP64 builds and NLTE builds).  The step is the largest
+// lower level over the table's range, rounded up to a multiple of 1/16 so that every split is exact;
+// lists with negative or non-finite records keep exp() per line.
+static int build_lines64(slgpu_ctx *c)
+{
+    if (!(c->line_top > 0.0) || c->d.line_step > 0.0) return 0;
+    const double step = std::ceil(c->line_top / (EXP_K1 * EXP_K2 - 1) * 16.0) / 16.0;
+    if (step > 1e6) return 0;
+    int rc = dalloc(c, &c->d.lines64, c->nline_used);
+    if (!rc && !c->d.etab) rc = dalloc(c, &c->d.etab, (size_t)EXP_ROWS * c->nx);
+    if (rc) return rc;
+    c->d.line_step = step;
+    launch_lines64(c, c->nline_used);
+    HIPCHK(hipGetLastError());
     return 0;
 }
 
@@ -568,6 +600,8 @@ int opacity_build_impl(slgpu_ctx *c, const slgpu_gas *gas, int flags, double *ou
         if (any) elz[nel++] = z;
     }
     c->d.nel = nel;
+    c->hckt_max = 0.0;
+    for (int i = 0; i < nc; ++i) c->hckt_max = std::max(c->hckt_max, PC_H * PC_C / (PC_KB * gas->temp[i]));
     PhaseTimer tm(c, 0);
     // per-call host inputs (small: nc and nion*nc doubles)
     double *dn = c->d.natom_in, *dv = c->d.vol_in, *de = c->d.nelec_in;   // kept for the backward

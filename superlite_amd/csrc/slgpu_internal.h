@@ -20,6 +20,16 @@ struct LineRec {
     int pad;        // in the ion-ordered copy: lines left in this record's ion run
 };
 
+// A line of the FP64 line sums, in ion order within its group: its lower level split over the
+// rows of the cell's exponential tables, chi = (EXP_K2 k1 + k2) step + r (k_opacity64).
+struct Line64 {
+    double gxs, r;
+    uint32_t k1, k2;    // byte offsets of the rows k1 and EXP_K1 + k2, 512 bytes a row
+    uint32_t ion;       // 512 times the ion index, plus 1 on the last line of its run
+    float chi;
+};
+constexpr int EXP_K1 = 32, EXP_K2 = 32, EXP_ROWS = EXP_K1 + EXP_K2;
+
 // Per-cell DDMC constants (diffusion11.f90:95-152), evaluated once per iteration.
 struct CellDDMC {
     double emgreyinv;   // 1/capgrey (LTE) or 1/capemitgrey (NLTE), nan -> 0
@@ -62,9 +72,13 @@ struct Dev {
     // lines
     const LineRec *lines;
     const LineRec *lines_ion;   // the same records, sorted by ion within each group (backward)
+    Line64 *lines64;            // the records of the FP64 line sums, in lines_ion's order
+    double *etab;               // EXP_ROWS*nc: the cells' exponential tables, cell fastest
+    double line_step;           // the tables' fine step [1/cm]; 0: no tables (see build_lines64)
     const int *gstart;          // ng+2: lines of group g (1-based) are [gstart[g], gstart[g+1])
     // tables
     double *bfxs;               // ng*nion, xs(ig, k)*1e-18 (Mb -> cm^2)
+    uint32_t *bfmask;           // ng*((nion+31)/32): which of a group's bfxs are not zero
     const double *gff;          // 81*41 Fortran order
     // per-iteration gas state (cell-fastest, [k*nc + i])
     double *hckt, *hlparr, *ocg, *ocT, *sig, *tempinv, *temp, *mass, *natomfr;
@@ -78,8 +92,6 @@ struct Dev {
     double *ctpart;                       // 2*((ng+1023)/1024)*nx: the means' per-slice partial sums
     double *gmpart;                       // 2*((ng+63)/64)*nx: the means backward's per-tile
                                           // partial sums of dL/dT and dL/dsig
-    double *ffW;                          // FF_NU*nx: backward, sum over groups of G*help spread
-                                          // onto the two u nodes of each group
     int *el_z;                  // nel present elements (ascending iz)
     // opacity products
     double *capT;               // ng*nc cell-fastest scratch
@@ -119,8 +131,12 @@ struct Dev {
     double *natom_in, *vol_in, *nelec_in; // nc
     double *ginvT;                        // nion*nc (ion-major)
     double *gcapT;                        // ng*nc cell-fastest dL/dcap after the means
-    double *gcell;                        // 4*nc: dL/dT (means), dL/dsig, dL/dhckt, dL/dhlparr
-    double *gfr, *goc;                    // 30*nc, nion*nc element- / ion-major
+    // the backward's accumulators, one allocation in this order (vjp_acc_doubles)
+    double *goc;                          // GACC_COPIES*nion*nc ion-major
+    double *ffW;                          // GACC_COPIES*FF_NU*nc: sum over groups of G*help spread
+                                          // onto the two u nodes of each group
+    double *gcell;                        // 2*nc: dL/dhckt, dL/dhlparr
+    double *gfr;                          // 30*nc element-major
     double *tally, *jrad, *tot;           // nc, jrad_copies*nc*ng, 8
     double *eamp;                         // nc grd_eamp
     int jrad_copies;                      // replicas of grd_jrad that spread atomic traffic
@@ -155,6 +171,12 @@ struct NlteDev {
     double *capemitgrey;                        // nc
 };
 
+constexpr int GACC_COPIES = 8;          // copies of the backward's most contended accumulators
+inline size_t vjp_acc_doubles(int nion, size_t nc)
+{
+    return ((size_t)GACC_COPIES * ((nion > 1 ? nion : 1) + FF_NU) + 2 + 30) * nc;
+}
+
 struct Timer {
     hipEvent_t a, b;
     bool armed = false;
@@ -179,6 +201,8 @@ struct slgpu_ctx {
     std::vector<int16_t> h_liz, h_lii;
     std::vector<float> h_gxs, h_chilw;
     std::vector<double> h_emit_cache;
+    double line_top = 0.0;      // largest lower level of the used lines [1/cm]; 0: no tables
+    double hckt_max = 0.0;      // largest hc/kT of the last build's cells
     int opac_flags = 0;         // flags of the last opacity build (its backward uses them)
     std::vector<void *> allocations;
     bool have_eos_data = false, have_eos = false;
@@ -200,6 +224,8 @@ void launch_bfxs(slgpu_ctx *c, const float *d_ph1, const float *d_ph2, const int
 void launch_cell_prep(slgpu_ctx *c, const double *d_natom, const double *d_vol,
                       const double *d_nelec, const double *d_oc, const double *d_ginv,
                       int flags);
+void launch_lines64(slgpu_ctx *c, int64_t n);
+int line_degree(const slgpu_ctx *c);
 void launch_eos_ndens(slgpu_ctx *c, const double *temp, const double *mass, const double *natom,
                       const double *natomfr, double *ndens);
 void launch_nlte_rad_est(slgpu_ctx *c, double *radtemp, double *jrad);
@@ -229,6 +255,59 @@ void launch_eos_vjp(slgpu_ctx *c, const double *temp, const double *mass, const 
                     const double *oc, const double *g_natom, const double *g_fr,
                     const double *g_ne, const double *g_oc, double *out_T, double *out_mass,
                     double *out_mf);
+
+// ---------------------------------------------------------------------------
+// The FP64 line sums.  exp(-chi h), with h = hc/kT of the cell, is the product of two entries of
+// the cell's tables and a short polynomial: chi = (K2 k1 + k2) step + r, |r| <= step/2, splits
+// exactly (step has few bits, chi is single), so
+//   exp(-chi h) = E1[k1] E2[k2] P(-r h),   E1[k1] = exp(-K2 k1 step h),  E2[k2] = exp(-k2 step h).
+// The tables (64 entries per cell, k_exp_table) stand in LDS as rows of the block's 64 cells; k1, k2, r
+// and gxs are the same for the whole wave and come as scalars.  That is 10 FP64 operations
+// and two LDS rows per line and cell, against about 50 for exp() and the reference's product;
+// its error is that of the table entries (2 units in the last place), below the rounding of
+// the product chi h that exp() takes.  P is the Taylor polynomial of degree DEG; the launch
+// picks the smallest whose remainder at the largest |r h| stays under 2^-53.
+template <int DEG> __device__ __forceinline__ double exp_poly(double x)
+{
+    constexpr double inv[13] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,
+                                1.0 / 40320, 1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600};
+    double p = inv[DEG];
+    #pragma unroll
+    for (int k = DEG - 1; k >= 0; --k) p = fma(p, x, inv[k]);
+    return p;
+}
+
+// The tile of a block: blocks go round-robin over the 8 XCDs, so XCD q takes the q-th eighth of the
+// tiles in order.  Consecutive tiles (the cell blocks of one group block) then run on one XCD and
+// read that group block's lines from its L2 once.
+__device__ __forceinline__ uint32_t xcd_tile()
+{
+    const uint32_t n = gridDim.x, b = blockIdx.x, q = b & 7u, per = n >> 3, rest = n & 7u;
+    return q * per + (q < rest ? q : rest) + (b >> 3);
+}
+
+// Bring lines [a, b) (the first 512) into L2: a wave reads them one trip after the other with scalar
+// loads, each of which would otherwise wait for HBM.  One 4-byte read per 128-byte line; the
+// caller consumes the result once it has waited for something else.
+__device__ __forceinline__ uint32_t touch_lines(const Line64 *lines, int a, int b, int lane)
+{
+    const int l0 = a + lane * 4, l1 = l0 + 256;
+    const uint32_t v0 = l0 < b ? lines[l0].k1 : 0u, v1 = l1 < b ? lines[l1].k1 : 0u;
+    return v0 | v1;
+}
+
+// one row's entry of the lane, from the lane's column and a byte offset
+__device__ __forceinline__ double row_at(const double *column, uint32_t offset)
+{
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(column) + offset);
+}
+
+// the entries of a line's cell tables times its polynomial; e_lane: the lane's column of the tables
+template <int DEG>
+__device__ __forceinline__ double line_exp(const Line64 &q, const double *e_lane, double nh)
+{
+    return row_at(e_lane, q.k1) * row_at(e_lane, q.k2) * exp_poly<DEG>(q.r * nh);
+}
 
 // physical_opacity.f:228-243: sum over elements of g_ff(u, gamma^2) z^2 natomfr for cell ic at
 // the u coordinate (iu, du). The bilinear g_ff is linear in the table rows of u, so the

@@ -146,6 +146,46 @@ __global__ __launch_bounds__(128) void k_ff_table(Dev d, const double *__restric
     if (j == 0) d.ffclamp[ic] = m;
 }
 
+// acc plus the bound-free sum of group g in cell ic, ion by ion (physical_opacity.f:177-189;
+// cross sections precomputed per group and ion).  Only ions with a nonzero cross section are
+// visited: above the ground states' thresholds, most groups of an optical grid, there is none.
+__device__ __forceinline__ double bf_add(const Dev &d, int g, int ic, double acc)
+{
+    const double *xs = d.bfxs + (size_t)(g - 1) * d.nion, *oc = d.ocT + ic;
+    const int nw = (d.nion + 31) / 32;
+    for (int w = 0; w < nw; ++w)
+        for (uint32_t m = d.bfmask[(size_t)(g - 1) * nw + w]; m != 0u; m &= m - 1u) {
+            const int k = w * 32 + __builtin_ctz(m);
+            acc += xs[k] * oc[(size_t)k * d.nx];
+        }
+    return acc;
+}
+
+// bit k of a group's words: ion k's cross section is not zero
+__global__ __launch_bounds__(256) void k_bfmask(Dev d)
+{
+    const int nw = (d.nion + 31) / 32, t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= d.ng * nw) return;
+    const int g = t / nw, w = t - g * nw;
+    uint32_t m = 0u;
+    for (int k = 0; k < 32 && w * 32 + k < d.nion; ++k)
+        if (d.bfxs[(size_t)g * d.nion + w * 32 + k] != 0.0) m |= 1u << k;
+    d.bfmask[t] = m;
+}
+
+// the free-free opacity at the left group edge wl (physical_opacity.f:210-243)
+__device__ __forceinline__ double ff_term(const Dev &d, double hckt, double wl, int ic, double ffc1,
+                                          const double *__restrict__ rgg_tab)
+{
+    const double u = hckt * (1.0 / wl);
+    const double ru = 10.0 * (log10(u) + 4.0) + 1.0;
+    int iu = (int)floor(ru);
+    iu = iu < 1 ? 1 : (iu > FF_NU - 1 ? FF_NU - 1 : iu);
+    const double du = ru - iu;
+    const double help = ffc1 * sqrt(hckt) * (1.0 - exp(-u)) * (wl * wl * wl) * d.hlparr[ic];
+    return help * ff_gaunt_sum(d, ic, iu, du, rgg_tab);
+}
+
 // Fused bb + bf + ff for one (cell, group); result into capT[g*nc + i] (cell-fastest).
 // blockDim = 256 = 64 cells x 4 groups; grid = (ceil(nc/64), ceil(ng/4)).
 // S: the block's 64 cells' line populations oc*ginv of every ion are staged in LDS once
@@ -249,51 +289,148 @@ __global__ __launch_bounds__(256) void k_opacity(Dev d, int flags, double ffc1,
             }
             acc += sum64 * phi * expfac;
         } else {
-            if constexpr (S) {
-                LineRec *ln = s_lines[threadIdx.x >> 6];
-                for (int base = l0; base < l1; base += 64) {
-                    const int n = l1 - base < 64 ? l1 - base : 64;
-                    wave_lds_sync();
-                    if (lane < n) ln[lane] = d.lines[base + lane];
-                    wave_lds_sync();
-                    #pragma unroll 2
-                    for (int j = 0; j < n; ++j) {
-                        const LineRec r = ln[j];
-                        const double o = s_oc[r.ion * 64 + lane];
-                        // the select keeps the product and the sum separately rounded
-                        const double term = phi * (double)r.gxs * o * exp(-((double)r.chilw * hckt)) * expfac;
-                        acc += (o > 0.0) ? term : 0.0;
-                    }
-                }
-            } else {
-                for (int l = l0; l < l1; ++l) {
-                    const LineRec r = d.lines[l];         // uniform: scalar loads
-                    const double o = ocg[(size_t)r.ion * nc];
-                    const double term = phi * (double)r.gxs * o * exp(-((double)r.chilw * hckt)) * expfac;
-                    acc += (o > 0.0) ? term : 0.0;
-                }
+            for (int l = l0; l < l1; ++l) {
+                const LineRec r = d.lines[l];             // uniform: scalar loads
+                const double o = ocg[(size_t)r.ion * nc];
+                const double term = phi * (double)r.gxs * o * exp(-((double)r.chilw * hckt)) * expfac;
+                acc += (o > 0.0) ? term : 0.0;
             }
         }
     }
-    if (!(flags & SLGPU_NOBF)) {
-        // physical_opacity.f:177-189 (cross sections precomputed per group and ion)
-        const double *xs = d.bfxs + (size_t)(g - 1) * d.nion;
-        for (int k = 0; k < d.nion; ++k) {
-            const double x = xs[k];
-            if (x != 0.0) acc += x * d.ocT[(size_t)k * nc + ic];
+    if (!(flags & SLGPU_NOBF)) acc = bf_add(d, g, ic, acc);
+    if (!(flags & SLGPU_NOFF)) acc += ff_term(d, hckt, wlo, ic, ffc1, rgg_tab);
+    if (act) d.capT[(size_t)(g - 1) * nc + i] = massive ? acc : 0.0;
+}
+
+// The records of the FP64 line sums from the ion-ordered lines (step: see slgpu_ctx), one thread each
+__global__ __launch_bounds__(256) void k_lines64(const LineRec *__restrict__ in, Line64 *__restrict__ out,
+                                                 int64_t n, double step)
+{
+    const int64_t l = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (l >= n) return;
+    const LineRec q = in[l];
+    const double chi = (double)q.chilw;
+    int k = (int)rint(chi / step);
+    k = k < 0 ? 0 : (k > EXP_K1 * EXP_K2 - 1 ? EXP_K1 * EXP_K2 - 1 : k);
+    Line64 o;
+    o.gxs = (double)q.gxs;
+    o.r = chi - k * step;                                      // exact
+    o.k1 = (uint32_t)(k / EXP_K2) * 512u;
+    o.k2 = (uint32_t)(EXP_K1 + k % EXP_K2) * 512u;
+    o.ion = (uint32_t)q.ion * 512u + (q.pad == 1 ? 1u : 0u);
+    o.chi = q.chilw;
+    out[l] = o;
+}
+
+// The cells' exponential tables: rows k1 < EXP_K1 hold exp(-EXP_K2 k1 step h), the rest
+// exp(-k2 step h), the rounding of the exponent's product carried in first order
+__global__ __launch_bounds__(256) void k_exp_table(Dev d)
+{
+    const int t = blockIdx.x * 256 + threadIdx.x, nc = d.nx;
+    if (t >= EXP_ROWS * nc) return;
+    const int row = t / nc, i = t - row * nc;
+    const double a = (row < EXP_K1 ? EXP_K2 * row : row - EXP_K1) * d.line_step, h = d.hckt[i];
+    const double y = a * h, e = exp(-y);
+    d.etab[t] = fma(-fma(a, h, -y), e, e);
+}
+
+// Fused bb + bf + ff in FP64, result into capT[g*nc + i] (cell-fastest).  One wave holds 64 cells
+// of one group as in k_opacity; 16 waves share the cells' tables and populations in LDS, and
+// WPG waves share a group's lines when the grid would otherwise leave the chip idle (their
+// sums meet in LDS in a fixed order).  The lines come in ion order: per run of one ion's
+// lines one population row, per line the terms gxs exp(-chi h) alone.
+// Its tiles are ordered so that one XCD reads a group block's lines for all cell blocks, and each wave
+// brings its lines into its L2 first (both together 0.57 -> 0.48 ms at c2).
+// c2 (400 x 10^4 x 2e6 lines): 1.08 ms with exp() per line and the reference's product, 0.48 ms
+// so; c5 (1000 x 10^4 x 4e6) 4.15 -> 1.92 ms; 64 x 250 x 1e5 53 -> 13 us.  What bounds it now is FP64
+// issue: 15 vector operations per line, 78% of the issue slots.
+template <int DEG, int WPG>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_opacity64(Dev d, int flags, double ffc1,
+                                                    const double *__restrict__ rgg_tab,
+                                                    const Line64 *__restrict__ lines,
+                                                    const int *__restrict__ gstart,
+                                                    const double *__restrict__ etab)
+{
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    double *s_e = reinterpret_cast<double *>(s_raw);           // EXP_ROWS x 64
+    double *s_pop = s_e + EXP_ROWS * 64;                       // nion x 64
+    double *s_part = s_pop + (size_t)d.nion * 64;              // 16 x 64 when WPG > 1
+    const int nc = d.nx, ng = d.ng;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tile = xcd_tile(), ncb = (nc + 63) / 64;
+    const int c0 = (int)(tile % ncb) * 64, i = c0 + lane;
+    const bool bb = !(flags & SLGPU_NOBB);
+    const int g = (int)(tile / ncb) * (16 / WPG) + wave / WPG + 1, seg = wave % WPG;
+    int la = 0, lb = 0;                                        // the wave's lines
+    if (bb) {
+        if (g <= ng) {
+            const int l0 = gstart[g], n = gstart[g + 1] - l0;
+            la = l0 + (int)((int64_t)n * seg / WPG);
+            lb = l0 + (int)((int64_t)n * (seg + 1) / WPG);
         }
+        const uint32_t touched = touch_lines(lines, la, lb, lane);
+        for (int k = threadIdx.x; k < EXP_ROWS * 64; k += 1024) {
+            const int cc = c0 + (k & 63);
+            s_e[k] = cc < nc ? etab[(size_t)(k >> 6) * nc + cc] : 0.0;
+        }
+        for (int k = threadIdx.x; k < d.nion * 64; k += 1024) {
+            const int cc = c0 + (k & 63);
+            const double o = cc < nc ? d.ocg[(size_t)(k >> 6) * nc + cc] : 0.0;
+            s_pop[k] = o > 0.0 ? o : 0.0;                      // the reference skips such ions
+        }
+        asm volatile("" ::"v"(touched));
+        __syncthreads();
     }
-    if (!(flags & SLGPU_NOFF)) {
-        // physical_opacity.f:210-243 (left group edge)
-        const double wl = wlo;
-        const double u = hckt * (1.0 / wl);
-        const double ru = 10.0 * (log10(u) + 4.0) + 1.0;
-        int iu = (int)floor(ru);
-        iu = iu < 1 ? 1 : (iu > FF_NU - 1 ? FF_NU - 1 : iu);
-        const double du = ru - iu;
-        const double help = ffc1 * sqrt(hckt) * (1.0 - exp(-u)) * (wl * wl * wl) * d.hlparr[ic];
-        acc += help * ff_gaunt_sum(d, ic, iu, du, rgg_tab);
+    const bool act = i < nc;
+    const int ic = act ? i : nc - 1;
+    const double hckt = d.hckt[ic];
+    double sum = 0.0;
+    if (la < lb) {
+        const double nh = -hckt;
+        const double *e_lane = s_e + lane, *pop_lane = s_pop + lane;
+        int t = la;
+        double r = 0.0;
+        auto add = [&](const Line64 &q, double e) {
+            r = fma(q.gxs, e, r);
+            if (q.ion & 1u) {                                  // the run's last line (wave-uniform)
+                sum = fma(row_at(pop_lane, q.ion - 1u), r, sum);
+                r = 0.0;
+            }
+        };
+        // four lines per trip: their records arrive in one scalar wait, their rows in one LDS wait
+        for (; t + 4 <= lb; t += 4) {
+            const Line64 q0 = lines[t], q1 = lines[t + 1], q2 = lines[t + 2], q3 = lines[t + 3];
+            const double e0 = line_exp<DEG>(q0, e_lane, nh), e1 = line_exp<DEG>(q1, e_lane, nh);
+            const double e2 = line_exp<DEG>(q2, e_lane, nh), e3 = line_exp<DEG>(q3, e_lane, nh);
+            add(q0, e0);
+            add(q1, e1);
+            add(q2, e2);
+            add(q3, e3);
+        }
+        for (; t < lb; ++t) {
+            const Line64 q = lines[t];
+            add(q, line_exp<DEG>(q, e_lane, nh));
+        }
+        if (WPG > 1) sum = fma(row_at(pop_lane, lines[lb - 1].ion & ~1u), r, sum);     // a run cut by the share
     }
+    if constexpr (WPG > 1) {
+        s_part[wave * 64 + lane] = sum;
+        __syncthreads();
+        if (seg != 0) return;
+        #pragma unroll
+        for (int w = 1; w < WPG; ++w) sum += s_part[(wave + w) * 64 + lane];
+    }
+    if (g > ng) return;
+    const bool massive = act && d.mass[ic] > 0.0;
+    const double wlo = d.wl[g - 1], whi = d.wl[g];
+    double acc = 0.0;
+    if (bb) {
+        // physical_opacity.f:128-137: subgroup-centre profile and stimulated emission
+        const double wlc = 0.5 * (wlo + whi);
+        acc = sum * (wlc * wlc / ((whi - wlo) * PC_C)) * (1.0 - exp(-hckt * (1.0 / wlc)));
+    }
+    if (!(flags & SLGPU_NOBF)) acc = bf_add(d, g, ic, acc);
+    if (!(flags & SLGPU_NOFF)) acc += ff_term(d, hckt, wlo, ic, ffc1, rgg_tab);
     if (act) d.capT[(size_t)(g - 1) * nc + i] = massive ? acc : 0.0;
 }
 
@@ -389,6 +526,8 @@ void launch_bfxs(slgpu_ctx *c, const float *d_ph1, const float *d_ph2, const int
     if (n == 0) return;
     hipLaunchKernelGGL(k_bfxs, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d, d_ph1,
                        d_ph2, d_iz, d_ii);
+    n = c->ng * ((c->nion + 31) / 32);
+    hipLaunchKernelGGL(k_bfmask, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d);
 }
 
 void launch_cell_prep(slgpu_ctx *c, const double *d_natom, const double *d_vol,
@@ -399,6 +538,8 @@ void launch_cell_prep(slgpu_ctx *c, const double *d_natom, const double *d_vol,
     int n = c->nx * nk;
     hipLaunchKernelGGL(k_cell_prep, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d,
                        d_natom, d_vol, d_nelec, d_oc, d_ginv, flags, g_rgg_scratch(c));
+    if (c->d.line_step > 0.0 && !(flags & SLGPU_NOBB))
+        hipLaunchKernelGGL(k_exp_table, dim3((EXP_ROWS * c->nx + 255) / 256), dim3(256), 0, c->stream, c->d);
     if (!(flags & SLGPU_NOFF))
         hipLaunchKernelGGL(k_ff_table, dim3(c->nx), dim3(128), 0, c->stream, c->d,
                            (const double *)g_rgg_scratch(c));
@@ -414,25 +555,67 @@ double ff_prefactor()
 
 const double *rgg_scratch(slgpu_ctx *c) { return g_rgg_scratch(c); }
 
+void launch_lines64(slgpu_ctx *c, int64_t n)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_lines64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, c->d.lines_ion,
+                           c->d.lines64, n, c->d.line_step);
+}
+
+// degree of the line sums' polynomial for the last build's cells: the smallest of 6, 8 and 10 whose
+// Taylor remainder x^(n+1)/(n+1)! at the largest x = step/2 hc/kT is under 2^-53; 0 when there
+// are no tables or the cells are too cold for them (exp() per line then)
+int line_degree(const slgpu_ctx *c)
+{
+    const double x = 0.5 * c->d.line_step * c->hckt_max;
+    if (!(x > 0.0)) return 0;
+    return x <= 0.0177 ? 6 : (x <= 0.069 ? 8 : (x <= 0.176 ? 10 : 0));
+}
+
+template <int DEG>
+static void launch_opacity64(slgpu_ctx *c, int flags, double ffc1, const double *rgg, size_t lds)
+{
+    // Waves per group: the chip holds 8192 waves of this kernel, which one per group fills at
+    // c2 (70000); smaller grids share a group's lines among 4 or 16 (64 x 250 x 1e5 lines, 250
+    // waves: 13 us with 16, against the 53 us of the form with one wave per group and exp()).
+    const int64_t waves = (int64_t)((c->nx + 63) / 64) * c->ng;
+    const unsigned cb = (c->nx + 63) / 64;
+    const Dev &d = c->d;
+    if (waves >= 8192)
+        hipLaunchKernelGGL((k_opacity64<DEG, 1>), dim3(cb * ((c->ng + 15) / 16)), dim3(1024), lds, c->stream, d,
+                           flags, ffc1, rgg, d.lines64, d.gstart, d.etab);
+    else if (waves >= 2048)
+        hipLaunchKernelGGL((k_opacity64<DEG, 4>), dim3(cb * ((c->ng + 3) / 4)), dim3(1024), lds, c->stream, d,
+                           flags, ffc1, rgg, d.lines64, d.gstart, d.etab);
+    else
+        hipLaunchKernelGGL((k_opacity64<DEG, 16>), dim3(cb * c->ng), dim3(1024), lds, c->stream, d, flags, ffc1,
+                           rgg, d.lines64, d.gstart, d.etab);
+}
+
 void launch_opacity(slgpu_ctx *c, int flags)
 {
     const double ffc1 = ff_prefactor();
     dim3 grid((c->nx + 63) / 64, (c->ng + 3) / 4);
     const double *rgg = g_rgg_scratch(c);
-    const bool mixed = c->d.precision == SLGPU_MIXED;
-    // staged populations: nion x 64 cells, up to 64 KiB of LDS per block beside the 4 KiB
-    // of line records
-    const size_t lds = (size_t)c->nion * 64 * (mixed ? sizeof(float) : sizeof(double));
+    // precision form: staged populations, nion x 64 cells, up to 64 KiB of LDS per block beside
+    // the 4 KiB of line records
+    const size_t lds = (size_t)c->nion * 64 * sizeof(float);
     const bool staged = !c->force_unstaged && c->nion > 0 && lds <= 65536;
-    if (mixed && staged)
+    // FP64: tables, populations and the waves' partial sums within the CU's 160 KiB
+    const size_t lds64 = ((size_t)EXP_ROWS + c->nion + 16) * 64 * sizeof(double);
+    const int deg = c->force_unstaged || lds64 > 163840 ? 0 : line_degree(c);
+    if (c->d.precision == SLGPU_MIXED && staged)
         hipLaunchKernelGGL((k_opacity<true, true>), grid, dim3(256), lds, c->stream, c->d, flags,
                            ffc1, rgg);
-    else if (mixed)
+    else if (c->d.precision == SLGPU_MIXED)
         hipLaunchKernelGGL((k_opacity<true, false>), grid, dim3(256), 0, c->stream, c->d, flags,
                            ffc1, rgg);
-    else if (staged)
-        hipLaunchKernelGGL((k_opacity<false, true>), grid, dim3(256), lds, c->stream, c->d, flags,
-                           ffc1, rgg);
+    else if (deg == 6)
+        launch_opacity64<6>(c, flags, ffc1, rgg, lds64);
+    else if (deg == 8)
+        launch_opacity64<8>(c, flags, ffc1, rgg, lds64);
+    else if (deg == 10)
+        launch_opacity64<10>(c, flags, ffc1, rgg, lds64);
     else
         hipLaunchKernelGGL((k_opacity<false, false>), grid, dim3(256), 0, c->stream, c->d, flags,
                            ffc1, rgg);

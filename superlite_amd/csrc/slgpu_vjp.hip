@@ -6,9 +6,6 @@
 //
 //   k_vjp_means     16 cells x 64 groups per block: the means' gradients folded into
 //                   dL/dcap, plus their direct T and sigma_Thomson terms as per-tile partials
-//   k_vjp_means_sum one wave per cell: the tiles' partials of those terms
-//   k_vjp_ff_fr     one thread per (element, cell): the ff mass-fraction gradient of the
-//                   elements inside the g_ff table, from the per-cell node sums
 //   k_vjp_opacity   one thread per (cell, group), 64 cells x 16 groups per block: the bb
 //                   line terms recomputed (not stored) and ff, with per-ion and
 //                   per-element accumulators in LDS flushed once per block; bb in
@@ -19,15 +16,16 @@
 //                   accumulator once
 //   k_vjp_bf_mfma   the bf part, a contraction over groups of the cross sections with
 //                   dL/dcap, on the FP64 matrix cores
-//   k_vjp_finish    one thread per cell: chain rule through hckt = hc/kT, the ff prefactor
-//                   (natom/V)^2 n_e and sigma_T = c_T n_e natom/V
+//   k_vjp_lines64   the bb lines in FP64
+//   k_vjp_finish    one block per cell: the sums over tiles and copies, the ff mass-fraction
+//                   gradient from the node sums, and the chain rule through hckt = hc/kT, the
+//                   ff prefactor (natom/V)^2 n_e and sigma_T = c_T n_e natom/V
 //
 // The means are taken through the FP32-rounded cap as the forward evaluates them, with the
 // rounding treated as the identity.  In the precision form (SLGPU_MIXED) the recomputed
 // bb line terms are FP32 in short partial sums folded into FP64, like that form's forward; bf, ff,
 // the means and every accumulator stay FP64.  Elements absent from every cell are skipped
 // by the forward's ff sum, so their mass-fraction gradient is returned as 0.
-#include <type_traits>
 #include "slgpu_device.h"
 #include "slgpu_internal.h"
 
@@ -76,7 +74,7 @@ __device__ __forceinline__ double d_spectintv_dT(double tinv, const double *__re
 // turn, its lanes 64 consecutive groups, so cap32 and gc are read along the group axis; the
 // dL/dcap values go through an LDS tile and are stored along the cell axis of gcapT. The
 // per-cell sums of dL/dT and dL/dsig are wave sums in a fixed order, one partial per tile
-// (gmpart), added in tile order by k_vjp_means_sum.
+// (gmpart), added by k_vjp_finish.
 __global__ __launch_bounds__(256) void k_vjp_means(Dev d, const double *__restrict__ gc,
                                                    const double *__restrict__ gp,
                                                    const double *__restrict__ gr)
@@ -126,26 +124,13 @@ __global__ __launch_bounds__(256) void k_vjp_means(Dev d, const double *__restri
     }
 }
 
-// dL/dT and dL/dsig of the means: one wave per cell adds the tiles' partials (lane y takes
-// tiles y, y+64, ...; then a fixed-order wave sum); clears the slots the line and ff kernels
-// add into
-__global__ __launch_bounds__(64) void k_vjp_means_sum(Dev d, int nty)
+// The blocks of one cell tile add their sums to the same few thousand addresses, and an FP64
+// atomic on an address waits for the one before it: the tile's blocks go round-robin to
+// GACC_COPIES copies, which k_vjp_finish adds (FP64 bb lines of 122 cells x 6000 groups x 6e5
+// lines: 220 us with one copy, 183 us with 8).
+__device__ __forceinline__ double *goc_copy(const Dev &d)
 {
-    const int i = blockIdx.x, lane = threadIdx.x, nc = d.nx;
-    if (i >= nc) return;
-    double dT = 0.0, dsig = 0.0;
-    for (int y = lane; y < nty; y += 64) {
-        dT += d.gmpart[((size_t)0 * nty + y) * nc + i];
-        dsig += d.gmpart[((size_t)1 * nty + y) * nc + i];
-    }
-    dT = wave_sum(dT);
-    dsig = wave_sum(dsig);
-    if (lane == 0) {
-        d.gcell[0 * nc + i] = dT;
-        d.gcell[1 * nc + i] = dsig;
-        d.gcell[2 * nc + i] = 0.0;
-        d.gcell[3 * nc + i] = 0.0;
-    }
+    return d.goc + (size_t)(blockIdx.y % GACC_COPIES) * d.nion * d.nx;
 }
 
 // dynamic LDS: s_oc[nion][64] then s_fr[nel][64].  M: the precision form, whose bb line
@@ -164,7 +149,7 @@ __global__ __launch_bounds__(NWV * 64)
 __attribute__((amdgpu_waves_per_eu(P == 1 ? 6 : 1, 8)))
 void k_vjp_opacity(Dev d, int flags, double ffc1, const double *__restrict__ rgg_tab)
 {
-    using PT = typename std::conditional<M, float, double>::type;
+    using PT = float;              // staged populations: the precision form only
     constexpr bool BB = (P & 1) != 0, FF = (P & 2) != 0;
     constexpr int NT = NWV * 64;
     extern __shared__ double s_acc[];
@@ -188,6 +173,7 @@ void k_vjp_opacity(Dev d, int flags, double ffc1, const double *__restrict__ rgg
     __syncthreads();
     const double hckt = d.hckt[ic];
     double dh_acc = 0.0, dhl_acc = 0.0;
+    double *W = d.ffW + (size_t)(blockIdx.y % GACC_COPIES) * FF_NU * nc;
     int w_iu = 0;                                  // u node pair of the W run (0: none)
     double w_lo = 0.0, w_hi = 0.0;
     for (int q = 0; q < VJP_GROUPS / NWV; ++q) {
@@ -285,52 +271,15 @@ void k_vjp_opacity(Dev d, int flags, double ffc1, const double *__restrict__ rgg
                 s0 = pe * t0;
                 s1 = pe * t1;
             } else {
-                if constexpr (S) {
-                    LineRec *ln = s_lines[wave];
-                    int cur = -1;
-                    double oc_ = 0.0, sb = 0.0;
-                    for (int base0 = l0; base0 < l1; base0 += 64) {
-                        const int n = l1 - base0 < 64 ? l1 - base0 : 64;
-                        wave_lds_sync();
-                        if (lane < n) ln[lane] = d.lines_ion[base0 + lane];
-                        wave_lds_sync();
-                        // one run of an ion's lines at a time (pad: lines left in the run)
-                        for (int j = 0; j < n;) {
-                            const int ion = __builtin_amdgcn_readfirstlane(ln[j].ion);
-                            int len = __builtin_amdgcn_readfirstlane(ln[j].pad);
-                            len = len < n - j ? len : n - j;
-                            len = len > 1 ? len : 1;                 // always advances
-                            if (ion != cur) {
-                                if (sb != 0.0) atomicAdd(&s_bb[cur * 64 + lane], G * sb);
-                                cur = ion;
-                                sb = 0.0;
-                                oc_ = s_pop[ion * 64 + lane];
-                            }
-                            if (oc_ > 0.0) {
-                                for (int t = j; t < j + len; ++t) {
-                                    const LineRec r = ln[t];
-                                    const double base = phi * (double)r.gxs * exp(-((double)r.chilw * hckt)) * expfac;
-                                    const double term = base * oc_;
-                                    s0 += term;
-                                    s1 += term * (double)r.chilw;
-                                    sb += base;
-                                }
-                            }
-                            j += len;
-                        }
-                    }
-                    if (sb != 0.0) atomicAdd(&s_bb[cur * 64 + lane], G * sb);
-                } else {
-                    for (int l = l0; l < l1; ++l) {
-                        const LineRec r = d.lines[l];
-                        const double o = ocg[(size_t)r.ion * nc];
-                        if (o > 0.0) {
-                            const double base = phi * (double)r.gxs * exp(-((double)r.chilw * hckt)) * expfac;
-                            const double term = base * o;
-                            s0 += term;
-                            s1 += term * (double)r.chilw;
-                            atomicAdd(&s_bb[r.ion * 64 + lane], G * base);
-                        }
+                for (int l = l0; l < l1; ++l) {
+                    const LineRec r = d.lines[l];
+                    const double o = ocg[(size_t)r.ion * nc];
+                    if (o > 0.0) {
+                        const double base = phi * (double)r.gxs * exp(-((double)r.chilw * hckt)) * expfac;
+                        const double term = base * o;
+                        s0 += term;
+                        s1 += term * (double)r.chilw;
+                        atomicAdd(&s_bb[r.ion * 64 + lane], G * base);
                     }
                 }
             }
@@ -357,12 +306,12 @@ void k_vjp_opacity(Dev d, int flags, double ffc1, const double *__restrict__ rgg
             // Their mass-fraction gradient, sum over groups of G help g_ff zz, is
             // zz * sum_j A_k(j) W(j), with A_k element k's g_ff row interpolated in rgg and W
             // the groups' G*help spread over their two u nodes. W accumulates in registers
-            // while iu stays, and goes to ffW when it changes (k_vjp_ff_fr finishes the sum).
+            // while iu stays, and goes to ffW when it changes (k_vjp_finish finishes the sum).
             if (act) {
                 if (iu != w_iu) {
                     if (w_iu > 0) {
-                        atomicAdd(&d.ffW[(size_t)(w_iu - 1) * nc + ic], w_lo);
-                        atomicAdd(&d.ffW[(size_t)w_iu * nc + ic], w_hi);
+                        atomicAdd(&W[(size_t)(w_iu - 1) * nc + ic], w_lo);
+                        atomicAdd(&W[(size_t)w_iu * nc + ic], w_hi);
                     }
                     w_iu = iu;
                     w_lo = 0.0;
@@ -397,22 +346,117 @@ void k_vjp_opacity(Dev d, int flags, double ffc1, const double *__restrict__ rgg
         }
     }
     if (FF && act && w_iu > 0) {
-        atomicAdd(&d.ffW[(size_t)(w_iu - 1) * nc + ic], w_lo);
-        atomicAdd(&d.ffW[(size_t)w_iu * nc + ic], w_hi);
+        atomicAdd(&W[(size_t)(w_iu - 1) * nc + ic], w_lo);
+        atomicAdd(&W[(size_t)w_iu * nc + ic], w_hi);
     }
     if (act) {
-        if (dh_acc != 0.0) atomicAdd(&d.gcell[2 * nc + i], dh_acc);
-        if (FF) atomicAdd(&d.gcell[3 * nc + i], dhl_acc);
+        if (dh_acc != 0.0) atomicAdd(&d.gcell[i], dh_acc);
+        if (FF) atomicAdd(&d.gcell[nc + i], dhl_acc);
     }
     __syncthreads();
     for (int k = threadIdx.x; k < (nrow_b + nrow_f) * 64; k += NT) {
         const int row = k >> 6, cell = blockIdx.x * 64 + (k & 63);
         const double v = s_acc[k];
         if (cell < nc && v != 0.0) {
-            if (row < nrow_b) atomicAdd(&d.goc[(size_t)row * nc + cell], v * d.ginvT[(size_t)row * nc + cell]);
+            if (row < nrow_b) atomicAdd(&goc_copy(d)[(size_t)row * nc + cell], v * d.ginvT[(size_t)row * nc + cell]);
             else atomicAdd(&d.gfr[(size_t)(row - nrow_b) * nc + cell], v);
         }
     }
+}
+
+// The bb lines of the FP64 backward: the forward's line sums (line_exp in slgpu_internal.h) in
+// ion runs, per line the exponential and two FMAs (the run's sums of gxs e and gxs chi e), per
+// run the cell's two accumulators and one LDS atomic.  1024 threads share 64 cells' tables,
+// populations and per-ion accumulators; each wave takes `gpw` groups.
+template <int DEG>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_vjp_lines64(Dev d, int gpw, const Line64 *__restrict__ lines,
+                                                      const int *__restrict__ gstart,
+                                                      const double *__restrict__ etab)
+{
+    extern __shared__ double s_acc[];
+    const int nc = d.nx, ng = d.ng, nion = d.nion;
+    double *s_bb = s_acc, *s_pop = s_bb + (size_t)nion * 64, *s_e = s_pop + (size_t)nion * 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tile = xcd_tile(), ncb = (nc + 63) / 64;
+    const int c0 = (int)(tile % ncb) * 64, i = c0 + lane;
+    const int gb = (int)(tile / ncb), g0 = (gb * 16 + wave) * gpw + 1;
+    const bool act = i < nc;
+    const uint32_t touched = g0 <= ng ? touch_lines(lines, gstart[g0], gstart[g0 + 1], lane) : 0u;
+    for (int k = threadIdx.x; k < nion * 64; k += 1024) {
+        const int cc = c0 + (k & 63);
+        const double o = cc < nc ? d.ocg[(size_t)(k >> 6) * nc + cc] : 0.0;
+        s_bb[k] = 0.0;
+        s_pop[k] = o > 0.0 ? o : 0.0;
+    }
+    for (int k = threadIdx.x; k < EXP_ROWS * 64; k += 1024) {
+        const int cc = c0 + (k & 63);
+        s_e[k] = cc < nc ? etab[(size_t)(k >> 6) * nc + cc] : 0.0;
+    }
+    asm volatile("" ::"v"(touched));
+    __syncthreads();
+    const double hckt = d.hckt[act ? i : nc - 1], nh = -hckt;
+    const double *e_lane = s_e + lane, *pop_lane = s_pop + lane;
+    double dh = 0.0;
+    for (int q = 0; q < gpw; ++q) {
+        const int g = g0 + q;
+        if (g > ng) break;
+        if (q > 0) {
+            const uint32_t more = touch_lines(lines, gstart[g], gstart[g + 1], lane);
+            asm volatile("" ::"v"(more));
+        }
+        const double G = act ? d.gcapT[(size_t)(g - 1) * nc + i] : 0.0;
+        const double wlo = d.wl[g - 1], whi = d.wl[g];
+        const double wlc = 0.5 * (wlo + whi), wlinv = 1.0 / wlc;
+        const double ec = exp(-hckt * wlinv), expfac = 1.0 - ec;
+        const double gpe = G * (wlc * wlc / ((whi - wlo) * PC_C)) * expfac;
+        double s0 = 0.0, s1 = 0.0, sb = 0.0, sc = 0.0;
+        const int l1 = gstart[g + 1];
+        auto add = [&](const Line64 &q, double e) {
+            const double u = q.gxs * e;
+            sb += u;
+            sc = fma((double)q.chi, u, sc);
+            if (q.ion & 1u) {                                  // the run's last line (wave-uniform)
+                const double pop = row_at(pop_lane, q.ion - 1u);
+                s0 = fma(pop, sb, s0);
+                s1 = fma(pop, sc, s1);
+                const double v = gpe * sb;
+                if (pop > 0.0 && v != 0.0) atomicAdd(&s_bb[((q.ion - 1u) >> 3) + lane], v);
+                sb = 0.0;
+                sc = 0.0;
+            }
+        };
+        int t = gstart[g];
+        for (; t + 4 <= l1; t += 4) {
+            const Line64 q0 = lines[t], q1 = lines[t + 1], q2 = lines[t + 2], q3 = lines[t + 3];
+            const double e0 = line_exp<DEG>(q0, e_lane, nh), e1 = line_exp<DEG>(q1, e_lane, nh);
+            const double e2 = line_exp<DEG>(q2, e_lane, nh), e3 = line_exp<DEG>(q3, e_lane, nh);
+            add(q0, e0);
+            add(q1, e1);
+            add(q2, e2);
+            add(q3, e3);
+        }
+        for (; t < l1; ++t) {
+            const Line64 q = lines[t];
+            add(q, line_exp<DEG>(q, e_lane, nh));
+        }
+        dh += gpe * (s0 * wlinv * ec / expfac - s1);
+    }
+    if (act && dh != 0.0) atomicAdd(&d.gcell[i], dh);
+    __syncthreads();
+    for (int k = threadIdx.x; k < nion * 64; k += 1024) {
+        const int row = k >> 6, cell = c0 + (k & 63);
+        const double v = s_bb[k];
+        if (cell < nc && v != 0.0)
+            atomicAdd(&d.goc[((size_t)(gb % GACC_COPIES) * nion + row) * nc + cell], v * d.ginvT[(size_t)row * nc + cell]);
+    }
+}
+
+template <int DEG> static void launch_vjp_lines64(slgpu_ctx *c, size_t lds)
+{
+    // two groups per wave halve the accumulators' flushes; one where that leaves CUs without work
+    const int gpw = (int64_t)((c->nx + 63) / 64) * c->ng >= 32 * 512 ? 2 : 1;
+    hipLaunchKernelGGL((k_vjp_lines64<DEG>), dim3((c->nx + 63) / 64 * ((c->ng + 16 * gpw - 1) / (16 * gpw))),
+                       dim3(1024), lds, c->stream, c->d, gpw, c->d.lines64, c->d.gstart, c->d.etab);
 }
 
 // bf part of the backward on the matrix cores: d(sum_k bfxs(g,k) oc(k,i))/d(oc(k,i)) summed
@@ -444,53 +488,73 @@ __global__ __launch_bounds__(64) void k_vjp_bf_mfma(Dev d)
     #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int k = m0 + 4 * r + lk;
-        if (k < nion && cell_ok && acc[r] != 0.0) atomicAdd(&d.goc[(size_t)k * nc + cell], acc[r]);
+        if (k < nion && cell_ok && acc[r] != 0.0)
+            atomicAdd(&d.goc[((size_t)(blockIdx.z % GACC_COPIES) * nion + k) * nc + cell], acc[r]);
     }
 }
 
-// chain rule to the inputs; outputs in the forward's input layouts
-__global__ __launch_bounds__(256) void k_vjp_finish(Dev d, int flags, double *gT, double *gnat,
-                                                    double *gne, double *gfr_out, double *goc_out)
+// The sums over copies and tiles and the chain rule to the inputs, in the forward's input layouts;
+// one block of 128 threads per cell.
+//   dL/dT, dL/dsig of the means: the tiles' partials (lane y of wave 0 takes tiles y, y+64, ...).
+//   mass fractions of the elements inside the g_ff table (physical_opacity.f:228-243):
+//     gfr[k] += z^2 sum_j A_k(j) W(j), A_k(j) = (1 - dgg) g_ff[igg-1][j] + dgg g_ff[igg][j] element
+//     k's row at the cell's rgg, W the backward's G*help node sums; one wave per element.
+//     Elements past the table were summed per group.
+//   ion populations: a thread per ion.
+__global__ __launch_bounds__(128) void k_vjp_finish(Dev d, int flags, int nty, const double *__restrict__ rgg_tab,
+                                                    double *gT, double *gnat, double *gne, double *gfr_out,
+                                                    double *goc_out)
 {
     constexpr double cthomson = 8.0 * PC_PI * (PC_E * PC_E * PC_E * PC_E) /
                                 (3.0 * (PC_ME * PC_ME) * (PC_C * PC_C * PC_C * PC_C));
-    const int nc = d.nx;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc) return;
-    const double T = d.temp[i], hckt = d.hckt[i];
-    const double natom = d.natom_in[i], vol = d.vol_in[i], ne = d.nelec_in[i];
-    const double gsig = d.gcell[1 * nc + i], ghl = d.gcell[3 * nc + i];
-    const bool thomson = !(flags & SLGPU_NOTHOMSON) && d.mass[i] > 0.0;
-    gT[i] = d.gcell[0 * nc + i] + d.gcell[2 * nc + i] * (-hckt / T);
-    const double nv = natom / vol;
-    gne[i] = ghl * nv * nv + (thomson ? gsig * cthomson * natom / vol : 0.0);
-    gnat[i] = ghl * 2.0 * natom * ne / (vol * vol) + (thomson ? gsig * cthomson * ne / vol : 0.0);
-    for (int z = 0; z < 30; ++z) gfr_out[(size_t)i * 30 + z] = 0.0;
-    for (int k = 0; k < d.nel; ++k) gfr_out[(size_t)i * 30 + d.el_z[k] - 1] = d.gfr[(size_t)k * nc + i];
-    for (int k = 0; k < d.nion; ++k) goc_out[(size_t)i * d.nion + k] = d.goc[(size_t)k * nc + i];
-}
-
-// The mass-fraction gradient of the elements inside the g_ff table (physical_opacity.f:
-// 228-243): gfr[k][i] += z^2 * sum_j A_k(j) W(i, j), with A_k(j) = (1 - dgg) g_ff[igg-1][j] +
-// dgg g_ff[igg][j] element k's row at the cell's rgg and W the backward's G*help node sums.
-// One thread per (element, cell); elements past the table were summed per group.
-__global__ __launch_bounds__(256) void k_vjp_ff_fr(Dev d, const double *__restrict__ rgg_tab)
-{
-    const int nc = d.nx;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= d.nel * nc) return;
-    const int k = t / nc, i = t - k * nc;
-    const double rgg = rgg_tab[(size_t)k * nc + i];
-    if (rgg > FF_NGG) return;
-    int igg = (int)floor(rgg);
-    igg = igg < 1 ? 1 : (igg > FF_NGG - 1 ? FF_NGG - 1 : igg);
-    const double dgg = rgg - igg;
-    const double *lo = d.gff + (size_t)(igg - 1) * FF_NU, *hi = d.gff + (size_t)igg * FF_NU;
-    const double *W = d.ffW + i;                       // node-major, cell fastest
-    double s = 0.0;
-    for (int j = 0; j < FF_NU; ++j) s += ((1.0 - dgg) * lo[j] + dgg * hi[j]) * W[(size_t)j * nc];
-    const int z = d.el_z[k];
-    d.gfr[(size_t)k * nc + i] += (double)(z * z) * s;
+    __shared__ double s_W[128], s_fr[30];
+    const int nc = d.nx, i = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    double w = 0.0;
+    if (t < FF_NU)
+        for (int r = 0; r < GACC_COPIES; ++r) w += d.ffW[((size_t)r * FF_NU + t) * nc + i];
+    s_W[t] = w;
+    if (t < 30) s_fr[t] = 0.0;
+    for (int k = t; k < d.nion; k += 128) {
+        double v = 0.0;
+        for (int r = 0; r < GACC_COPIES; ++r) v += d.goc[((size_t)r * d.nion + k) * nc + i];
+        goc_out[(size_t)i * d.nion + k] = v;
+    }
+    __syncthreads();
+    for (int k = wave; k < d.nel; k += 2) {
+        const double rgg = rgg_tab[(size_t)k * nc + i];
+        double v = 0.0;
+        if (!(flags & SLGPU_NOFF) && !(rgg > FF_NGG)) {
+            int igg = (int)floor(rgg);
+            igg = igg < 1 ? 1 : (igg > FF_NGG - 1 ? FF_NGG - 1 : igg);
+            const double dgg = rgg - igg;
+            const double *lo = d.gff + (size_t)(igg - 1) * FF_NU, *hi = lo + FF_NU;
+            for (int j = lane; j < FF_NU; j += 64) v += ((1.0 - dgg) * lo[j] + dgg * hi[j]) * s_W[j];
+            v = wave_sum(v);
+        }
+        const int z = d.el_z[k];
+        if (lane == 0) s_fr[z - 1] = d.gfr[(size_t)k * nc + i] + (double)(z * z) * v;
+    }
+    double dT = 0.0, gsig = 0.0;
+    if (wave == 0) {
+        for (int y = lane; y < nty; y += 64) {
+            dT += d.gmpart[((size_t)0 * nty + y) * nc + i];
+            gsig += d.gmpart[((size_t)1 * nty + y) * nc + i];
+        }
+        dT = wave_sum(dT);
+        gsig = wave_sum(gsig);
+    }
+    __syncthreads();
+    if (t < 30) gfr_out[(size_t)i * 30 + t] = s_fr[t];
+    if (t == 0) {
+        const double T = d.temp[i], hckt = d.hckt[i];
+        const double natom = d.natom_in[i], vol = d.vol_in[i], ne = d.nelec_in[i];
+        const double ghl = d.gcell[nc + i];
+        const bool thomson = !(flags & SLGPU_NOTHOMSON) && d.mass[i] > 0.0;
+        gT[i] = dT + d.gcell[i] * (-hckt / T);
+        const double nv = natom / vol;
+        gne[i] = ghl * nv * nv + (thomson ? gsig * cthomson * natom / vol : 0.0);
+        gnat[i] = ghl * 2.0 * natom * ne / (vol * vol) + (thomson ? gsig * cthomson * ne / vol : 0.0);
+    }
 }
 
 void launch_opacity_vjp(slgpu_ctx *c, int flags, const double *gc, const double *gp,
@@ -498,53 +562,44 @@ void launch_opacity_vjp(slgpu_ctx *c, int flags, const double *gc, const double 
                         double *goc, double ffc1, const double *rgg)
 {
     const int nc = c->nx, ng = c->ng;
-    (void)hipMemsetAsync(c->d.goc, 0, (size_t)std::max(c->nion, 1) * nc * 8, c->stream);
-    (void)hipMemsetAsync(c->d.gfr, 0, (size_t)30 * nc * 8, c->stream);
-    (void)hipMemsetAsync(c->d.ffW, 0, (size_t)FF_NU * nc * 8, c->stream);
-    {
-        const int nty = (ng + 63) / 64;
-        hipLaunchKernelGGL(k_vjp_means, dim3((nc + 15) / 16, nty), dim3(256), 0, c->stream, c->d, gc, gp, gr);
-        hipLaunchKernelGGL(k_vjp_means_sum, dim3(nc), dim3(64), 0, c->stream, c->d, nty);
-    }
+    // the accumulators lie one behind the other (goc first): one fill
+    (void)hipMemsetAsync(c->d.goc, 0, vjp_acc_doubles(c->nion, nc) * sizeof(double), c->stream);
+    const int nty = (ng + 63) / 64;
+    hipLaunchKernelGGL(k_vjp_means, dim3((nc + 15) / 16, nty), dim3(256), 0, c->stream, c->d, gc, gp, gr);
     const bool mixed = c->d.precision == SLGPU_MIXED;
     const size_t acc_b = (size_t)(c->nion + c->d.nel) * 64 * sizeof(double);
     const size_t bb_b = (size_t)c->nion * 64 * sizeof(double), ff_b = (size_t)c->d.nel * 64 * sizeof(double);
-    const size_t pop_b = (size_t)c->nion * 64 * (mixed ? sizeof(float) : sizeof(double));
-    // With the populations staged and the line slots of 8 waves within 64 KiB of LDS, the bb
-    // lines run in 512-thread blocks (8 waves x 2 groups sharing the cells' accumulators) and
-    // ff in a kernel of its own; otherwise both in one 256-thread kernel, populations unstaged.
-    const bool staged = !c->force_unstaged && bb_b + pop_b + 8 * 64 * sizeof(LineRec) <= 65536;
+    const size_t pop_b = (size_t)c->nion * 64 * sizeof(float);
+    // The bb lines run in a kernel of their own, ff in another, when the cells' populations (and in
+    // FP64 their exponential tables) fit in LDS beside the accumulators; otherwise both in one
+    // 256-thread kernel, populations unstaged.  Precision form: 8 waves x 2 groups share the
+    // cells' accumulators within 64 KiB.
+    const size_t lds64 = ((size_t)2 * c->nion + EXP_ROWS) * 64 * sizeof(double);
+    const int deg = c->force_unstaged || mixed || lds64 > 163840 ? 0 : line_degree(c);
+    const bool staged = mixed ? !c->force_unstaged && bb_b + pop_b + 8 * 64 * sizeof(LineRec) <= 65536 : deg > 0;
     dim3 grid((nc + 63) / 64, (ng + VJP_GROUPS - 1) / VJP_GROUPS);
     if (staged) {
         if (!(flags & SLGPU_NOBB) && c->nion > 0) {
             if (mixed)
                 hipLaunchKernelGGL((k_vjp_opacity<true, true, 1, 8>), grid, dim3(512), bb_b + pop_b, c->stream,
                                    c->d, flags, ffc1, rgg);
-            else
-                hipLaunchKernelGGL((k_vjp_opacity<false, true, 1, 8>), grid, dim3(512), bb_b + pop_b, c->stream,
-                                   c->d, flags, ffc1, rgg);
+            else if (deg == 6) launch_vjp_lines64<6>(c, lds64);
+            else if (deg == 8) launch_vjp_lines64<8>(c, lds64);
+            else launch_vjp_lines64<10>(c, lds64);
         }
-        if (!(flags & SLGPU_NOFF) && c->d.nel > 0) {
-            if (mixed)
-                hipLaunchKernelGGL((k_vjp_opacity<true, false, 2, 4>), grid, dim3(256), ff_b, c->stream,
-                                   c->d, flags, ffc1, rgg);
-            else
-                hipLaunchKernelGGL((k_vjp_opacity<false, false, 2, 4>), grid, dim3(256), ff_b, c->stream,
-                                   c->d, flags, ffc1, rgg);
-        }
+        if (!(flags & SLGPU_NOFF) && c->d.nel > 0)
+            hipLaunchKernelGGL((k_vjp_opacity<true, false, 2, 4>), grid, dim3(256), ff_b, c->stream,
+                               c->d, flags, ffc1, rgg);
     } else if (mixed) {
         hipLaunchKernelGGL((k_vjp_opacity<true, false, 3, 4>), grid, dim3(256), acc_b, c->stream, c->d, flags, ffc1, rgg);
     } else {
         hipLaunchKernelGGL((k_vjp_opacity<false, false, 3, 4>), grid, dim3(256), acc_b, c->stream, c->d, flags, ffc1, rgg);
     }
-    if (!(flags & SLGPU_NOFF) && c->d.nel > 0)
-        hipLaunchKernelGGL(k_vjp_ff_fr, dim3((c->d.nel * nc + 255) / 256), dim3(256), 0, c->stream,
-                           c->d, rgg);
     if (!(flags & SLGPU_NOBF) && c->nion > 0)
         hipLaunchKernelGGL(k_vjp_bf_mfma, dim3((nc + 15) / 16, (c->nion + 15) / 16, BFM_SLICES),
                            dim3(64), 0, c->stream, c->d);
-    hipLaunchKernelGGL(k_vjp_finish, dim3((nc + 255) / 256), dim3(256), 0, c->stream, c->d,
-                       flags, gT, gnat, gne, gfr, goc);
+    hipLaunchKernelGGL(k_vjp_finish, dim3(nc), dim3(128), 0, c->stream, c->d, flags, nty, rgg, gT, gnat, gne,
+                       gfr, goc);
 }
 
 }  // namespace slgpu
