@@ -61,37 +61,6 @@ __device__ __forceinline__ int block_scan_int(int v, int *sh, int &total)
     return x + off;
 }
 
-// in-place running sum of row[0..n) in index order (loads batched, adds sequential)
-__device__ void running_sum(double *row, int n)
-{
-    double s = 0.0;
-    int j = 0;
-    for (; j + 8 <= n; j += 8) {
-        double v[8];
-        #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = row[j + k];
-        #pragma unroll
-        for (int k = 0; k < 8; ++k) { s = s + v[k]; row[j + k] = s; }
-    }
-    for (; j < n; ++j) { s = s + row[j]; row[j] = s; }
-}
-
-// sum of row[0..n) in index order
-__device__ double sequential_sum(const double *row, int n)
-{
-    double s = 0.0;
-    int j = 0;
-    for (; j + 8 <= n; j += 8) {
-        double v[8];
-        #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = row[j + k];
-        #pragma unroll
-        for (int k = 0; k < 8; ++k) s = s + v[k];
-    }
-    for (; j < n; ++j) s = s + row[j];
-    return s;
-}
-
 __device__ __forceinline__ double block_sum(double v, double *sh)
 {
     double t;
@@ -162,7 +131,7 @@ __device__ __forceinline__ void block_argmax_first(double &v, int &k, double *s_
     __syncthreads();
 }
 
-__global__ __launch_bounds__(NT) void k_leakage(Dev d)
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_leakage(Dev d)
 {
     __shared__ double shd[NW];
     __shared__ int shi[NW];
@@ -295,9 +264,7 @@ __global__ __launch_bounds__(NT) void k_leakage(Dev d)
     const double d2s = 1.0 / (1.0 - c_emitlump);
     double *cL = d.cumL + (size_t)(l - 1) * ng, *cR = d.cumR + (size_t)(l - 1) * ng;
     double *cD = d.cumD + (size_t)(l - 1) * ng, *cS = d.cumS + (size_t)(l - 1) * ng;
-    // terms in parallel, then each row's running sum in index order by one lane: the
-    // reference accumulates sequentially, and a sequential sum of nonnegative terms is
-    // monotone (a parallel scan is not, by rounding), which the samplers' searches need
+    // the rows' terms; k_row_sums turns them into running sums
     for (int p = threadIdx.x; p < nl_eff; p += NT) {
         // the Doppler scan runs ascending for redshift, descending for blueshift
         const int pd = divv >= 0 ? p : nl_eff - 1 - p;
@@ -319,27 +286,149 @@ __global__ __launch_bounds__(NT) void k_leakage(Dev d)
         const int g = gorder[p];
         cS[p] = spec[g - 1] * CAPE(g, l) * cgi * d2s;     // diffusion11.f90:574-581
     }
+}
+
+// The running sums of the cells' sampling rows (the four lumped rows of k_leakage) and of their source
+// spectra, normalised Planck at T_rad (interior_source.f90:69-75, 96-103).  The reference
+// accumulates sequentially, and a sequential sum of nonnegative terms is monotone (a parallel
+// scan is not, by rounding), which the samplers' searches need.  So each row is one lane's
+// chain of additions, 6 clocks each, and the work is to keep everything else off the chain:
+//   - an LDS access takes the pipe as long for 1 lane as for 64, so a block takes RS_ROWS rows,
+//     one per lane of its first wave (one row per block: 37 ns per value with the chip full);
+//   - the other eight waves store the tile before and fetch the tile after meanwhile;
+//   - the chain's LDS reads run 16 values ahead, in two register sets that take turns.
+// The source rows, which have two chains, start first.  400 x 10^4: 0.85 ms for the same chains on
+// global memory, 0.23 ms so (12 ns per value of the longest chain, the two source passes).
+constexpr int RS_ROWS = 8, RS_TILE = 256, RS_PITCH = RS_TILE + 2, RS_AHEAD = 16;
+constexpr int RS_THREADS = 576, RS_MOVERS = RS_THREADS - 64;
+
+// s and the running sums of the RS_TILE values of buf from s on, in index order
+__device__ __forceinline__ double chain_sum(double *buf, double s)
+{
+    double v[RS_AHEAD], w[RS_AHEAD];
+    #pragma unroll
+    for (int k = 0; k < RS_AHEAD; ++k) v[k] = buf[k];
+    #pragma unroll 1
+    for (int j = 0; j < RS_TILE; j += 2 * RS_AHEAD) {
+        #pragma unroll
+        for (int k = 0; k < RS_AHEAD; ++k) w[k] = buf[j + RS_AHEAD + k];
+        __builtin_amdgcn_sched_barrier(0);
+        #pragma unroll
+        for (int k = 0; k < RS_AHEAD; ++k) { s = s + v[k]; v[k] = s; }
+        #pragma unroll
+        for (int k = 0; k < RS_AHEAD; ++k) buf[j + k] = v[k];
+        __builtin_amdgcn_sched_barrier(0);
+        const int q = j + 2 * RS_AHEAD < RS_TILE ? j + 2 * RS_AHEAD : j;
+        #pragma unroll
+        for (int k = 0; k < RS_AHEAD; ++k) v[k] = buf[q + k];
+        __builtin_amdgcn_sched_barrier(0);
+        #pragma unroll
+        for (int k = 0; k < RS_AHEAD; ++k) { s = s + w[k]; w[k] = s; }
+        #pragma unroll
+        for (int k = 0; k < RS_AHEAD; ++k) buf[j + RS_AHEAD + k] = w[k];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    return s;
+}
+
+// For the block's rows r: sums of p[r][0..n[r]) / div[r] in index order, on lane r of the first
+// wave; OUT: the running sums replace the row.  nmax: the longest row.
+template <bool OUT>
+__device__ __forceinline__ double rows_sum(double *const *p, const int *n, const double *div, int nmax,
+                                           double (*buf)[RS_ROWS][RS_PITCH])
+{
+    constexpr int PER = RS_ROWS * RS_TILE / RS_MOVERS;
+    const int t = threadIdx.x, lt = t - 64, ntile = (nmax + RS_TILE - 1) / RS_TILE;
+    double s = 0.0;
+    for (int c = -1; c <= ntile; ++c) {
+        if (t >= 64) {
+            double v[PER];
+            #pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const int e = lt + q * RS_MOVERS, r = e / RS_TILE, j = (c + 1) * RS_TILE + e % RS_TILE;
+                v[q] = j < n[r] ? p[r][j] : 0.0;
+            }
+            #pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const int e = lt + q * RS_MOVERS, r = e / RS_TILE, k = e % RS_TILE, j = (c - 1) * RS_TILE + k;
+                if (OUT && c > 0 && j < n[r]) p[r][j] = buf[(c - 1) % 3][r][k];
+                if (c < ntile) buf[(c + 1) % 3][r][k] = OUT ? v[q] / div[r] : v[q];
+            }
+        } else if (t < RS_ROWS && c >= 0 && c < ntile) {
+            s = chain_sum(buf[c % 3][t], s);
+        }
+        __syncthreads();
+    }
+    return s;
+}
+
+// the source spectrum's terms (interior_source.f90:69-75)
+__global__ __launch_bounds__(256) void k_src_terms(Dev d)
+{
+    const int g = blockIdx.x * 256 + threadIdx.x + 1, l = blockIdx.y;
+    if (g <= d.ng) d.srccum[(size_t)l * d.ng + g - 1] = specintv_g(1.0 / d.radtemp[l], d.wlinv, g);
+}
+
+__global__ __launch_bounds__(RS_THREADS) void k_row_sums(Dev d)
+{
+    __shared__ __align__(16) double buf[3][RS_ROWS][RS_PITCH];
+    __shared__ double *p[RS_ROWS];
+    __shared__ double div[RS_ROWS];
+    __shared__ int n[RS_ROWS], s_max;
+    const int ng = d.ng, row = (int)blockIdx.y - 1, t = threadIdx.x;
+    if (t == 0) s_max = 0;
     __syncthreads();
-    if (threadIdx.x == 0) running_sum(cL, nl_eff);
-    else if (threadIdx.x == 64) running_sum(cR, nl_eff);
-    else if (threadIdx.x == 128) running_sum(cD, nl_eff);
-    else if (threadIdx.x == 192) running_sum(cS + nl_eff, ng - nl_eff);
+    if (t < RS_ROWS) {
+        const int l = blockIdx.x * RS_ROWS + t, lc = l < d.nx ? l : d.nx - 1;
+        const int nl = d.cell[lc].nlump;
+        double *base = row < 0 ? d.srccum : (row == 0 ? d.cumL : (row == 1 ? d.cumR : (row == 2 ? d.cumD : d.cumS + nl)));
+        int m = row < 0 ? ng : (nl == 0 ? 0 : (row == 3 ? ng - nl : nl));
+        if (l >= d.nx) m = 0;
+        p[t] = base + (size_t)lc * ng;
+        n[t] = m;
+        div[t] = 1.0;
+        atomicMax(&s_max, m);
+    }
+    __syncthreads();
+    if (s_max == 0) return;
+    if (row < 0) {
+        const double s = rows_sum<false>(p, n, div, s_max, buf);
+        if (t < RS_ROWS) div[t] = s;
+        __syncthreads();
+    }
+    rows_sum<true>(p, n, div, s_max, buf);
 }
 
 // emission_probability.f90:39-62 (grd_capemit, grd_capemitgrey in NLTE) and the in-bin
-// cumulative sums emitgroup.f:38-50 walks
+// cumulative sums emitgroup.f:38-50 walks.  A thread adds up a bin, in order; S: the cell's rows
+// pass through LDS both ways, since a wave's bins lie nepg groups apart (400 x 10^4: 87 us with
+// the strided global accesses, 53 us so).
+template <bool S>
 __global__ __launch_bounds__(256) void k_emitprob(Dev d)
 {
+    extern __shared__ double s_spec[];                         // ng doubles, then ng floats
     __shared__ double binsum[1024];
     __shared__ double pref[1025];
     const int ng = d.ng, nep = d.nep, nepg = d.nepg;
     const int l = blockIdx.x + 1;
     const double *spec = d.specarr + (size_t)(l - 1) * ng;
+    const float *cap = d.capem32 + (size_t)(l - 1) * ng;
+    double *cum = d.emitcum + (size_t)(l - 1) * ng, *out = cum;
+    if constexpr (S) {
+        float *s_cap = reinterpret_cast<float *>(s_spec + ng);
+        for (int g = threadIdx.x; g < ng; g += 256) {
+            s_spec[g] = spec[g];
+            s_cap[g] = cap[g];
+        }
+        __syncthreads();
+        spec = s_spec;
+        cap = s_cap;
+        out = s_spec;
+    }
     for (int b = threadIdx.x; b < nep; b += 256) {
-        const int g0 = b * nepg + 1;
         const int g1 = (b + 1) * nepg < ng ? (b + 1) * nepg : ng;
         double s = 0.0;
-        for (int g = g0; g <= g1; ++g) s += spec[g - 1] * CAPE(g, l);
+        for (int g = b * nepg; g < g1; ++g) s = fma(spec[g], (double)cap[g], s);
         binsum[b] = s;
     }
     __syncthreads();
@@ -349,81 +438,150 @@ __global__ __launch_bounds__(256) void k_emitprob(Dev d)
         pref[0] = 0.0;
         for (int iep = 1; iep <= nep - 1; ++iep) {
             help = help + binsum[iep - 1];
-            ep[iep - 1] = help;
             pref[iep] = help;
         }
-        ep[nep - 1] = d.capemgrey[l - 1];
     }
     __syncthreads();
-    double *cum = d.emitcum + (size_t)(l - 1) * ng;
     for (int b = threadIdx.x; b < nep; b += 256) {
-        const int g0 = b * nepg + 1;
+        ep[b] = b < nep - 1 ? pref[b + 1] : d.capemgrey[l - 1];
         const int g1 = (b + 1) * nepg < ng ? (b + 1) * nepg : ng;
         double s = pref[b];
-        for (int g = g0; g <= g1; ++g) {
-            s = s + spec[g - 1] * CAPE(g, l);
-            cum[g - 1] = s;
+        for (int g = b * nepg; g < g1; ++g) {
+            s = fma(spec[g], (double)cap[g], s);
+            out[g] = s;
         }
+    }
+    if constexpr (S) {
+        __syncthreads();
+        const int n = nep * nepg < ng ? nep * nepg : ng;
+        for (int g = threadIdx.x; g < n; g += 256) cum[g] = s_spec[g];
     }
 }
 
-// normalised Planck at T_rad and its cumulative (interior_source.f90:69-75, 96-103):
-// terms in parallel; the normalising sum and the running sum in group order, as the
-// reference's loops do
-__global__ __launch_bounds__(NT) void k_srccum(Dev d)
+// first index j in [from, n) with cum[j] > r of a monotone row whose entries before `from` are not:
+// steps that double, then a search between the last two
+__device__ __forceinline__ int first_above_from(const double *cum, int from, int n, double r)
 {
-    __shared__ double s_norm;
-    const int ng = d.ng;
-    const int l = blockIdx.x;
-    const double tr = 1.0 / d.radtemp[l];
-    double *cum = d.srccum + (size_t)l * ng;
-    for (int g = threadIdx.x + 1; g <= ng; g += NT) cum[g - 1] = specintv_g(tr, d.wlinv, g);
-    __syncthreads();
-    if (threadIdx.x == 0) s_norm = sequential_sum(cum, ng);
-    __syncthreads();
-    const double s = s_norm;
-    for (int g = threadIdx.x + 1; g <= ng; g += NT) cum[g - 1] = cum[g - 1] / s;
-    __syncthreads();
-    if (threadIdx.x == 0) running_sum(cum, ng);
+    int lo = from, step = 1;
+    while (lo < n && !(cum[lo + step <= n ? lo + step - 1 : n - 1] > r)) {
+        lo = lo + step < n ? lo + step : n;
+        step <<= 1;
+    }
+    return lo >= n ? n : first_above(cum, lo, lo + step <= n ? lo + step - 1 : n - 1, r);
 }
 
-// exact bucket maps of the five group samplers; one thread per (bucket, cell, table)
-__global__ __launch_bounds__(256) void k_bucket_tables(Dev d)
+// Exact bucket maps of the five group samplers: one block per (cell, table), which searches the
+// row in LDS (S; rows past the CU's LDS are searched in global memory), each thread a stretch
+// of 16 buckets.  The answers of a stretch rise, so each search starts from the one before.
+// They change hands in LDS: the entries are then made in bucket order, where neighbouring lanes
+// load the same groups' opacities and store side by side.  400 x 10^4: 200 us, against 640 us
+// with two full searches per bucket on global memory; random LDS reads and the gathers bound it.
+template <bool S>
+__global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
 {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    const int ic = blockIdx.y + 1, t = blockIdx.z;
-    if (b >= BT_K) return;
+    extern __shared__ double s_row[];
+    constexpr int PER = BT_K / 1024;
+    const int ic = blockIdx.x + 1, t = blockIdx.y, ng = d.ng, nep = d.nep, nepg = d.nepg;
     uint32_t *row = d.btab + ((size_t)t * d.nx + (ic - 1)) * BT_K;
-    const double rlo = bt_lo(b), rhi = bt_hi(b);
-    uint32_t e = 0;
-    if (t == TAB_E) {
-        const int glo = emitgroup_direct(d, rlo, ic), ghi = emitgroup_direct(d, rhi, ic);
-        if (glo == ghi) e = BT_PURE | dest_flags(d, t, ic, glo) | (uint32_t)glo;
-        else e = ((uint32_t)ghi << 15) | (uint32_t)glo;
-    } else {
-        const LumpRow L = lump_row(d, t, ic, d.cell[ic - 1].nlump);
-        if (L.cnt > 0) {                    // rows of cells without lumping are never sampled
-            const int jlo = first_above(L.cum, 0, L.cnt, rlo);
-            const int jhi = first_above(L.cum, 0, L.cnt, rhi);
-            const int plo = jlo < L.cnt ? jlo : L.cnt - 1, phi = jhi < L.cnt ? jhi : L.cnt - 1;
-            if (plo == phi) {
-                const int g = lump_group(d, L, ic, jlo);
-                e = BT_PURE | dest_flags(d, t, ic, g) | (uint32_t)g;
-            } else {
-                e = ((uint32_t)jhi << 15) | (uint32_t)jlo;
-            }
-        }
+    const bool emit = t == TAB_E;
+    const int nlump = d.cell[ic - 1].nlump;
+    const LumpRow L = lump_row(d, emit ? TAB_S : t, ic, nlump);
+    if (!emit && (nlump == 0 || L.cnt <= 0)) {     // rows of cells without lumping are never sampled
+        for (int b = threadIdx.x; b < BT_K; b += 1024) row[b] = 0u;
+        return;
     }
-    row[b] = e;
+    const double *cum = emit ? d.emitcum + (size_t)(ic - 1) * ng : L.cum;
+    const double *ep = d.emitprob + (size_t)(ic - 1) * nep;
+    const int n = emit ? ng : L.cnt;
+    __shared__ int s_nan;
+    if (threadIdx.x == 0) s_nan = 0;
+    __syncthreads();
+    for (int k = threadIdx.x; k < n; k += 1024) {
+        const double v = cum[k];
+        if constexpr (S) s_row[k] = v;
+        if (v != v) s_nan = 1;
+    }
+    if constexpr (S) {
+        if (emit)
+            for (int k = threadIdx.x; k < nep; k += 1024) s_row[ng + k] = ep[k];
+        cum = s_row;
+        ep = s_row + ng;
+    }
+    __syncthreads();
+    // a row with a NaN (see slgpu_sample.h) keeps two searches of the whole row per bucket
+    const bool whole = s_nan != 0;
+    const double cg = d.capemgrey[ic - 1];
+    const int b0 = threadIdx.x * PER;
+    uint32_t ans[PER];
+    int at = 0;
+    #pragma unroll
+    for (int k = 0; k < 2 * PER; ++k) {
+        const double r = k & 1 ? bt_hi(b0 + k / 2) : bt_lo(b0 + k / 2);
+        int v;
+        if (emit) {
+            const double r1 = r * cg;
+            if (k == 0 || whole) {
+                v = emitgroup_search(d, r1, ep, cum);
+            } else {
+                // the bin index and the place in the bin resume at the answer before
+                int iep = (at - 1) / nepg;
+                while (iep < nep - 1 && ep[iep] <= r1) ++iep;
+                const int ig = iep * nepg + 1, igp1 = ig + nepg - 1 < ng ? ig + nepg - 1 : ng;
+                v = first_above_from(cum, (ig > at ? ig : at) - 1, igp1 - 1, r1) + 1;
+            }
+        } else {
+            v = k == 0 || whole ? first_above(cum, 0, n, r) : first_above_from(cum, at, n, r);
+        }
+        at = v;
+        ans[k / 2] = k & 1 ? ans[k / 2] | (uint32_t)v << 15 : (uint32_t)v;
+    }
+    __syncthreads();
+    uint32_t *s_ans = reinterpret_cast<uint32_t *>(s_row);
+    #pragma unroll
+    for (int k = 0; k < PER; ++k) s_ans[b0 + k] = ans[k];
+    __syncthreads();
+    // a pure bucket's group and its destination's flags: the cell lc that receives the particle
+    // (none past the outer face: it escapes) and the group a Doppler event shifts it to
+    const int lc = t == TAB_L ? ic - 1 : (t == TAB_R ? ic + 1 : ic), shift = t != TAB_D ? 0 : (d.divv[ic - 1] >= 0 ? 1 : -1);
+    const bool inside = lc >= 1 && lc <= d.nx;
+    const int ls = inside ? lc : ic;
+    const double dx = d.xarr[ls] - d.xarr[ls - 1], sg = d.sig[ls - 1];
+    const bool lumps = d.cell[ls - 1].nlump > 0;
+    #pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int b = threadIdx.x + k * 1024;
+        uint32_t e = s_ans[b];
+        const int lo = (int)(e & 0x7fffu), hi = (int)(e >> 15);
+        const bool pure = emit ? lo == hi : (lo < n ? lo : n - 1) == (hi < n ? hi : n - 1);
+        const int g = !pure ? 0 : (emit ? lo : lump_group(d, L, ic, lo));
+        if (g > 0) {
+            int g2 = g + shift;
+            g2 = g2 < 1 ? 1 : (g2 > ng ? ng : g2);
+            const double cp = cap_of(d, g2, ls);
+            const bool thin = d.puretran || (sg + cp) * dx < d.tauddmc;
+            e = BT_PURE | (uint32_t)g;
+            if (inside) e |= thin ? BT_THIN : (cp * dx >= d.taulump && lumps ? BT_LUMP : 0u);
+        }
+        row[b] = e;
+    }
 }
 
 void launch_ddmc_tables(slgpu_ctx *c)
 {
     hipLaunchKernelGGL(k_leakage, dim3(c->nx), dim3(NT), 0, c->stream, c->d);
-    hipLaunchKernelGGL(k_emitprob, dim3(c->nx), dim3(256), 0, c->stream, c->d);
-    hipLaunchKernelGGL(k_bucket_tables, dim3(BT_K / 256, c->nx, NTAB), dim3(256), 0, c->stream,
-                       c->d);
-    hipLaunchKernelGGL(k_srccum, dim3(c->nx), dim3(NT), 0, c->stream, c->d);
+    hipLaunchKernelGGL(k_src_terms, dim3((c->ng + 255) / 256, c->nx), dim3(256), 0, c->stream, c->d);
+    hipLaunchKernelGGL(k_row_sums, dim3((c->nx + RS_ROWS - 1) / RS_ROWS, 5), dim3(RS_THREADS), 0, c->stream, c->d);
+    const size_t rows = (size_t)c->ng * (sizeof(double) + sizeof(float));
+    if (rows <= 143000)                            // beside 16 KB of bin sums
+        hipLaunchKernelGGL(k_emitprob<true>, dim3(c->nx), dim3(256), rows, c->stream, c->d);
+    else
+        hipLaunchKernelGGL(k_emitprob<false>, dim3(c->nx), dim3(256), 0, c->stream, c->d);
+    const size_t lds = (size_t)(c->ng + c->d.nep) * sizeof(double), answers = BT_K * sizeof(uint32_t);
+    if (lds <= 160000)
+        hipLaunchKernelGGL(k_bucket_tables<true>, dim3(c->nx, NTAB), dim3(1024), lds > answers ? lds : answers,
+                           c->stream, c->d);
+    else
+        hipLaunchKernelGGL(k_bucket_tables<false>, dim3(c->nx, NTAB), dim3(1024), answers, c->stream, c->d);
 }
 
 }  // namespace slgpu

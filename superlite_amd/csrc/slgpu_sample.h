@@ -89,20 +89,23 @@ __device__ __forceinline__ int first_above(const double *__restrict__ cum, int l
     return lo;
 }
 
-// GRID/emitgroup.f:3-54 by direct search: binsrch over the binned emission probabilities,
-// then the first group of the bin whose running sum exceeds r*capgrey (r*capemitgrey in NLTE)
-__device__ __forceinline__ int emitgroup_direct(const Dev &d, double r, int ic)
+// GRID/emitgroup.f:3-54 by direct search: binsrch over the binned emission probabilities ep,
+// then the first group of the bin whose running sum cum exceeds r1 = r*capgrey (r*capemitgrey in
+// NLTE)
+__device__ __forceinline__ int emitgroup_search(const Dev &d, double r1, const double *ep, const double *cum)
 {
-    const int ng = d.ng;
-    const double *ep = d.emitprob + (size_t)(ic - 1) * d.nep;
-    const double r1 = r * d.capemgrey[ic - 1];
     int iep = binsrch(r1, ep, d.nep, true);
     if (iep > d.nep - 1) iep = d.nep - 1;
     if (iep < 0) iep = 0;
     const int ig = iep * d.nepg + 1;
-    const int igp1 = ig + d.nepg - 1 < ng ? ig + d.nepg - 1 : ng;
-    const double *cum = d.emitcum + (size_t)(ic - 1) * ng;
+    const int igp1 = ig + d.nepg - 1 < d.ng ? ig + d.nepg - 1 : d.ng;
     return first_above(cum, ig - 1, igp1 - 1, r1) + 1;
+}
+
+__device__ __forceinline__ int emitgroup_direct(const Dev &d, double r, int ic)
+{
+    return emitgroup_search(d, r * d.capemgrey[ic - 1], d.emitprob + (size_t)(ic - 1) * d.nep,
+                            d.emitcum + (size_t)(ic - 1) * d.ng);
 }
 
 // emitgroup restricted to results in [glo, ghi]: the bin index (binsrch with widerange,
@@ -149,21 +152,6 @@ __device__ __forceinline__ int lump_group(const Dev &d, const LumpRow &L, int ic
 {
     const int pos = L.rev ? (j < L.cnt ? L.cnt - 1 - j : 0) : L.lo + (j < L.cnt ? j : L.cnt - 1);
     return d.gorder[(size_t)(ic - 1) * d.ng + pos];
-}
-
-// BT_THIN / BT_LUMP of the group a table's event moves the particle to, in the cell that
-// receives it (0 past the outer face: the particle escapes instead)
-__device__ __forceinline__ uint32_t dest_flags(const Dev &d, int t, int ic, int iiig)
-{
-    int lc = ic, g = iiig;
-    if (t == TAB_L) lc = ic - 1;
-    else if (t == TAB_R) lc = ic + 1;
-    else if (t == TAB_D) {
-        if (d.divv[ic - 1] >= 0) g = iiig + 1 > d.ng ? d.ng : iiig + 1;
-        else g = iiig - 1 < 1 ? 1 : iiig - 1;
-    }
-    if (lc < 1 || lc > d.nx) return 0u;
-    return group_flags(d, g, lc);
 }
 
 // sampled group of table t in cell ic for draw r, given the draw's bucket entry e of that

@@ -1112,7 +1112,7 @@ __global__ __launch_bounds__(256) void k_sample_groups(Dev d, int t, int direct,
     const int nlump = d.cell[ic - 1].nlump;
     if (t != TAB_E) {
         const LumpRow L = lump_row(d, t, ic, nlump);
-        if (L.cnt == 0) { out[k] = 0; return; }
+        if (nlump == 0 || L.cnt == 0) { out[k] = 0; return; }
         if (direct) { out[k] = lump_group(d, L, ic, first_above(L.cum, 0, L.cnt, r[k])); return; }
     } else if (direct) {
         out[k] = emitgroup_direct(d, r[k], ic);
