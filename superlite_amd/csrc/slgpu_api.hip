@@ -508,7 +508,7 @@ static int upload_lines(slgpu_ctx *c)
         top = std::max(top, (double)q.chilw);
     }
     c->line_top = plain && !recs.empty() ? std::max(top, 1.0) : 0.0;
-    if (c->cfg.precision == SLGPU_FP64) rc = build_lines64(c);
+    if (c->cfg.precision == SLGPU_FP64 || c->have_nlte) rc = build_lines64(c);
     HIPCHK(hipStreamSynchronize(c->stream));
     return rc;
 }
@@ -776,20 +776,20 @@ int slgpu_set_nlte_data(slgpu_ctx *c, int nlev, int nlin, int ncoll, const doubl
         igs[k] = (g >= 1 && g <= ng) ? g : 0;
         if (igs[k]) cnt[igs[k]]++;
     }
-    std::vector<int> hstart(ng + 2, 0), hidx;
+    std::vector<int> hstart(ng + 2, 0);
     for (int g = 1; g <= ng; ++g) hstart[g + 1] = hstart[g] + cnt[g];
     std::vector<int> fill(hstart);
-    hidx.assign(std::max(hstart[ng + 1], 1), 0);
+    std::vector<HLine> hline(std::max(hstart[ng + 1], 1));
     for (int k = 0; k < nlin; ++k)
-        if (igs[k]) hidx[fill[igs[k]]++] = k;
+        if (igs[k]) hline[fill[igs[k]]++] = {f[k], gl[k], gu[k], aul[k], wl0[k], llw[k] - 1, lup[k] - 1};
     int kH = -1;
     for (int k = 0; k < c->nion; ++k)
         if (c->h_ion_iz[k] == 1 && c->h_ion_ii[k] == 1) kH = k;
     NlteDev &q = c->nl;
     if (c->have_nlte) {
-        void *ps[] = {q.glev, q.wl0, q.f, q.gl, q.gu, q.aul, q.bul, q.blu, q.cc, q.dele, q.pic, q.rrc,
-                      q.delepi, q.llw, q.lup, q.igs, q.cl, q.cu, q.levpi, q.hstart, q.hidx, q.radtemp,
-                      q.ndens, q.rc, q.A, q.pop, q.gpi, q.ipiv, q.flag, q.capemitT, q.emissT,
+        void *ps[] = {q.glev, q.aul, q.bul, q.blu, q.cc, q.dele, q.pic, q.rrc,
+                      q.delepi, q.llw, q.lup, q.igs, q.cl, q.cu, q.levpi, q.hstart, q.hline, q.radtemp,
+                      q.ndens, q.A, q.pop, q.popT, q.flag, q.capemitT, q.emissT,
                       q.capemit32, q.capemitgrey};
         for (void *p : ps) dfree(c, p);
         c->have_nlte = false;
@@ -806,19 +806,17 @@ int slgpu_set_nlte_data(slgpu_ctx *c, int nlev, int nlin, int ncoll, const doubl
     const int nc1 = std::max(ncoll, 1);
     int rc = 0;
     rc |= dalloc(c, &q.glev, nlev);
-    rc |= dalloc(c, &q.wl0, nlin); rc |= dalloc(c, &q.f, nlin); rc |= dalloc(c, &q.gl, nlin);
-    rc |= dalloc(c, &q.gu, nlin); rc |= dalloc(c, &q.aul, nlin); rc |= dalloc(c, &q.bul, nlin);
-    rc |= dalloc(c, &q.blu, nlin);
+    rc |= dalloc(c, &q.aul, nlin); rc |= dalloc(c, &q.bul, nlin); rc |= dalloc(c, &q.blu, nlin);
     rc |= dalloc(c, &q.cc, (size_t)4 * nc1); rc |= dalloc(c, &q.dele, nc1);
     rc |= dalloc(c, &q.pic, (size_t)4 * nlev); rc |= dalloc(c, &q.rrc, (size_t)4 * nlev);
     rc |= dalloc(c, &q.delepi, nlev);
     rc |= dalloc(c, &q.llw, nlin); rc |= dalloc(c, &q.lup, nlin); rc |= dalloc(c, &q.igs, nlin);
     rc |= dalloc(c, &q.cl, nc1); rc |= dalloc(c, &q.cu, nc1); rc |= dalloc(c, &q.levpi, nlev);
-    rc |= dalloc(c, &q.hstart, ng + 2); rc |= dalloc(c, &q.hidx, hidx.size());
+    rc |= dalloc(c, &q.hstart, ng + 2); rc |= dalloc(c, &q.hline, hline.size());
     rc |= dalloc(c, &q.radtemp, nc); rc |= dalloc(c, &q.ndens, (size_t)2 * nc);
-    rc |= dalloc(c, &q.rc, (size_t)nc * nlev * nlev); rc |= dalloc(c, &q.A, (size_t)nc * nlev * nlev);
-    rc |= dalloc(c, &q.pop, (size_t)nc * nlev); rc |= dalloc(c, &q.gpi, (size_t)nc * nlev);
-    rc |= dalloc(c, &q.ipiv, (size_t)nc * nlev); rc |= dalloc(c, &q.flag, 1);
+    if (!nlte_in_lds(nlev)) rc |= dalloc(c, &q.A, (size_t)nc * nlev * (nlev + 1));
+    rc |= dalloc(c, &q.pop, (size_t)nc * nlev); rc |= dalloc(c, &q.popT, (size_t)nc * nlev);
+    rc |= dalloc(c, &q.flag, 1);
     rc |= dalloc(c, &q.capemitT, (size_t)nc * ng); rc |= dalloc(c, &q.emissT, (size_t)nc * ng);
     rc |= dalloc(c, &q.capemit32, (size_t)nc * ng); rc |= dalloc(c, &q.capemitgrey, nc);
     if (rc) return rc;
@@ -826,9 +824,7 @@ int slgpu_set_nlte_data(slgpu_ctx *c, int nlev, int nlin, int ncoll, const doubl
         return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream);
     };
     HIPCHK(up(q.glev, glev, nlev * 8));
-    HIPCHK(up(q.wl0, wl0, nlin * 8)); HIPCHK(up(q.f, f, nlin * 8)); HIPCHK(up(q.gl, gl, nlin * 8));
-    HIPCHK(up(q.gu, gu, nlin * 8)); HIPCHK(up(q.aul, aul, nlin * 8)); HIPCHK(up(q.bul, bul, nlin * 8));
-    HIPCHK(up(q.blu, blu, nlin * 8));
+    HIPCHK(up(q.aul, aul, nlin * 8)); HIPCHK(up(q.bul, bul, nlin * 8)); HIPCHK(up(q.blu, blu, nlin * 8));
     if (ncoll > 0) {
         HIPCHK(up(q.cc, coll_c, (size_t)4 * ncoll * 8)); HIPCHK(up(q.dele, dele, ncoll * 8));
         HIPCHK(up(q.cl, llw_coll, ncoll * 4)); HIPCHK(up(q.cu, lup_coll, ncoll * 4));
@@ -837,10 +833,12 @@ int slgpu_set_nlte_data(slgpu_ctx *c, int nlev, int nlin, int ncoll, const doubl
     HIPCHK(up(q.delepi, dele_pi, nlev * 8));
     HIPCHK(up(q.llw, llw, nlin * 4)); HIPCHK(up(q.lup, lup, nlin * 4)); HIPCHK(up(q.igs, igs.data(), nlin * 4));
     HIPCHK(up(q.levpi, lev_pi, nlev * 4));
-    HIPCHK(up(q.hstart, hstart.data(), (ng + 2) * 4)); HIPCHK(up(q.hidx, hidx.data(), hidx.size() * 4));
+    HIPCHK(up(q.hstart, hstart.data(), (ng + 2) * 4)); HIPCHK(up(q.hline, hline.data(), hline.size() * sizeof(HLine)));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->have_nlte = true;
-    return 0;
+    rc = build_lines64(c);          // NLTE builds take the FP64 line sums in both precision forms
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return rc;
 }
 
 int slgpu_opacity_build_nlte(slgpu_ctx *c, const slgpu_gas *gas, const double *radtemp,

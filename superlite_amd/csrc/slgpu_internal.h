@@ -155,21 +155,42 @@ struct Dev {
 
 // NLTE hydrogen (physical_opacity_nlte.f): the species data of slgpu_set_nlte_data, the
 // per-call inputs and the work arrays, passed by value to the NLTE kernels only.
+// One NLTE line, in the order of its group; a wave reads it as one uniform record.
+struct HLine {
+    double f, gl, gu, aul, wl0;
+    int lw, lu;                                 // level indices from 0
+};
+
+// What the (cell, group) kernel of an NLTE build needs beside Dev.
+struct NlteOut {
+    const int *hstart;
+    const HLine *hline;
+    const double *popT, *ndens;                 // (n, nc), (nc, 2)
+    double *capemitT, *emissT;                  // (ng, nc)
+};
+
 struct NlteDev {
     int n = 0, nlin = 0, ncoll = 0, kH = -1;    // levels, lines, collision lines, H I ion index
-    double *glev, *wl0, *f, *gl, *gu, *aul, *bul, *blu;   // nlev / nlin
+    double *glev, *aul, *bul, *blu;             // nlev / nlin
     double *cc, *dele;                          // 4*ncoll, ncoll
     double *pic, *rrc, *delepi;                 // 4*nlev, 4*nlev, nlev
     int *llw, *lup, *igs;                       // nlin (igs: group of the line, 0 outside)
     int *cl, *cu, *levpi;                       // ncoll, ncoll, nlev
-    int *hstart, *hidx;                         // ng+2 offsets, the lines by group in file order
+    int *hstart;                                // ng+2 offsets
+    HLine *hline;                               // the lines by group, in file order
     double *radtemp, *ndens;                    // nc, 2*nc (H I, H II per cell)
-    double *rc, *A, *pop, *gpi;                 // nc*n*n, nc*n*n, nc*n, nc*n
-    int *ipiv, *flag;                           // nc*n, 1
+    double *A;                                  // nc*n*(n+1), where the matrix does not fit LDS
+    double *pop, *popT;                         // nc*n, and its transpose
+    int *flag;                                  // 1
     double *capemitT, *emissT;                  // (ng, nc) cell-fastest
     float *capemit32;                           // (nc, ng)
     double *capemitgrey;                        // nc
 };
+
+inline __host__ __device__ NlteOut nlte_out(const NlteDev &q)
+{
+    return {q.hstart, q.hline, q.popT, q.ndens, q.capemitT, q.emissT};
+}
 
 constexpr int GACC_COPIES = 8;          // copies of the backward's most contended accumulators
 inline size_t vjp_acc_doubles(int nion, size_t nc)
@@ -234,6 +255,8 @@ void launch_opacity_finish(slgpu_ctx *c);
 void launch_cell_tables(slgpu_ctx *c);
 void launch_opacity_nlte(slgpu_ctx *c, int flags, double ffc1, const double *rgg);
 void launch_nlte_means(slgpu_ctx *c);
+bool nlte_in_lds(int n);
+bool launch_opacity64_nlte(slgpu_ctx *c, int flags, double ffc1, const double *rgg);
 double ff_prefactor();
 const double *rgg_scratch(slgpu_ctx *c);
 void launch_opacity_vjp(slgpu_ctx *c, int flags, const double *gc, const double *gp,
@@ -307,6 +330,25 @@ template <int DEG>
 __device__ __forceinline__ double line_exp(const Line64 &q, const double *e_lane, double nh)
 {
     return row_at(e_lane, q.k1) * row_at(e_lane, q.k2) * exp_poly<DEG>(q.r * nh);
+}
+
+// The NLTE species' lines of group g in cell ic (physical_opacity_nlte.f:304-345): absorption with
+// stimulated emission from the populations and emission, bnu the group centre's Planck function
+__device__ __forceinline__ void nlte_lines(const NlteOut &q, int g, int ic, int nc, double phi, double bnu,
+                                           double &cap, double &cape, double &em)
+{
+#pragma clang fp contract(off)
+    const double fconst = PC_PI * (PC_E * PC_E) / (PC_ME * PC_C);
+    const double nd = q.ndens[2 * (size_t)ic], *pop = q.popT + ic;
+    for (int h = q.hstart[g]; h < q.hstart[g + 1]; ++h) {
+        const HLine r = q.hline[h];                     // uniform: scalar loads
+        const double npl = pop[(size_t)r.lw * nc] * nd;
+        const double npu = pop[(size_t)r.lu * nc] * nd;
+        cap += npl * fconst * r.f * phi * (1.0 - (npu * r.gl / (npl * r.gu)));
+        const double emithelp = npu * r.aul * phi * PC_H * PC_C / (4.0 * PC_PI * (r.wl0 * PC_ANG));
+        cape += emithelp / bnu;
+        em += emithelp;
+    }
 }
 
 // physical_opacity.f:228-243: sum over elements of g_ff(u, gamma^2) z^2 natomfr for cell ic at

@@ -344,12 +344,14 @@ __global__ __launch_bounds__(256) void k_exp_table(Dev d)
 // c2 (400 x 10^4 x 2e6 lines): 1.08 ms with exp() per line and the reference's product, 0.48 ms
 // so; c5 (1000 x 10^4 x 4e6) 4.15 -> 1.92 ms; 64 x 250 x 1e5 53 -> 13 us.  What bounds it now is FP64
 // issue: 15 vector operations per line, 78% of the issue slots.
-template <int DEG, int WPG>
+// NLTE: the build of slgpu_nlte.hip, its other species' lines as one sum for cap, capemit and emiss
+// (c2: 1.11 ms with exp() per line and three sums, 0.52 ms so).
+template <int DEG, int WPG, bool NLTE>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_opacity64(Dev d, int flags, double ffc1,
                                                     const double *__restrict__ rgg_tab,
                                                     const Line64 *__restrict__ lines,
                                                     const int *__restrict__ gstart,
-                                                    const double *__restrict__ etab)
+                                                    const double *__restrict__ etab, NlteOut q, int kskip)
 {
     extern __shared__ __align__(16) unsigned char s_raw[];
     double *s_e = reinterpret_cast<double *>(s_raw);           // EXP_ROWS x 64
@@ -376,7 +378,8 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
         for (int k = threadIdx.x; k < d.nion * 64; k += 1024) {
             const int cc = c0 + (k & 63);
             const double o = cc < nc ? d.ocg[(size_t)(k >> 6) * nc + cc] : 0.0;
-            s_pop[k] = o > 0.0 ? o : 0.0;                      // the reference skips such ions
+            // the reference skips such ions, and the NLTE species' lines are not LTE lines
+            s_pop[k] = o > 0.0 && !(NLTE && (k >> 6) == kskip) ? o : 0.0;
         }
         asm volatile("" ::"v"(touched));
         __syncthreads();
@@ -423,6 +426,28 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     if (g > ng) return;
     const bool massive = act && d.mass[ic] > 0.0;
     const double wlo = d.wl[g - 1], whi = d.wl[g];
+    if constexpr (NLTE) {
+        double cap = 0.0, cape = 0.0, em = 0.0;
+        if (bb && massive) {
+            const double wlc = 0.5 * (wlo + whi), phi = wlc * wlc / ((whi - wlo) * PC_C);
+            const double T = d.temp[ic], bnu = (wlc * wlc / PC_C) * planck(wlc, T);
+            nlte_lines(q, g, ic, nc, phi, bnu, cap, cape, em);
+            const double lte = sum * phi * (1.0 - exp(-hckt * (1.0 / wlc)));
+            cap += lte;
+            cape += lte;
+            em += lte * bnu;
+        }
+        double cont = 0.0;                                     // bf and ff: left edge
+        if (!(flags & SLGPU_NOBF)) cont = bf_add(d, g, ic, cont);
+        if (!(flags & SLGPU_NOFF)) cont += ff_term(d, hckt, wlo, ic, ffc1, rgg_tab);
+        if (act) {
+            const size_t o = (size_t)(g - 1) * nc + i;
+            d.capT[o] = massive ? cap + cont : 0.0;
+            q.capemitT[o] = massive ? cape + cont : 0.0;
+            q.emissT[o] = massive ? em + cont * ((wlo * wlo / PC_C) * planck(wlo, d.temp[ic])) : 0.0;
+        }
+        return;
+    }
     double acc = 0.0;
     if (bb) {
         // physical_opacity.f:128-137: subgroup-centre profile and stimulated emission
@@ -572,24 +597,53 @@ int line_degree(const slgpu_ctx *c)
     return x <= 0.0177 ? 6 : (x <= 0.069 ? 8 : (x <= 0.176 ? 10 : 0));
 }
 
-template <int DEG>
-static void launch_opacity64(slgpu_ctx *c, int flags, double ffc1, const double *rgg, size_t lds)
+// LDS of k_opacity64: tables, populations and the waves' partial sums
+static size_t opacity64_lds(const slgpu_ctx *c)
+{
+    return ((size_t)EXP_ROWS + c->nion + 16) * 64 * sizeof(double);
+}
+
+// the polynomial's degree where k_opacity64 applies (its LDS within the CU's 160 KiB), else 0
+static int opacity64_degree(const slgpu_ctx *c)
+{
+    return c->force_unstaged || opacity64_lds(c) > 163840 ? 0 : line_degree(c);
+}
+
+template <int DEG, bool NLTE>
+static void launch_opacity64(slgpu_ctx *c, int flags, double ffc1, const double *rgg)
 {
     // Waves per group: the chip holds 8192 waves of this kernel, which one per group fills at
     // c2 (70000); smaller grids share a group's lines among 4 or 16 (64 x 250 x 1e5 lines, 250
     // waves: 13 us with 16, against the 53 us of the form with one wave per group and exp()).
     const int64_t waves = (int64_t)((c->nx + 63) / 64) * c->ng;
     const unsigned cb = (c->nx + 63) / 64;
+    const size_t lds = opacity64_lds(c);
     const Dev &d = c->d;
+    const NlteOut q = NLTE ? nlte_out(c->nl) : NlteOut();
     if (waves >= 8192)
-        hipLaunchKernelGGL((k_opacity64<DEG, 1>), dim3(cb * ((c->ng + 15) / 16)), dim3(1024), lds, c->stream, d,
-                           flags, ffc1, rgg, d.lines64, d.gstart, d.etab);
+        hipLaunchKernelGGL((k_opacity64<DEG, 1, NLTE>), dim3(cb * ((c->ng + 15) / 16)), dim3(1024), lds, c->stream,
+                           d, flags, ffc1, rgg, d.lines64, d.gstart, d.etab, q, c->nl.kH);
     else if (waves >= 2048)
-        hipLaunchKernelGGL((k_opacity64<DEG, 4>), dim3(cb * ((c->ng + 3) / 4)), dim3(1024), lds, c->stream, d,
-                           flags, ffc1, rgg, d.lines64, d.gstart, d.etab);
+        hipLaunchKernelGGL((k_opacity64<DEG, 4, NLTE>), dim3(cb * ((c->ng + 3) / 4)), dim3(1024), lds, c->stream,
+                           d, flags, ffc1, rgg, d.lines64, d.gstart, d.etab, q, c->nl.kH);
     else
-        hipLaunchKernelGGL((k_opacity64<DEG, 16>), dim3(cb * c->ng), dim3(1024), lds, c->stream, d, flags, ffc1,
-                           rgg, d.lines64, d.gstart, d.etab);
+        hipLaunchKernelGGL((k_opacity64<DEG, 16, NLTE>), dim3(cb * c->ng), dim3(1024), lds, c->stream, d, flags,
+                           ffc1, rgg, d.lines64, d.gstart, d.etab, q, c->nl.kH);
+}
+
+template <bool NLTE> static bool launch_opacity64(slgpu_ctx *c, int flags, double ffc1, const double *rgg)
+{
+    switch (opacity64_degree(c)) {
+    case 6: launch_opacity64<6, NLTE>(c, flags, ffc1, rgg); return true;
+    case 8: launch_opacity64<8, NLTE>(c, flags, ffc1, rgg); return true;
+    case 10: launch_opacity64<10, NLTE>(c, flags, ffc1, rgg); return true;
+    default: return false;
+    }
+}
+
+bool launch_opacity64_nlte(slgpu_ctx *c, int flags, double ffc1, const double *rgg)
+{
+    return launch_opacity64<true>(c, flags, ffc1, rgg);
 }
 
 void launch_opacity(slgpu_ctx *c, int flags)
@@ -601,22 +655,13 @@ void launch_opacity(slgpu_ctx *c, int flags)
     // the 4 KiB of line records
     const size_t lds = (size_t)c->nion * 64 * sizeof(float);
     const bool staged = !c->force_unstaged && c->nion > 0 && lds <= 65536;
-    // FP64: tables, populations and the waves' partial sums within the CU's 160 KiB
-    const size_t lds64 = ((size_t)EXP_ROWS + c->nion + 16) * 64 * sizeof(double);
-    const int deg = c->force_unstaged || lds64 > 163840 ? 0 : line_degree(c);
     if (c->d.precision == SLGPU_MIXED && staged)
         hipLaunchKernelGGL((k_opacity<true, true>), grid, dim3(256), lds, c->stream, c->d, flags,
                            ffc1, rgg);
     else if (c->d.precision == SLGPU_MIXED)
         hipLaunchKernelGGL((k_opacity<true, false>), grid, dim3(256), 0, c->stream, c->d, flags,
                            ffc1, rgg);
-    else if (deg == 6)
-        launch_opacity64<6>(c, flags, ffc1, rgg, lds64);
-    else if (deg == 8)
-        launch_opacity64<8>(c, flags, ffc1, rgg, lds64);
-    else if (deg == 10)
-        launch_opacity64<10>(c, flags, ffc1, rgg, lds64);
-    else
+    else if (!launch_opacity64<false>(c, flags, ffc1, rgg))
         hipLaunchKernelGGL((k_opacity<false, false>), grid, dim3(256), 0, c->stream, c->d, flags,
                            ffc1, rgg);
 }
