@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -76,6 +77,22 @@ int dalloc(slgpu_ctx *c, T **p, size_t n)
     return 0;
 }
 
+// one allocation for several arrays, one directly behind the other (multiples of 4 bytes; 8-byte
+// elements before 4-byte ones)
+int dparts(slgpu_ctx *c, std::initializer_list<std::pair<void **, size_t>> parts)
+{
+    size_t n = 0;
+    for (const auto &x : parts) n += x.second;
+    char *p = nullptr;
+    const int rc = dalloc(c, &p, n);
+    if (rc) return rc;
+    for (const auto &x : parts) {
+        *x.first = p;
+        p += x.second;
+    }
+    return 0;
+}
+
 void dfree(slgpu_ctx *c, void *p)
 {
     if (!p) return;
@@ -88,10 +105,10 @@ struct PhaseTimer {
     slgpu_ctx *c;
     int slot;
     PhaseTimer(slgpu_ctx *c_, int s) : c(c_), slot(s) { hipEventRecord(c->ev[2 * s], c->stream); }
-    int stop()
+    // the phase ends when its outputs are on the host
+    int stop(Outputs &out)
     {
-        hipEventRecord(c->ev[2 * slot + 1], c->stream);
-        hipError_t e = hipEventSynchronize(c->ev[2 * slot + 1]);
+        hipError_t e = out.finish(c->ev[2 * slot + 1]);
         if (e != hipSuccess) return fail(SLGPU_EHIP, std::string("device: ") + hipGetErrorString(e));
         float ms = 0.f;
         hipEventElapsedTime(&ms, c->ev[2 * slot], c->ev[2 * slot + 1]);
@@ -213,32 +230,25 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.ffB, (size_t)nc * FF_NU);
     rc |= dalloc(c, &d.ffclamp, nc);
     rc |= dalloc(c, &d.ffC, (size_t)nc * FF_NU);
-    rc |= dalloc(c, &d.sig, nc);
     rc |= dalloc(c, &d.tempinv, nc);
-    rc |= dalloc(c, &d.temp, nc);
-    rc |= dalloc(c, &d.mass, nc);
-    rc |= dalloc(c, &d.natomfr, 30 * nc);
-    rc |= dalloc(c, &d.el_z, 30);
+    // what crosses the bus together lies together, in the order of the transfers
+    rc |= dparts(c, {{(void **)&d.temp, nc * 8}, {(void **)&d.mass, nc * 8}, {(void **)&d.natomfr, 30 * nc * 8},
+                     {(void **)&d.natom_in, nc * 8}, {(void **)&d.vol_in, nc * 8},
+                     {(void **)&d.nelec_in, nc * 8}, {(void **)&d.el_z, 30 * 4}});
+    rc |= dparts(c, {{(void **)&d.sig, nc * 8}, {(void **)&d.capgrey, nc * 8}, {(void **)&d.capross, nc * 8}});
     rc |= dalloc(c, &d.capT, cg);
     rc |= dalloc(c, &d.cap64, cg);
     rc |= dalloc(c, &d.cap32, cg);
     rc |= dalloc(c, &d.emiss, cg);
-    rc |= dalloc(c, &d.capgrey, nc);
-    rc |= dalloc(c, &d.capross, nc);
     d.capem32 = d.cap32;
     d.capemgrey = d.capgrey;
     d.nlte = 0;
     rc |= dalloc(c, &d.specarr, cg);
-    rc |= dalloc(c, &d.opaclump, 11 * nc);
-    rc |= dalloc(c, &d.emitprob, (size_t)cfg->nep * nc);
+    rc |= dparts(c, {{(void **)&d.opaclump, 11 * nc * 8}, {(void **)&d.emitprob, (size_t)cfg->nep * nc * 8}});
     rc |= dalloc(c, &d.emitcum, cg);
-    rc |= dalloc(c, &d.emit, nc);
-    rc |= dalloc(c, &d.radtemp, nc);
+    rc |= dparts(c, {{(void **)&d.emit, nc * 8}, {(void **)&d.radtemp, nc * 8}});
     rc |= dalloc(c, &d.srccum, cg);
     rc |= dalloc(c, &d.cell, nc);
-    rc |= dalloc(c, &d.natom_in, nc);
-    rc |= dalloc(c, &d.vol_in, nc);
-    rc |= dalloc(c, &d.nelec_in, nc);
     rc |= dalloc(c, &d.gcapT, cg);
     rc |= dalloc(c, &d.gmpart, (size_t)2 * ((ng + 63) / 64) * nc);
     rc |= dalloc(c, &d.ctpart, (size_t)2 * ((ng + 1023) / 1024) * nc);
@@ -262,8 +272,8 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.perr, np);
     rc |= dalloc(c, &d.pnstep, np);
     rc |= dalloc(c, &d.pix, np);
-    rc |= dalloc(c, &d.tally, nc);
-    rc |= dalloc(c, &d.eamp, nc);
+    rc |= dparts(c, {{(void **)&d.tally, nc * 8}, {(void **)&d.eamp, nc * 8}, {(void **)&d.tot, 8 * 8},
+                     {(void **)&d.ct, 10 * 8}, {(void **)&d.queue, 8}});
     // grd_jrad gets one atomic per event; on small grids every lane hits a few hot
     // (cell, group) entries, so blocks add into one of R replicas (R from a 256 MiB budget,
     // 1..32) that a reduction folds into replica 0 after the transport
@@ -273,12 +283,7 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
         d.jrad_copies = (int)(r < 1 ? 1 : (r > 32 ? 32 : r));
     }
     rc |= dalloc(c, &d.jrad, (size_t)d.jrad_copies * cg);
-    rc |= dalloc(c, &d.tot, 8);
-    rc |= dalloc(c, &d.ct, 10);
-    rc |= dalloc(c, &d.queue, 1);
-    rc |= dalloc(c, &d.lum, ng);
-    rc |= dalloc(c, &d.dev, ng);
-    rc |= dalloc(c, &d.num, ng);
+    rc |= dparts(c, {{(void **)&d.lum, ng * 8}, {(void **)&d.dev, ng * 8}, {(void **)&d.num, ng * 4}});
     rc |= dalloc(c, &d.flags, 1);
     rc |= dalloc(c, &d.eos_ni, 30);
     rc |= dalloc(c, &d.eos_e, 30 * 31);
@@ -286,13 +291,16 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.eos_g1, 30 * 31);
     rc |= dalloc(c, &d.eos_amass, 30);
     rc |= dalloc(c, &d.eos_sahac2, nc);
-    rc |= dalloc(c, &c->eos_temp, nc);
-    rc |= dalloc(c, &c->eos_mass, nc);
-    rc |= dalloc(c, &c->eos_massfr, 30 * nc);
-    rc |= dalloc(c, &c->eos_nelec, nc);
-    rc |= dalloc(c, &c->eos_natom, nc);
-    rc |= dalloc(c, &c->eos_natomfr, 30 * nc);
-    rc |= dalloc(c, &c->eos_niter, nc);
+    rc |= dparts(c, {{(void **)&c->eos_temp, nc * 8}, {(void **)&c->eos_mass, nc * 8},
+                     {(void **)&c->eos_massfr, 30 * nc * 8}, {(void **)&c->eos_nelec, nc * 8},
+                     {(void **)&c->eos_natom, nc * 8}, {(void **)&c->eos_natomfr, 30 * nc * 8},
+                     {(void **)&c->eos_niter, nc * 4}});
+    if (!rc) {
+        // inputs of a call: 35 per-cell numbers and two per ion; outputs: up to 20 bytes per (cell,
+        // group) and some hundred per cell.  What does not fit goes straight from the caller's memory.
+        const hipError_t e = c->io.create(std::min((size_t)4 << 20, nc * 167 * 8 + 4096), 20 * cg + 200 * 8 * nc);
+        if (e != hipSuccess) rc = fail(SLGPU_ENOMEM, std::string("hipHostMalloc: ") + hipGetErrorString(e));
+    }
     if (rc) {
         std::string m = g_err;
         slgpu_destroy(c);
@@ -309,6 +317,7 @@ int slgpu_destroy(slgpu_ctx *c)
     if (c->stream) hipStreamSynchronize(c->stream);
     for (void *p : c->allocations) hipFree(p);
     c->allocations.clear();
+    c->io.destroy();
     for (int k = 0; k < 24; ++k) hipEventDestroy(c->ev[k]);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
@@ -388,7 +397,9 @@ int slgpu_set_ions(slgpu_ctx *c, int nion, const int *ion_iz, const int *ion_ii)
     dfree(c, c->d.ion_z);
     dfree(c, c->d.ion_i);
     dfree(c, c->eos_oc);
-    dfree(c, c->eos_ginv);
+    dfree(c, c->stage);
+    dfree(c, c->vjp_out);
+    dfree(c, c->eos_vjp);
     dfree(c, c->d.ocg);
     dfree(c, c->d.ocT);
     dfree(c, c->d.ginvT);
@@ -405,8 +416,12 @@ int slgpu_set_ions(slgpu_ctx *c, int nion, const int *ion_iz, const int *ion_ii)
     rc |= dalloc(c, &c->d.bfmask, (size_t)(std::max(nion, 1) + 31) / 32 * c->ng);
     rc |= dalloc(c, &c->d.ion_z, std::max(nion, 1));
     rc |= dalloc(c, &c->d.ion_i, std::max(nion, 1));
-    rc |= dalloc(c, &c->eos_oc, (size_t)std::max(nion, 1) * nc);
-    rc |= dalloc(c, &c->eos_ginv, (size_t)std::max(nion, 1) * nc);
+    c->eos_oc = c->stage = c->vjp_out = c->eos_vjp = nullptr;
+    const size_t ni = std::max(nion, 1);
+    rc |= dparts(c, {{(void **)&c->eos_oc, ni * nc * 8}, {(void **)&c->eos_ginv, ni * nc * 8}});
+    rc |= dalloc(c, &c->stage, 2 * ni * nc);
+    rc |= dalloc(c, &c->vjp_out, (33 + ni) * nc);
+    rc |= dalloc(c, &c->eos_vjp, (64 + ni) * nc);
     if (rc) return rc;
     c->d.ffW = c->d.goc + (size_t)GACC_COPIES * std::max(nion, 1) * nc;
     c->d.gcell = c->d.ffW + (size_t)GACC_COPIES * FF_NU * nc;
@@ -577,7 +592,7 @@ int slgpu_set_ff_table(slgpu_ctx *c, const double *gff)
 namespace {
 
 // The opacity build (O2-O8) with the per-call staging of the ion populations oc and ginv
-// (2 * nion * nc doubles) at `stage`: a fresh allocation for slgpu_opacity_build, the
+// (2 * nion * nc doubles) at `stage`: the context's for slgpu_opacity_build, the
 // library's static scratch array for slgpu_opacity_build_noalloc.
 // the NLTE part of a build (physical_opacity_nlte): per-call inputs and extra outputs
 struct NlteCall {
@@ -593,7 +608,7 @@ int opacity_build_impl(slgpu_ctx *c, const slgpu_gas *gas, int flags, double *ou
 {
     const int nc = c->nx, ng = c->ng, nion = c->nion;
     // present elements (ff adds exactly zero for the others, physical_opacity.f:240-241)
-    int nel = 0, elz[30];
+    int nel = 0, elz[30] = {};
     for (int z = 1; z <= 30; ++z) {
         bool any = false;
         for (int i = 0; i < nc && !any; ++i) any = gas->natomfr[(size_t)i * 30 + z - 1] != 0.0;
@@ -606,22 +621,24 @@ int opacity_build_impl(slgpu_ctx *c, const slgpu_gas *gas, int flags, double *ou
     // per-call host inputs (small: nc and nion*nc doubles)
     double *dn = c->d.natom_in, *dv = c->d.vol_in, *de = c->d.nelec_in;   // kept for the backward
     double *doc = stage, *dgi = stage + (size_t)std::max(nion, 1) * nc;
-    HIPCHK(hipMemcpyAsync(c->d.temp, gas->temp, nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d.mass, gas->mass, nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d.natomfr, gas->natomfr, (size_t)nc * 30 * 8, hipMemcpyHostToDevice, c->stream));
-    if (nel > 0) HIPCHK(hipMemcpyAsync(c->d.el_z, elz, nel * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(dn, gas->natom, nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(dv, gas->vol, nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(de, gas->nelec, nc * 8, hipMemcpyHostToDevice, c->stream));
+    Inputs in(c->io, c->stream);
+    in.add(c->d.temp, gas->temp, nc * 8);
+    in.add(c->d.mass, gas->mass, nc * 8, true);
+    in.add(c->d.natomfr, gas->natomfr, (size_t)nc * 30 * 8, true);
+    in.add(dn, gas->natom, nc * 8, true);
+    in.add(dv, gas->vol, nc * 8, true);
+    in.add(de, gas->nelec, nc * 8, true);
+    in.add(c->d.el_z, elz, sizeof(elz), true);
     if (nion > 0) {
-        HIPCHK(hipMemcpyAsync(doc, gas->oc, (size_t)nion * nc * 8, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(dgi, gas->ginv, (size_t)nion * nc * 8, hipMemcpyHostToDevice, c->stream));
+        in.add(doc, gas->oc, (size_t)nion * nc * 8);
+        in.add(dgi, gas->ginv, (size_t)nion * nc * 8, true);
     }
     if (nlc) {
-        HIPCHK(hipMemcpyAsync(c->nl.radtemp, nlc->radtemp, nc * 8, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->nl.ndens, nlc->ndens, (size_t)2 * nc * 8, hipMemcpyHostToDevice, c->stream));
+        in.add(c->nl.radtemp, nlc->radtemp, nc * 8);
+        in.add(c->nl.ndens, nlc->ndens, (size_t)2 * nc * 8, true);
         HIPCHK(hipMemsetAsync(c->nl.flag, 0, sizeof(int), c->stream));
     }
+    HIPCHK(in.send());
     hipEventRecord(c->ev[22], c->stream);
     launch_cell_prep(c, dn, dv, de, doc, dgi, flags);
     hipEventRecord(c->ev[10], c->stream);
@@ -637,29 +654,26 @@ int opacity_build_impl(slgpu_ctx *c, const slgpu_gas *gas, int flags, double *ou
     hipEventRecord(c->ev[23], c->stream);
     HIPCHK(hipGetLastError());
     const size_t cg = (size_t)nc * ng;
+    Outputs out(c->io, c->stream);
+    int flag = 0;
     if (nlc) {
-        if (nlc->out_capemit)
-            HIPCHK(hipMemcpyAsync(nlc->out_capemit, c->nl.capemit32, cg * 4, hipMemcpyDeviceToHost, c->stream));
-        if (nlc->out_capemitgrey)
-            HIPCHK(hipMemcpyAsync(nlc->out_capemitgrey, c->nl.capemitgrey, nc * 8, hipMemcpyDeviceToHost, c->stream));
-        if (nlc->out_npop)
-            HIPCHK(hipMemcpyAsync(nlc->out_npop, c->nl.pop, (size_t)nc * c->nl.n * 8, hipMemcpyDeviceToHost, c->stream));
+        out.add(&flag, c->nl.flag, sizeof(int));
+        out.add(nlc->out_capemit, c->nl.capemit32, cg * 4);
+        out.add(nlc->out_capemitgrey, c->nl.capemitgrey, nc * 8);
+        out.add(nlc->out_npop, c->nl.pop, (size_t)nc * c->nl.n * 8);
     }
-    if (out_cap64) HIPCHK(hipMemcpyAsync(out_cap64, c->d.cap64, cg * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_cap32) HIPCHK(hipMemcpyAsync(out_cap32, c->d.cap32, cg * 4, hipMemcpyDeviceToHost, c->stream));
-    if (out_emiss) HIPCHK(hipMemcpyAsync(out_emiss, c->d.emiss, cg * 4, hipMemcpyDeviceToHost, c->stream));
-    if (out_sig) HIPCHK(hipMemcpyAsync(out_sig, c->d.sig, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_capgrey) HIPCHK(hipMemcpyAsync(out_capgrey, c->d.capgrey, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_capross) HIPCHK(hipMemcpyAsync(out_capross, c->d.capross, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    int rc = tm.stop();
-    if (!rc && nlc) {
-        int flag = 0;
-        HIPCHK(hipMemcpy(&flag, c->nl.flag, sizeof(int), hipMemcpyDeviceToHost));
-        if (flag) {
-            c->have_opacity = false;        // the device opacity is partly overwritten
-            c->have_prep = false;
-            return fail(SLGPU_EINVAL, "nlte opacity: rate matrix numerically singular");
-        }
+    out.add(out_cap64, c->d.cap64, cg * 8);
+    out.add(out_cap32, c->d.cap32, cg * 4);
+    out.add(out_emiss, c->d.emiss, cg * 4);
+    out.add(out_sig, c->d.sig, nc * 8);
+    out.add(out_capgrey, c->d.capgrey, nc * 8, true);
+    out.add(out_capross, c->d.capross, nc * 8, true);
+    out.start();
+    int rc = tm.stop(out);
+    if (!rc && flag) {
+        c->have_opacity = false;            // the device opacity is partly overwritten
+        c->have_prep = false;
+        return fail(SLGPU_EINVAL, "nlte opacity: rate matrix numerically singular");
     }
     float kms = 0.f;
     hipEventElapsedTime(&kms, c->ev[10], c->ev[11]);
@@ -703,14 +717,8 @@ int slgpu_opacity_build(slgpu_ctx *c, const slgpu_gas *gas, int flags, double *o
 {
     int rc = check_opacity_inputs(c, gas);
     if (rc) return rc;
-    double *stage = nullptr;
-    rc = dalloc(c, &stage, (size_t)2 * std::max(c->nion, 1) * c->nx);
-    if (rc) return rc;
-    rc = opacity_build_impl(c, gas, flags, out_cap64, out_cap32, out_sig, out_capgrey,
-                            out_capross, out_emiss, stage);
-    hipStreamSynchronize(c->stream);
-    dfree(c, stage);
-    return rc;
+    return opacity_build_impl(c, gas, flags, out_cap64, out_cap32, out_sig, out_capgrey,
+                              out_capross, out_emiss, c->stage);
 }
 
 int slgpu_opacity_build_noalloc(slgpu_ctx *c, const slgpu_gas *gas, int flags,
@@ -789,7 +797,7 @@ int slgpu_set_nlte_data(slgpu_ctx *c, int nlev, int nlin, int ncoll, const doubl
     if (c->have_nlte) {
         void *ps[] = {q.glev, q.aul, q.bul, q.blu, q.cc, q.dele, q.pic, q.rrc,
                       q.delepi, q.llw, q.lup, q.igs, q.cl, q.cu, q.levpi, q.hstart, q.hline, q.radtemp,
-                      q.ndens, q.A, q.pop, q.popT, q.flag, q.capemitT, q.emissT,
+                      q.A, q.pop, q.popT, q.flag, q.capemitT, q.emissT,
                       q.capemit32, q.capemitgrey};
         for (void *p : ps) dfree(c, p);
         c->have_nlte = false;
@@ -813,7 +821,7 @@ int slgpu_set_nlte_data(slgpu_ctx *c, int nlev, int nlin, int ncoll, const doubl
     rc |= dalloc(c, &q.llw, nlin); rc |= dalloc(c, &q.lup, nlin); rc |= dalloc(c, &q.igs, nlin);
     rc |= dalloc(c, &q.cl, nc1); rc |= dalloc(c, &q.cu, nc1); rc |= dalloc(c, &q.levpi, nlev);
     rc |= dalloc(c, &q.hstart, ng + 2); rc |= dalloc(c, &q.hline, hline.size());
-    rc |= dalloc(c, &q.radtemp, nc); rc |= dalloc(c, &q.ndens, (size_t)2 * nc);
+    rc |= dparts(c, {{(void **)&q.radtemp, (size_t)nc * 8}, {(void **)&q.ndens, (size_t)2 * nc * 8}});
     if (!nlte_in_lds(nlev)) rc |= dalloc(c, &q.A, (size_t)nc * nlev * (nlev + 1));
     rc |= dalloc(c, &q.pop, (size_t)nc * nlev); rc |= dalloc(c, &q.popT, (size_t)nc * nlev);
     rc |= dalloc(c, &q.flag, 1);
@@ -858,15 +866,9 @@ int slgpu_opacity_build_nlte(slgpu_ctx *c, const slgpu_gas *gas, const double *r
                 return fail(SLGPU_EINVAL, "nlte opacity: radtemp and the H I density must be positive "
                                           "and the H II density non-negative in every massive cell");
         }
-    double *stage = nullptr;
-    rc = dalloc(c, &stage, (size_t)2 * std::max(c->nion, 1) * c->nx);
-    if (rc) return rc;
     NlteCall nlc{radtemp, ndens, out_capemit, out_capemitgrey, out_npop};
-    rc = opacity_build_impl(c, gas, flags, out_cap64, out_cap32, out_sig, out_capgrey,
-                            out_capross, out_emiss, stage, &nlc);
-    hipStreamSynchronize(c->stream);
-    dfree(c, stage);
-    return rc;
+    return opacity_build_impl(c, gas, flags, out_cap64, out_cap32, out_sig, out_capgrey,
+                              out_capross, out_emiss, c->stage, &nlc);
 }
 
 int slgpu_nlte_rad_est(slgpu_ctx *c, double *radtemp, double *out_jrad)
@@ -876,20 +878,22 @@ int slgpu_nlte_rad_est(slgpu_ctx *c, double *radtemp, double *out_jrad)
     const int nc = c->nx, ng = c->ng;
     for (int i = 0; i < nc; ++i)
         if (!(radtemp[i] > 0.0)) return fail(SLGPU_EINVAL, "grd_radtemp must be positive");
-    double *drt = nullptr, *dj = nullptr;
-    int rc = dalloc(c, &drt, nc);
-    if (!rc && out_jrad) rc = dalloc(c, &dj, (size_t)nc * ng);
-    if (!rc) {
-        HIPCHK(hipMemcpyAsync(drt, radtemp, nc * 8, hipMemcpyHostToDevice, c->stream));
-        launch_nlte_rad_est(c, drt, dj);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(radtemp, drt, nc * 8, hipMemcpyDeviceToHost, c->stream));
-        if (dj) HIPCHK(hipMemcpyAsync(out_jrad, dj, (size_t)nc * ng * 8, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
+    if (!c->est) {
+        int rc = dalloc(c, &c->est, (size_t)nc * (ng + 1));
+        if (rc) return rc;
     }
-    if (drt) dfree(c, drt);
-    if (dj) dfree(c, dj);
-    return rc;
+    double *drt = c->est, *dj = out_jrad ? c->est + nc : nullptr;
+    Inputs in(c->io, c->stream);
+    in.add(drt, radtemp, nc * 8);
+    HIPCHK(in.send());
+    launch_nlte_rad_est(c, drt, dj);
+    HIPCHK(hipGetLastError());
+    Outputs out(c->io, c->stream);
+    out.add(radtemp, drt, nc * 8);
+    out.add(out_jrad, dj, (size_t)nc * ng * 8, true);
+    out.start();
+    HIPCHK(out.finish(c->ev[1]));
+    return 0;
 }
 
 int slgpu_ddmc_prep(slgpu_ctx *c, const double *radtemp, double lbol, double *out_opaclump,
@@ -911,14 +915,18 @@ int slgpu_ddmc_prep(slgpu_ctx *c, const double *radtemp, double lbol, double *ou
     double st = 0.0;
     for (int i = 0; i < nc; ++i) { emit[i] = emit[i] / s * lbol; st += emit[i]; }
     PhaseTimer tm(c, 1);
-    HIPCHK(hipMemcpyAsync(c->d.emit, emit.data(), nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d.radtemp, radtemp, nc * 8, hipMemcpyHostToDevice, c->stream));
+    Inputs in(c->io, c->stream);
+    in.add(c->d.emit, emit.data(), nc * 8);
+    in.add(c->d.radtemp, radtemp, nc * 8, true);
+    HIPCHK(in.send());
     launch_ddmc_tables(c);
     launch_ddmc_probs(c);
     HIPCHK(hipGetLastError());
-    if (out_opaclump) HIPCHK(hipMemcpyAsync(out_opaclump, c->d.opaclump, (size_t)11 * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_emitprob) HIPCHK(hipMemcpyAsync(out_emitprob, c->d.emitprob, (size_t)c->cfg.nep * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    int rc = tm.stop();
+    Outputs out(c->io, c->stream);
+    out.add(out_opaclump, c->d.opaclump, (size_t)11 * nc * 8);
+    out.add(out_emitprob, c->d.emitprob, (size_t)c->cfg.nep * nc * 8, true);
+    out.start();
+    int rc = tm.stop(out);
     if (rc) return rc;
     if (out_emit) std::memcpy(out_emit, emit.data(), nc * 8);
     if (out_sthermal) *out_sthermal = st;
@@ -941,14 +949,18 @@ int slgpu_sources(slgpu_ctx *c, int64_t nstot, uint32_t iteration, int *out_nvol
     std::vector<int64_t> pstart(c->nx + 1, 0);
     for (int i = 0; i < c->nx; ++i) pstart[i + 1] = pstart[i] + nvol[i];
     PhaseTimer tm(c, 2);
-    HIPCHK(hipMemcpyAsync((void *)c->d.pstart, pstart.data(), (c->nx + 1) * 8, hipMemcpyHostToDevice, c->stream));
+    Inputs in(c->io, c->stream);
+    in.add((void *)c->d.pstart, pstart.data(), (c->nx + 1) * 8);
+    HIPCHK(in.send());
     HIPCHK(hipMemsetAsync(c->d.flags, 0, 4, c->stream));
     c->d.npart = nnew;
     launch_sources(c, iteration);
     HIPCHK(hipGetLastError());
     int flag = 0;
-    HIPCHK(hipMemcpyAsync(&flag, c->d.flags, 4, hipMemcpyDeviceToHost, c->stream));
-    int rc = tm.stop();
+    Outputs out(c->io, c->stream);
+    out.add(&flag, c->d.flags, 4);
+    out.start();
+    int rc = tm.stop(out);
     if (rc) return rc;
     if (flag) return fail(SLGPU_EINVAL, "interior_source: position rejection did not terminate");
     if (out_nvol) std::memcpy(out_nvol, nvol.data(), c->nx * sizeof(int));
@@ -966,25 +978,23 @@ int slgpu_transport(slgpu_ctx *c, uint32_t iteration, double *out_tally, double 
     const int nc = c->nx, ng = c->ng;
     PhaseTimer tm(c, 3);
     // particle_advance.f90:65-67: zero the tallies
-    HIPCHK(hipMemsetAsync(c->d.tally, 0, nc * 8, c->stream));
-    HIPCHK(hipMemsetAsync(c->d.eamp, 0, nc * 8, c->stream));
+    HIPCHK(hipMemsetAsync(c->d.tally, 0, (size_t)2 * nc * 8 + (8 + 10 + 1) * 8, c->stream));   // to the queue
     HIPCHK(hipMemsetAsync(c->d.jrad, 0, (size_t)c->d.jrad_copies * nc * ng * 8, c->stream));
-    HIPCHK(hipMemsetAsync(c->d.tot, 0, 8 * 8, c->stream));
-    HIPCHK(hipMemsetAsync(c->d.ct, 0, 10 * 8, c->stream));
     hipEventRecord(c->ev[12], c->stream);
-    HIPCHK(hipMemsetAsync(c->d.queue, 0, 8, c->stream));
     launch_transport(c, iteration);
     hipEventRecord(c->ev[13], c->stream);
     launch_jrad_reduce(c);
     HIPCHK(hipGetLastError());
     double tot[8];
     unsigned long long ct[10];
-    HIPCHK(hipMemcpyAsync(tot, c->d.tot, 8 * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(ct, c->d.ct, 10 * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_tally) HIPCHK(hipMemcpyAsync(out_tally, c->d.tally, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_eamp) HIPCHK(hipMemcpyAsync(out_eamp, c->d.eamp, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_jrad) HIPCHK(hipMemcpyAsync(out_jrad, c->d.jrad, (size_t)nc * ng * 8, hipMemcpyDeviceToHost, c->stream));
-    int rc = tm.stop();
+    Outputs out(c->io, c->stream);
+    out.add(out_jrad, c->d.jrad, (size_t)nc * ng * 8);
+    out.add(out_tally, c->d.tally, nc * 8);
+    out.add(out_eamp, c->d.eamp, nc * 8, true);
+    out.add(tot, c->d.tot, 8 * 8, true);
+    out.add(ct, c->d.ct, 10 * 8, true);
+    out.start();
+    int rc = tm.stop(out);
     if (rc) return rc;
     float kms = 0.f;
     hipEventElapsedTime(&kms, c->ev[12], c->ev[13]);
@@ -1006,15 +1016,15 @@ int slgpu_fluxtally(slgpu_ctx *c, double *out_luminos, double *out_lumdev, int *
     if (!c->have_transport) return fail(SLGPU_EORDER, "slgpu_transport must run first");
     const int ng = c->ng;
     PhaseTimer tm(c, 4);
-    HIPCHK(hipMemsetAsync(c->d.lum, 0, ng * 8, c->stream));
-    HIPCHK(hipMemsetAsync(c->d.dev, 0, ng * 8, c->stream));
-    HIPCHK(hipMemsetAsync(c->d.num, 0, ng * 4, c->stream));
+    HIPCHK(hipMemsetAsync(c->d.lum, 0, (size_t)ng * 20, c->stream));       // lum, dev and num
     launch_fluxtally(c);
     HIPCHK(hipGetLastError());
-    if (out_luminos) HIPCHK(hipMemcpyAsync(out_luminos, c->d.lum, ng * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_lumdev) HIPCHK(hipMemcpyAsync(out_lumdev, c->d.dev, ng * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_lumnum) HIPCHK(hipMemcpyAsync(out_lumnum, c->d.num, ng * 4, hipMemcpyDeviceToHost, c->stream));
-    return tm.stop();
+    Outputs out(c->io, c->stream);
+    out.add(out_luminos, c->d.lum, ng * 8);
+    out.add(out_lumdev, c->d.dev, ng * 8, true);
+    out.add(out_lumnum, c->d.num, ng * 4, true);
+    out.start();
+    return tm.stop(out);
 }
 
 int slgpu_get_particles(slgpu_ctx *c, int64_t n, uint8_t *stat, double *x, double *mu,
@@ -1022,15 +1032,17 @@ int slgpu_get_particles(slgpu_ctx *c, int64_t n, uint8_t *stat, double *x, doubl
 {
     if (!c) return fail(SLGPU_EINVAL, "null context");
     if (n < 0 || n > c->d.npart) return fail(SLGPU_EINVAL, "n exceeds the particle count");
-    if (stat) HIPCHK(hipMemcpyAsync(stat, c->d.pstat, n, hipMemcpyDeviceToHost, c->stream));
-    if (x) HIPCHK(hipMemcpyAsync(x, c->d.px, n * 8, hipMemcpyDeviceToHost, c->stream));
-    if (mu) HIPCHK(hipMemcpyAsync(mu, c->d.pmu, n * 8, hipMemcpyDeviceToHost, c->stream));
-    if (wl) HIPCHK(hipMemcpyAsync(wl, c->d.pwl, n * 8, hipMemcpyDeviceToHost, c->stream));
-    if (e) HIPCHK(hipMemcpyAsync(e, c->d.pe, n * 8, hipMemcpyDeviceToHost, c->stream));
-    if (ig) HIPCHK(hipMemcpyAsync(ig, c->d.pig, n * 4, hipMemcpyDeviceToHost, c->stream));
-    if (nstep) HIPCHK(hipMemcpyAsync(nstep, c->d.pnstep, n * 8, hipMemcpyDeviceToHost, c->stream));
-    if (err) HIPCHK(hipMemcpyAsync(err, c->d.perr, n * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    Outputs out(c->io, c->stream);
+    out.add(x, c->d.px, n * 8);
+    out.add(mu, c->d.pmu, n * 8);
+    out.add(wl, c->d.pwl, n * 8);
+    out.add(e, c->d.pe, n * 8);
+    out.add(nstep, c->d.pnstep, n * 8);
+    out.add(ig, c->d.pig, n * 4);
+    out.add(err, c->d.perr, n * 4);
+    out.add(stat, c->d.pstat, n);
+    out.start();
+    HIPCHK(out.finish(c->ev[5]));
     return 0;
 }
 
@@ -1049,38 +1061,41 @@ int opacity_vjp_impl(slgpu_ctx *c, bool dev, const double *grad_cap64, const dou
         return fail(SLGPU_EINVAL, "opacity backward: ions + elements exceed 128 per cell");
     PhaseTimer tm(c, 7);
     const size_t cg = (size_t)nc * ng;
-    double *dgc = nullptr, *dgp = nullptr, *dgr = nullptr, *out = nullptr;
-    int rc = 0;
+    double *dgc = nullptr, *dgp = nullptr, *dgr = nullptr;
     if (!dev) {
-        if (grad_cap64) rc |= dalloc(c, &dgc, cg);
-        if (grad_capgrey) rc |= dalloc(c, &dgp, nc);
-        if (grad_capross) rc |= dalloc(c, &dgr, nc);
+        if (!c->vjp_in) {
+            int rc = dalloc(c, &c->vjp_in, cg + 2 * (size_t)nc);
+            if (rc) return rc;
+        }
+        if (grad_cap64) dgc = c->vjp_in + 2 * (size_t)nc;
+        if (grad_capgrey) dgp = c->vjp_in;
+        if (grad_capross) dgr = c->vjp_in + nc;
     }
-    const size_t nout = (size_t)nc * (3 + 30 + std::max(nion, 1));
-    rc |= dalloc(c, &out, nout);
-    if (rc) return rc;
-    if (dgc) HIPCHK(hipMemcpyAsync(dgc, grad_cap64, cg * 8, hipMemcpyHostToDevice, c->stream));
-    if (dgp) HIPCHK(hipMemcpyAsync(dgp, grad_capgrey, nc * 8, hipMemcpyHostToDevice, c->stream));
-    if (dgr) HIPCHK(hipMemcpyAsync(dgr, grad_capross, nc * 8, hipMemcpyHostToDevice, c->stream));
+    Inputs in(c->io, c->stream);
+    if (dgp) in.add(dgp, grad_capgrey, nc * 8);
+    if (dgr) in.add(dgr, grad_capross, nc * 8, true);
+    if (dgc) in.add(dgc, grad_cap64, cg * 8, true);
+    HIPCHK(in.send());
     const double *igc = dev ? grad_cap64 : dgc, *igp = dev ? grad_capgrey : dgp, *igr = dev ? grad_capross : dgr;
-    double *gT = out, *gn = out + nc, *ge = out + 2 * nc, *gf = out + 3 * nc, *go = out + 33 * (size_t)nc;
+    double *gT = c->vjp_out, *gn = gT + nc, *ge = gT + 2 * nc, *gf = gT + 3 * nc, *go = gT + 33 * (size_t)nc;
     hipEventRecord(c->ev[20], c->stream);
     launch_opacity_vjp(c, c->opac_flags, igc, igp, igr, gT, gn, ge, gf, go, ff_prefactor(),
                        rgg_scratch(c));
     hipEventRecord(c->ev[21], c->stream);
     HIPCHK(hipGetLastError());
-    if (out_grad_temp) HIPCHK(hipMemcpyAsync(out_grad_temp, gT, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_grad_natom) HIPCHK(hipMemcpyAsync(out_grad_natom, gn, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_grad_nelec) HIPCHK(hipMemcpyAsync(out_grad_nelec, ge, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_grad_natomfr) HIPCHK(hipMemcpyAsync(out_grad_natomfr, gf, (size_t)30 * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_grad_oc && nion > 0) HIPCHK(hipMemcpyAsync(out_grad_oc, go, (size_t)nion * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    rc = tm.stop();
+    Outputs out(c->io, c->stream);
+    out.add(out_grad_temp, gT, nc * 8);
+    out.add(out_grad_natom, gn, nc * 8, true);
+    out.add(out_grad_nelec, ge, nc * 8, true);
+    out.add(out_grad_natomfr, gf, (size_t)30 * nc * 8, true);
+    out.add(out_grad_oc, go, (size_t)nion * nc * 8, true);
+    out.start();
+    const int rc = tm.stop(out);
     if (!rc) {
         float kms = 0.f;
         hipEventElapsedTime(&kms, c->ev[20], c->ev[21]);
         c->t_ms[10] += kms;
     }
-    dfree(c, dgc); dfree(c, dgp); dfree(c, dgr); dfree(c, out);
     return rc;
 }
 }  // namespace
@@ -1196,22 +1211,26 @@ int slgpu_eos(slgpu_ctx *c, const double *temp, const double *mass, const double
     if (!(acc > 0.0)) acc = 1e-8;                            // ionsmod.f:183
     PhaseTimer tm(c, 8);
     HIPCHK(hipMemsetAsync(c->d.flags, 0, 4, c->stream));
-    HIPCHK(hipMemcpyAsync(c->eos_temp, temp, nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->eos_mass, mass, nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->eos_massfr, massfr, (size_t)30 * nc * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->eos_nelec, nelec, nc * 8, hipMemcpyHostToDevice, c->stream));
+    Inputs in(c->io, c->stream);
+    in.add(c->eos_temp, temp, nc * 8);
+    in.add(c->eos_mass, mass, nc * 8, true);
+    in.add(c->eos_massfr, massfr, (size_t)30 * nc * 8, true);
+    in.add(c->eos_nelec, nelec, nc * 8, true);
+    HIPCHK(in.send());
     launch_eos(c, c->eos_temp, c->eos_mass, c->eos_massfr, acc, c->eos_nelec, c->eos_natom,
                c->eos_natomfr, c->eos_oc, c->eos_ginv, c->eos_niter);
     HIPCHK(hipGetLastError());
     int flag = 0;
-    HIPCHK(hipMemcpyAsync(&flag, c->d.flags, 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(nelec, c->eos_nelec, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_natom) HIPCHK(hipMemcpyAsync(out_natom, c->eos_natom, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_natomfr) HIPCHK(hipMemcpyAsync(out_natomfr, c->eos_natomfr, (size_t)30 * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_oc && nion > 0) HIPCHK(hipMemcpyAsync(out_oc, c->eos_oc, (size_t)nion * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_ginv && nion > 0) HIPCHK(hipMemcpyAsync(out_ginv, c->eos_ginv, (size_t)nion * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_niter) HIPCHK(hipMemcpyAsync(out_niter, c->eos_niter, nc * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    int rc = tm.stop();
+    Outputs out(c->io, c->stream);
+    out.add(&flag, c->d.flags, 4);
+    out.add(nelec, c->eos_nelec, nc * 8);
+    out.add(out_natom, c->eos_natom, nc * 8, true);
+    out.add(out_natomfr, c->eos_natomfr, (size_t)30 * nc * 8, true);
+    out.add(out_niter, c->eos_niter, nc * sizeof(int), true);
+    out.add(out_oc, c->eos_oc, (size_t)nion * nc * 8);
+    out.add(out_ginv, c->eos_ginv, (size_t)nion * nc * 8, true);
+    out.start();
+    int rc = tm.stop(out);
     if (rc) return rc;
     if (flag) {
         c->have_eos = false;
@@ -1226,14 +1245,16 @@ int slgpu_eos_nlte_ndens(slgpu_ctx *c, double *out_ndens)
     if (!c || !out_ndens) return fail(SLGPU_EINVAL, "null argument");
     if (!c->have_eos) return fail(SLGPU_EORDER, "slgpu_eos must run first");
     const int nc = c->nx;
-    double *dn = nullptr;
-    int rc = dalloc(c, &dn, (size_t)2 * nc);
-    if (rc) return rc;
-    launch_eos_ndens(c, c->eos_temp, c->eos_mass, c->eos_natom, c->eos_natomfr, dn);
+    if (!c->ndens) {
+        int rc = dalloc(c, &c->ndens, (size_t)2 * nc);
+        if (rc) return rc;
+    }
+    launch_eos_ndens(c, c->eos_temp, c->eos_mass, c->eos_natom, c->eos_natomfr, c->ndens);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out_ndens, dn, (size_t)2 * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    dfree(c, dn);
+    Outputs out(c->io, c->stream);
+    out.add(out_ndens, c->ndens, (size_t)2 * nc * 8);
+    out.start();
+    HIPCHK(out.finish(c->ev[17]));
     return 0;
 }
 
@@ -1245,25 +1266,27 @@ int slgpu_eos_vjp(slgpu_ctx *c, const double *grad_natom, const double *grad_nat
     if (!c->have_eos) return fail(SLGPU_EORDER, "slgpu_eos must run first");
     const int nc = c->nx, nion = c->nion;
     PhaseTimer tm(c, 9);
-    double *buf = nullptr;
-    const size_t nin = (size_t)nc * (2 + 30 + std::max(nion, 1)), nout = (size_t)nc * 32;
-    int rc = dalloc(c, &buf, nin + nout);
-    if (rc) return rc;
+    double *buf = c->eos_vjp;
+    const size_t nin = (size_t)nc * (2 + 30 + std::max(nion, 1));
     double *gna = buf, *gne = buf + nc, *gfr = buf + 2 * (size_t)nc, *goc = buf + 32 * (size_t)nc;
     double *oT = buf + nin, *om = oT + nc, *omf = om + nc;
-    if (grad_natom) HIPCHK(hipMemcpyAsync(gna, grad_natom, nc * 8, hipMemcpyHostToDevice, c->stream));
-    if (grad_nelec) HIPCHK(hipMemcpyAsync(gne, grad_nelec, nc * 8, hipMemcpyHostToDevice, c->stream));
-    if (grad_natomfr) HIPCHK(hipMemcpyAsync(gfr, grad_natomfr, (size_t)30 * nc * 8, hipMemcpyHostToDevice, c->stream));
-    if (grad_oc && nion > 0) HIPCHK(hipMemcpyAsync(goc, grad_oc, (size_t)nion * nc * 8, hipMemcpyHostToDevice, c->stream));
+    if (!(grad_natom && grad_nelec && grad_natomfr && grad_oc))     // gradients not given are zero
+        HIPCHK(hipMemsetAsync(buf, 0, nin * 8, c->stream));
+    Inputs in(c->io, c->stream);
+    if (grad_natom) in.add(gna, grad_natom, nc * 8);
+    if (grad_nelec) in.add(gne, grad_nelec, nc * 8, true);
+    if (grad_natomfr) in.add(gfr, grad_natomfr, (size_t)30 * nc * 8, true);
+    if (grad_oc) in.add(goc, grad_oc, (size_t)nion * nc * 8, true);
+    HIPCHK(in.send());
     launch_eos_vjp(c, c->eos_temp, c->eos_mass, c->eos_massfr, c->eos_nelec, c->eos_natom,
                    c->eos_natomfr, c->eos_oc, gna, gfr, gne, goc, oT, om, omf);
     HIPCHK(hipGetLastError());
-    if (out_grad_temp) HIPCHK(hipMemcpyAsync(out_grad_temp, oT, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_grad_mass) HIPCHK(hipMemcpyAsync(out_grad_mass, om, nc * 8, hipMemcpyDeviceToHost, c->stream));
-    if (out_grad_massfr) HIPCHK(hipMemcpyAsync(out_grad_massfr, omf, (size_t)30 * nc * 8, hipMemcpyDeviceToHost, c->stream));
-    rc = tm.stop();
-    dfree(c, buf);
-    return rc;
+    Outputs out(c->io, c->stream);
+    out.add(out_grad_temp, oT, nc * 8);
+    out.add(out_grad_mass, om, nc * 8, true);
+    out.add(out_grad_massfr, omf, (size_t)30 * nc * 8, true);
+    out.start();
+    return tm.stop(out);
 }
 
 int slgpu_timers(slgpu_ctx *c, double *ms, int n, int reset)

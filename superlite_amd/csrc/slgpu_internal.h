@@ -9,6 +9,7 @@
 
 #include "../../include/slgpu.h"
 #include "slgpu_device.h"
+#include "slgpu_hostio.h"
 
 namespace slgpu {
 
@@ -231,6 +232,10 @@ struct slgpu_ctx {
     double *eos_temp = nullptr, *eos_mass = nullptr, *eos_massfr = nullptr, *eos_nelec = nullptr,
            *eos_natom = nullptr, *eos_natomfr = nullptr, *eos_oc = nullptr, *eos_ginv = nullptr;
     int *eos_niter = nullptr;
+    double *stage = nullptr;    // ion populations of an opacity build (oc, ginv)
+    double *vjp_out = nullptr, *vjp_in = nullptr, *eos_vjp = nullptr;   // backward's workspaces
+    double *est = nullptr, *ndens = nullptr;        // slgpu_nlte_rad_est, slgpu_eos_nlte_ndens
+    slgpu::HostIO io;
     slgpu::NlteDev nl;          // NLTE species data and work arrays (slgpu_set_nlte_data)
     bool have_nlte = false;
     void *scratch = nullptr;    // device address of the library's static scratch array on this context's GPU

@@ -186,9 +186,9 @@ class Context:
                 _c(oc, np.float64), _c(ginv, np.float64)]
         gas = Gas(*[_p(x) for x in keep])
         out = {}
-        if "cap64" in want: out["cap64"] = np.zeros((nc, ng))
-        if "cap" in want: out["cap"] = np.zeros((nc, ng), np.float32)
-        if "emiss" in want: out["emiss"] = np.zeros((nc, ng), np.float32)
+        if "cap64" in want: out["cap64"] = np.empty((nc, ng))
+        if "cap" in want: out["cap"] = np.empty((nc, ng), np.float32)
+        if "emiss" in want: out["emiss"] = np.empty((nc, ng), np.float32)
         for k in ("sig", "capgrey", "capross"):
             if k in want: out[k] = np.zeros(nc)
         self.builds += 1
@@ -226,8 +226,8 @@ class Context:
                 _c(oc, np.float64), _c(ginv, np.float64)]
         gas = Gas(*[_p(x) for x in keep])
         rt, nd = _c(radtemp, np.float64), _c(ndens, np.float64)
-        out = dict(cap64=np.zeros((nc, ng)), cap=np.zeros((nc, ng), np.float32),
-                   capemit=np.zeros((nc, ng), np.float32), emiss=np.zeros((nc, ng), np.float32),
+        out = dict(cap64=np.empty((nc, ng)), cap=np.empty((nc, ng), np.float32),
+                   capemit=np.empty((nc, ng), np.float32), emiss=np.empty((nc, ng), np.float32),
                    sig=np.zeros(nc), capgrey=np.zeros(nc), capemitgrey=np.zeros(nc),
                    capross=np.zeros(nc), npop=np.zeros((nc, max(self.nlev, 1))))
         self.builds += 1
@@ -241,7 +241,7 @@ class Context:
         """nlte_rad_est after the transport: the updated radtemp (nc) and the group-centre
         intensity jrad (nc, ng), or None without want_jrad."""
         rt = np.array(radtemp, np.float64)
-        jrad = np.zeros((self.nx, self.ng)) if want_jrad else None
+        jrad = np.empty((self.nx, self.ng)) if want_jrad else None
         self._check(self.L.slgpu_nlte_rad_est(self.h, _p(rt), _p(jrad)))
         return rt, jrad
 
@@ -266,7 +266,7 @@ class Context:
     def transport(self, iteration, want=True, check=True):
         nc, ng = self.nx, self.ng
         tally = np.zeros(nc) if want else None
-        jrad = np.zeros((nc, ng)) if want else None
+        jrad = np.empty((nc, ng)) if want else None
         eamp = np.zeros(nc) if want else None
         tot = np.zeros(7)
         ct = np.zeros(10, np.int64)
