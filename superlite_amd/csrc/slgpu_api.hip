@@ -256,6 +256,7 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.gprob, cg);
     rc |= dalloc(c, &d.gshort, cg);
     rc |= dalloc(c, &d.cshort, nc);
+    rc |= dalloc(c, &d.geo, nc);
     rc |= dalloc(c, &d.gorder, cg);
     rc |= dalloc(c, &d.cumL, cg);
     rc |= dalloc(c, &d.cumR, cg);

@@ -144,6 +144,8 @@ struct Philox {
         w2 = w3 = 0;
     }
 
+    // U: rounds per loop trip
+    template <int U = 2>
     __device__ __forceinline__ static void block(uint32_t c0, uint32_t c1, uint32_t c2,
                                                  uint32_t c3, uint32_t k0, uint32_t k1,
                                                  uint32_t out[4])
@@ -153,7 +155,7 @@ struct Philox {
         // as one 64-bit product (one v_mad_u64_u32 instead of v_mul_lo_u32 + v_mul_hi_u32;
         // same bits), and each three-input XOR is one v_bitop3_b32 (truth table 0x96 =
         // a ^ b ^ c): four VALU instructions per round.
-        #pragma unroll 2
+        #pragma unroll U
         for (int r = 0; r < 10; ++r) {
             const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
             const uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x96);

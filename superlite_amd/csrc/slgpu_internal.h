@@ -31,6 +31,14 @@ struct Line64 {
 };
 constexpr int EXP_K1 = 32, EXP_K2 = 32, EXP_ROWS = EXP_K1 + EXP_K2;
 
+// What an IMC event reads of its cell: faces, their velocities, sigma_T, dv/dr, 3c/divv,
+// capgrey (capemitgrey in NLTE), the longest chord, v - dv/dr r at the inner face and the
+// number of lumped groups.
+struct CellGeo {
+    double xl, xr, vl, vr, sg, dvdr, c3, em, far, vhelp;
+    int nlump, pad[3];
+};
+
 // Per-cell DDMC constants (diffusion11.f90:95-152), evaluated once per iteration.
 struct CellDDMC {
     double emgreyinv;   // 1/capgrey (LTE) or 1/capemitgrey (NLTE), nan -> 0
@@ -48,9 +56,9 @@ struct DdmcProb {
 
 // The same for the transport's short step: the event thresholds as 32-bit words compared with
 // a generator word (k_ddmc_probs), half the bytes of the FP64 record per random gather.
-struct ShortProb {              // an unlumped (cell, group): scatter above w3
+struct ShortProb {              // an unlumped (cell, group): scatter above w3, Doppler shift below w1
     double denom;
-    uint32_t w3, pad;
+    uint32_t w3, w1;            // w1: its upper 30 bits; below, BT_LUMP and BT_THIN of the shift's group
 };
 struct ShortCell {              // a cell's lumped step, and its divv
     double denom, divv;
@@ -116,6 +124,7 @@ struct Dev {
     DdmcProb *cprob;            // nc     lumped-group step of each cell
     DdmcProb *gprob;            // nc*ng  unlumped step of each (cell, group), group-fastest
     ShortProb *gshort;          // nc*ng  the short step's form of gprob
+    CellGeo *geo;
     ShortCell *cshort;          // nc     and of cprob
     int *gorder;                // nc*ng  lumped groups ascending, then unlumped ascending
     double *cumL, *cumR, *cumD, *cumS;   // nc*ng cumulative lumped sampling weights

@@ -108,24 +108,40 @@ __device__ __forceinline__ int emitgroup_direct(const Dev &d, double r, int ic)
                             d.emitcum + (size_t)(ic - 1) * d.ng);
 }
 
-// emitgroup restricted to results in [glo, ghi]: the bin index (binsrch with widerange,
-// clamped to 0..nep-1, counts the bins whose cumulative value is <= r1) and the in-bin
-// position are both monotone in r1, so each search resumes at the bucket's lower answer
-__device__ __forceinline__ int emitgroup_range(const Dev &d, double r, int ic, int glo, int ghi)
+// first_above on a short range, four values in flight: a bucket's candidates span 2 to 16 groups, and
+// each value waited for by itself costs an L2 round trip
+__device__ __forceinline__ int first_above4(const double *__restrict__ cum, int lo, int hi, double r)
+{
+    for (; lo < hi; lo += 4) {
+        const int last = hi - 1;
+        const double v0 = cum[lo], v1 = cum[lo + 1 < last ? lo + 1 : last];
+        const double v2 = cum[lo + 2 < last ? lo + 2 : last], v3 = cum[lo + 3 < last ? lo + 3 : last];
+        const int k = v0 > r ? 0 : (v1 > r ? 1 : (v2 > r ? 2 : (v3 > r ? 3 : 4)));
+        if (k < 4) return lo + k;
+    }
+    return hi;
+}
+
+// emitgroup restricted to results in [glo, ghi] (em: capgrey, capemitgrey in NLTE), and the group's
+// opacity: the bin index (binsrch with widerange, clamped to 0..nep-1, counts the bins whose
+// cumulative value is <= r1) and the in-bin position are both monotone in r1, so each search
+// resumes at the bucket's lower answer
+__device__ __forceinline__ int emitgroup_range(const Dev &d, double r, double em, int ic, int glo, int ghi, double &cp)
 {
     const int ng = d.ng, nepg = d.nepg;
     const double *ep = d.emitprob + (size_t)(ic - 1) * d.nep;
-    const double r1 = r * d.capemgrey[ic - 1];
+    const float *row = d.cap32 + (size_t)(ic - 1) * ng;
+    const float first = row[glo - 1];                          // the opacities' line travels with the sums
+    const double r1 = r * em;
     int iep = (glo - 1) / nepg;
     const int iep_hi = (ghi - 1) / nepg;
     while (iep < iep_hi && ep[iep] <= r1) ++iep;
     const int ig = iep * nepg + 1;
     const int igp1 = ig + nepg - 1 < ng ? ig + nepg - 1 : ng;
-    const double *cum = d.emitcum + (size_t)(ic - 1) * ng;
-    int j = (ig > glo ? ig : glo) - 1;
-    const int hi = igp1 - 1;
-    while (j < hi && !(cum[j] > r1)) ++j;
-    return j + 1;
+    const int g = first_above4(d.emitcum + (size_t)(ic - 1) * ng, (ig > glo ? ig : glo) - 1,
+                               igp1 - 1, r1) + 1;
+    cp = (double)(g == glo ? first : row[g - 1]);
+    return g;
 }
 
 // one lumped sampling row: cum[0..cnt) with answer positions lo + j (reversed for the
@@ -166,11 +182,14 @@ __device__ __forceinline__ int sample_entry(const Dev &d, int t, int ic, int nlu
     }
     fl = -1;
     const int lo = (int)(e & 0x7fffu), hi = (int)((e >> 15) & 0x7fffu);
-    if (t == TAB_E) return emitgroup_range(d, r, ic, lo, hi);
+    if (t == TAB_E) {
+        double cp;
+        return emitgroup_range(d, r, d.capemgrey[ic - 1], ic, lo, hi, cp);
+    }
     const LumpRow L = lump_row(d, t, ic, nlump);
-    int j = lo;
-    while (j < hi && !(L.cum[j] > r)) ++j;
-    return lump_group(d, L, ic, j);
+    const int g_lo = lump_group(d, L, ic, lo);                 // travels with the sums
+    const int j = first_above4(L.cum, lo, hi, r);
+    return j == lo ? g_lo : lump_group(d, L, ic, j);
 }
 
 // the same with the entry loaded here; `thin` is -1 (impure bucket: not evaluated) or 0/1

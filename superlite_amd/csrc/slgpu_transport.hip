@@ -150,7 +150,18 @@ template <bool M> __device__ __forceinline__ double p_adiabatic(double divv, dou
                             : 1.0f - expf(-a);
         return 1.0 - (double)d;
     } else {
-        return exp(-divv * t / 3);
+        // most steps lose less than 2^-5, where the series' remainder a^8/8! is under 2^-55: eight
+        // operations instead of exp()'s forty
+        const double a = divv * t * (1.0 / 3.0);
+        if (!(fabs(a) <= 0x1p-5)) return exp(-divv * t / 3);
+        double f = -1.0 / 5040.0;
+        f = fma(f, a, 1.0 / 720.0);
+        f = fma(f, a, -1.0 / 120.0);
+        f = fma(f, a, 1.0 / 24.0);
+        f = fma(f, a, -1.0 / 6.0);
+        f = fma(f, a, 0.5);
+        f = fma(f, a, -1.0);
+        return fma(f, a, 1.0);
     }
 }
 // r^3-uniform radius in [xl, xr]: (r*xr^3 + (1-r)*xl^3)**(1.0/3.0) with the reference's
@@ -191,11 +202,13 @@ __device__ __forceinline__ double thomson_aniso_mu(double r1)
     return 1.0 - 2.0 * r1;
 }
 
-// What an IMC pass reads of its cell and group, requested together at the top of the pass:
+// What an IMC pass reads of its cell and group, requested together at the top of the pass, the
+// cell's part as one record (nine arrays took as many address computations and requests):
 // the conversion that most passes begin with and the event then wait for one round trip
 // instead of one at each branch.
 struct ImcIn {
-    double xl, xr, vl, vr, sg, dvdr, c3, wi0, wi1;     // faces, their velocities, sigma_T, WLI(ig), WLI(ig+1)
+    CellGeo g;
+    double wi0, wi1;                                   // WLI(ig), WLI(ig+1)
     float cp, cpup, cpdn;                              // gas_cap of the group and of its two neighbours
 };
 
@@ -207,14 +220,22 @@ __device__ __forceinline__ void imc_request(const Dev &d, const Ptcl &p, ImcIn &
     q.cpup = row[ig < ng ? ig : ig - 1];
     q.cpdn = row[ig > 1 ? ig - 2 : ig - 1];
     q.wi0 = WLI(ig); q.wi1 = WLI(ig + 1);
-    q.xl = XA(ix); q.xr = XA(ix + 1);
-    q.vl = VXA(ix); q.vr = VXA(ix + 1);
-    q.sg = SIGT(ix);
-    q.dvdr = d.dvdr[ix - 1];
-    q.c3 = d.c3divv[ix - 1];
+    q.g = d.geo[ix - 1];
 }
 
-template <bool M>
+// the smallest double whose quotient by c is at least 0.1
+constexpr double NEWTON_DV = 0x1.656165a400000p+31;
+static_assert(NEWTON_DV / PC_C >= 0.1 && 0x1.656165a3fffffp+31 / PC_C < 0.1, "NEWTON_DV");
+
+// BT_THIN and BT_LUMP of a group of opacity cp in the cell (group_flags of slgpu_sample.h)
+__device__ __forceinline__ uint32_t cell_flags(const Dev &d, const CellGeo &q, double cp)
+{
+    const double dx = q.xr - q.xl;
+    if (d.puretran || (q.sg + cp) * dx < d.tauddmc) return BT_THIN;
+    return cp * dx >= d.taulump && q.nlump > 0 ? BT_LUMP : 0u;
+}
+
+template <bool M, bool X>
 __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, double &erd, double &jrd,
                            double &eamp, double &evelo)
 {
@@ -227,8 +248,8 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
     erd = 0.0; jrd = 0.0; eamp = 0.0;
     double elabfact = 1.0 - mu * vx * CINV;
     const double elabfactold = elabfact;
-    const double xl = q.xl, xr = q.xr;
-    const double far = 2.0 * fabs(sqrt(xr * xr - xl * xl));
+    const double xl = q.g.xl, xr = q.g.xr;
+    const double far = q.g.far;
     if (ix == 1 || mu >= -sqrt(1.0 - (xl / x) * (xl / x))) {
         db = fabs(sqrt(xr * xr - (1.0 - mu * mu) * x * x) - mu * x);
         ixnext = ix + 1;
@@ -238,16 +259,17 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
     }
     // the neighbour cell, for an event at the face
     const int nb = ixnext < 1 ? 1 : (ixnext > nx ? nx : ixnext);
-    const double cap_nb = CAPT(ig, nb), sig_nb = SIGT(nb), dx_nb = DXX(nb);
+    const CellGeo &gn = d.geo[nb - 1];
+    const double cap_nb = CAPT(ig, nb), sig_nb = gn.sg, dx_nb = gn.xr - gn.xl;
     if (db != db) return 1;
-    const double sg = q.sg, cp = (double)q.cp;
+    const double sg = q.g.sg, cp = (double)q.cp;
+    const double dvdr = q.g.dvdr;
     if (sg > 0.0) { r1 = s.draw(); dthm = p_path<M>(r1, elabfact * sg); }
     else dthm = far;
     if (cp <= 0.0) dcol = far;
     else { r1 = s.draw(); dcol = p_path<M>(r1, elabfact * cp); }
-    const double dvdr = q.dvdr;
-    const double vhelp = q.vl - dvdr * xl;
-    if (fabs(vx - vhelp) / PC_C >= 0.1) {
+    const double vhelp = q.g.vhelp;
+    if (fabs(vx - vhelp) >= NEWTON_DV) {                      // / c >= 0.1
         // Newton-Raphson Doppler distance (transport11.f90:159-199)
         const double epstol = 1e-3;
         int it = 0;
@@ -272,8 +294,8 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
         }
         if (ddop <= 0.0 || it == 100) ddop = far;
     } else {
-        if (dvdr > 0 && ig < ng) ddop = q.c3 * (elabfact - wl * q.wi1);
-        else if (dvdr < 0 && ig > 1) ddop = q.c3 * (elabfact - wl * q.wi0);
+        if (dvdr > 0 && ig < ng) ddop = q.g.c3 * (elabfact - wl * q.wi1);
+        else if (dvdr < 0 && ig > 1) ddop = q.g.c3 * (elabfact - wl * q.wi0);
         else ddop = far;
         if (ddop < 0.0) ddop = far;
     }
@@ -288,7 +310,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
     if (dd < 0.0) return 4;
     const double xold = x;
     x = sqrt(x * x + dd * dd + 2.0 * dd * x * mu);
-    vx = (q.vl * (xr - x) + q.vr * (x - xl)) / (xr - xl);
+    vx = (q.g.vl * (xr - x) + q.g.vr * (x - xl)) / (xr - xl);
     if (x == 0.0) mu = 1.0;
     else mu = (xold * mu + dd) / x;
     erd = e * elabfact * elabfact * dd * CINV;
@@ -305,7 +327,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
     }
     if (dd == dthm || dd == dcol) {
         r1 = s.draw();
-        if (dd == dthm && d.thm_aniso) mu = thomson_aniso_mu(r1);
+        if (X && dd == dthm && d.thm_aniso) mu = thomson_aniso_mu(r1);
         else mu = 1.0 - 2.0 * r1;
         mu = (mu + vx * CINV) / (1.0 + vx * mu * CINV);
     } else if (dd == db) {
@@ -323,12 +345,18 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
         e = e * help;
         if (ng != 1) {
             r1 = s.draw();
-            int fl;
-            ig = sample_entry(d, TAB_E, ic, 0, r1, bt_row(d, TAB_E, ic)[bt_key(r1)], fl);
-            if (fl < 0) fl = (int)group_flags(d, ig, ic);
-            if (!(fl & (int)BT_THIN)) {
+            const uint32_t ent = bt_row(d, TAB_E, ic)[bt_key(r1)];
+            uint32_t fl = ent & (BT_THIN | BT_LUMP);
+            if (ent & BT_PURE) {
+                ig = (int)(ent & 0x7fffu);
+            } else {
+                double cg;
+                ig = emitgroup_range(d, r1, q.g.em, ic, (int)(ent & 0x7fffu), (int)((ent >> 15) & 0x7fffu), cg);
+                fl = cell_flags(d, q.g, cg);
+            }
+            if (!(fl & BT_THIN)) {
                 p.itype = 2;
-                p.nflag = NF_VALID | ((uint32_t)fl & BT_LUMP);
+                p.nflag = NF_VALID | (fl & BT_LUMP);
             }
         }
         if (p.itype == 2) {
@@ -348,7 +376,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
         const int l = ix + 1;
         if ((sig_nb + cap_nb) * dx_nb < d.tauddmc || d.puretran) {
             x = xr;
-            vx = q.vr;
+            vx = q.g.vr;
             ix = ix + 1;
         } else {
             mu = (mu - vx * CINV) / (1.0 - vx * mu * CINV);
@@ -368,18 +396,18 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
                 mu = -(r1 > r2 ? r1 : r2);
                 mu = (mu + vx * CINV) / (1.0 + vx * mu * CINV);
                 x = xr;
-                vx = q.vr;
+                vx = q.g.vr;
             }
         }
     } else if (dd == db) {
         const int l = ix - 1;
         if ((sig_nb + cap_nb) * dx_nb < d.tauddmc || d.puretran) {
             x = xl;
-            vx = q.vl;
+            vx = q.g.vl;
             ix = ix - 1;
         } else {
             mu = (mu - vx * CINV) / (1.0 - vx * mu * CINV);
-            if (d.ampfact && mu < 0.0) {
+            if (X && d.ampfact && mu < 0.0) {
                 // amplification factor (transport11.f90:410-421)
                 double h = 1.0 / fabs(mu);
                 h = h < 100.0 ? h : 100.0;
@@ -404,7 +432,7 @@ __device__ int transport11(const Dev &d, Ptcl &p, StepRng &s, const ImcIn &q, do
                 mu = r1 > r2 ? r1 : r2;
                 mu = (mu + vx * CINV) / (1.0 + vx * mu * CINV);
                 x = xl;
-                vx = q.vl;
+                vx = q.g.vl;
             }
         }
     } else if (dd == ddop) {
@@ -538,7 +566,10 @@ __global__ __launch_bounds__(256) void k_ddmc_probs(Dev d)
     ShortProb sp;
     sp.denom = q.t3 == q.t3 ? q.denom : q.t3;
     sp.w3 = word_threshold(q.t3);
-    sp.pad = 0;
+    // the Doppler shift of an unlumped particle: the threshold's upper 30 bits and the flags of the
+    // group it leads to
+    const int to = DIVV(ix) >= 0 ? (ig + 1 > ng ? ng : ig + 1) : (ig < 2 ? 1 : ig - 1);
+    sp.w1 = (word_threshold(q.t1) & ~3u) | (group_flags(d, to, ic) >> 29 & 3u);
     d.gshort[(size_t)(ic - 1) * ng + ig - 1] = sp;
     if (ig == 1) {
         const DdmcProb c = ddmc_prob(OPL(1, ic), OPL(2, ic), cc.emitlump, cc.caplump, cc.doplump);
@@ -732,14 +763,14 @@ __device__ void imc_entry(const Dev &d, Ptcl &p, const StepRng &s, const ImcIn &
     }
     const double ra = next(), rb = next();
     if (face) {
-        x = kind == PEND_LEFT ? q.xr : q.xl;                  // the face crossed into cell ix
-        vx = kind == PEND_LEFT ? q.vr : q.vl;
+        x = kind == PEND_LEFT ? q.g.xr : q.g.xl;                  // the face crossed into cell ix
+        vx = kind == PEND_LEFT ? q.g.vr : q.g.vl;
         mu = ra > rb ? ra : rb;
         if (kind == PEND_LEFT) mu = -mu;
     } else {
         mu = 1.0 - 2.0 * ra;
-        x = shell_position<M>(q.xl, q.xr, rb);
-        vx = (q.vl * (q.xr - x) + q.vr * (x - q.xl)) / (q.xr - q.xl);
+        x = shell_position<M>(q.g.xl, q.g.xr, rb);
+        vx = (q.g.vl * (q.g.xr - x) + q.g.vr * (x - q.g.xl)) / (q.g.xr - q.g.xl);
     }
     mu = (mu + vx * CINV) / (1.0 + vx * mu * CINV);
     const double help = 1.0 / (1.0 - vx * mu * CINV);
@@ -824,9 +855,18 @@ __device__ __forceinline__ void cold_store(const Ptcl &p, Cold &s)
 // together.  The logarithm and the next step's Philox block are computed while they travel.
 // Any other step is left untouched for diffusion11 (NF_FULL).  The draws, the arithmetic and
 // the order of the sums are diffusion11's.  least: the lanes below which the wave leaves.
-// What bounds it is that round trip (1.1 us for a lane alone, in 160 KB of thresholds and 64 KB
-// of entries per cell and table).  Against a full diffusion11 pass per DDMC step, c2 (400 x 10^4) at 2^20
-// particles went from 3.69 to 2.87 s in the precision form and from 4.69 to 3.75 s in FP64.
+// An unlumped particle's Doppler shift samples no group: its threshold and the flags of the group it
+// leads to come with the record of its group.
+// What bounds it is instruction issue: four waves of a SIMD share it, and a lane alone is held up by
+// dependent instructions and branches more than by the round trip.  So the tables' addresses stay in
+// scalar registers, conditions are combined instead of branched on, and the generator's ten rounds
+// are unrolled (in a loop of five trips they cost 15% of the transport).  Requesting the entry of the
+// step after next as well, which is known to follow a pure effective scatter, halves the round
+// trips but adds a generator block and an entry per step: 5% slower.
+// Against a full diffusion11 pass per DDMC step, c2 (400 x 10^4) at 2^20 particles went from 3.69 to
+// 2.87 s in the precision form and from 4.69 to 3.75 s in FP64; the leaner loop together with
+// CellGeo and the unlumped Doppler shift took c2 at 2^17 particles from 1.03-1.09 to 0.90-0.98 s,
+// FP64 (154 x 6000, 10^5 particles) from 0.35-0.38 to 0.31-0.34 s.
 template <bool M>
 __device__ __forceinline__ void short_run(const Dev &d, Ptcl &p, uint32_t pid, uint32_t k0, uint32_t k1,
                                           int64_t &istep, double &evelo, int &run_ic, double &run_e,
@@ -834,37 +874,54 @@ __device__ __forceinline__ void short_run(const Dev &d, Ptcl &p, uint32_t pid, u
                                           int least)
 {
     const uint32_t ng = d.ng, nx = d.nx;
+    // in registers for the whole run, not fetched again from the kernel's arguments
+#define GLOBAL_CONST __attribute__((address_space(1))) const
+    GLOBAL_CONST uint32_t *btab = (GLOBAL_CONST uint32_t *)d.btab;
+    GLOBAL_CONST ShortProb *gshort = (GLOBAL_CONST ShortProb *)d.gshort;
+    GLOBAL_CONST ShortCell *cshort = (GLOBAL_CONST ShortCell *)d.cshort;
+    asm volatile("" : "+s"(btab), "+s"(gshort), "+s"(cshort));
+    auto cell = [&](uint32_t ic) {
+        GLOBAL_CONST ShortCell *q = cshort + ic;
+        return ShortCell{q->denom, q->divv, q->w1, q->w2, q->w3, 0u};
+    };
     uint32_t o[4];
     Philox::block(pid, (uint32_t)(istep + 1), StepRng::PHASE, 0u, k0, k1, o);
-    ShortCell c = d.cshort[p.ix - 1], cn = c;                  // of the particle's cell, of the next
+    ShortCell c = cell(p.ix - 1), cn = c;                    // of the particle's cell, of the next
     uint32_t wlg = 0;                                          // group edge a Doppler shift left wl at
-    bool go = true;
-    uint32_t t, ent, w3;
+    bool go = true, open;
+    uint32_t t, ent, w3, w1;
     double denom;
     auto request = [&]() {
         const uint32_t ic = p.ix, w = o[1];
         const bool lump = (p.nflag & BT_LUMP) != 0;
-        t = !lump ? TAB_E : (w > c.w3 ? TAB_S : (w < c.w1 ? TAB_D : (w < c.w2 ? TAB_L : TAB_R)));
-        ent = d.btab[((t * nx + (ic - 1)) << BT_BITS) + (o[2] >> (32 - BT_BITS))];
+        const uint32_t tl = w > c.w3 ? TAB_S : (w < c.w1 ? TAB_D : (w < c.w2 ? TAB_L : TAB_R));
+        t = lump ? tl : (uint32_t)TAB_E;
+        ent = btab[((t * nx + (ic - 1)) << BT_BITS) + (o[2] >> (32 - BT_BITS))];
+        // undecided, or a face of the mesh: not a short step
+        open = lump & ((w == c.w1) | (w == c.w2) | (w == c.w3) | ((t == TAB_L) & (ic == 1)) |
+                                  ((t == TAB_R) & (ic == nx)));
         denom = c.denom;
-        w3 = c.w3;
+        w3 = w1 = 0u;
         if (!lump) {
-            const ShortProb q = d.gshort[(ic - 1) * ng + (p.ig - 1)];
-            denom = q.denom;
-            w3 = q.w3;
-        } else if (w == c.w1 || w == c.w2 || w == c.w3 || (t == TAB_L && ic == 1) || (t == TAB_R && ic == nx)) {
-            denom = __builtin_nan("");                         // undecided, or a face of the mesh
-        } else if (t == TAB_L || t == TAB_R) {
-            cn = d.cshort[t == TAB_L ? ic - 2 : ic];
+            GLOBAL_CONST ShortProb *q = gshort + ((ic - 1) * ng + (p.ig - 1));
+            denom = q->denom;
+            w3 = q->w3;
+            w1 = q->w1;
         }
+        if ((t <= TAB_R) & !open) cn = cell(t == TAB_L ? ic - 2 : ic);
     };
     request();
     do {
         const double lrt = p_log<M>(Philox::u42(o[0], o[3] & 0x3FFu));
-        const uint32_t w = o[1];
-        Philox::block(pid, (uint32_t)(istep + 2), StepRng::PHASE, 0u, k0, k1, o);
+        const uint32_t w = o[1], r2_hi = o[2], r2_lo = o[3] >> 20;
+        Philox::block<10>(pid, (uint32_t)(istep + 2), StepRng::PHASE, 0u, k0, k1, o);
+        asm volatile("" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));     // before the wait
         __builtin_amdgcn_sched_barrier(0);
-        if ((ent & BT_PURE) && denom == denom && (t != TAB_E || w > w3)) {
+        // an unlumped particle's Doppler shift samples no group
+        const bool shift = (w & ~3u) < (w1 & ~3u);
+        ent = shift ? BT_PURE | (w1 & 3u) << 29 | (uint32_t)p.ig : ent;
+        t = shift ? (uint32_t)TAB_D : t;
+        if (((ent & BT_PURE) != 0u) & !open & (denom == denom) & ((t != TAB_E) | (w > w3))) {
             const uint32_t ic = p.ix;
             const double ddmct = fabs(lrt * denom * CINV);
             const double erd = p.e * ddmct, jrd = PC_C * erd;
@@ -889,6 +946,10 @@ __device__ __forceinline__ void short_run(const Dev &d, Ptcl &p, uint32_t pid, u
                 p.itype = 1;
                 p.nflag = (kind << 1) | (ent & BT_LUMP);
                 cold.pend_f[threadIdx.x] = f;
+                if (shift) {                                   // whose third draw is still unused
+                    p.nflag |= NF_R2FREE;
+                    cold.pend_r2[threadIdx.x] = Philox::u42(r2_hi, r2_lo & 0x3FFu);
+                }
                 atomicAdd(&bt.ct[4], 1ull);
                 go = false;
             } else {
@@ -917,7 +978,9 @@ __device__ __forceinline__ void short_run(const Dev &d, Ptcl &p, uint32_t pid, u
 // particles.  A pool smaller than the lanes resident on the chip is spread over all waves: its
 // time is the longest walk's, and a step costs a lane 1.9 us with one neighbour in its wave
 // against 3 us with 31 (8192 particles on c2: 1.34 s in full waves, 0.59 s spread).
-template <bool M>
+// X: the amplification factor or anisotropic Thomson scattering is on; without them the kernel
+// holds 5 KB less code and needs no scratch memory (36 bytes per lane otherwise).
+template <bool M, bool X>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(M ? SLGPU_WAVES_MIXED : SLGPU_WAVES_FP64, 8)))
 void k_transport(Dev d, uint32_t iteration, int lanes)
@@ -1007,7 +1070,7 @@ void k_transport(Dev d, uint32_t iteration, int lanes)
         if (imc) {
             double ea;
             atomicAdd(&bt.ct[1], 1ull);
-            ierr = transport11<M>(d, p, s, q, erd, jrd, ea, evelo);
+            ierr = transport11<M, X>(d, p, s, q, erd, jrd, ea, evelo);
             if (ea != 0.0) {                                   // particle_advance.f90:216-217
                 atomicAdd(&d.eamp[icold - 1], ea);
                 atomicAdd(&bt.tot[6], ea);
@@ -1084,8 +1147,27 @@ void launch_sources(slgpu_ctx *c, uint32_t iteration)
                        c->d, iteration);
 }
 
+// the transport's per-cell record, from what was set last
+__global__ __launch_bounds__(256) void k_cell_geo(Dev d)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= d.nx) return;
+    CellGeo g;
+    g.xl = d.xarr[i]; g.xr = d.xarr[i + 1];
+    g.vl = d.vxarr[i]; g.vr = d.vxarr[i + 1];
+    g.sg = d.sig[i]; g.dvdr = d.dvdr[i]; g.c3 = d.c3divv[i];
+    g.em = d.capemgrey[i];
+    g.far = 2.0 * fabs(sqrt(g.xr * g.xr - g.xl * g.xl));
+    g.vhelp = g.vl - g.dvdr * g.xl;
+    g.nlump = d.cell[i].nlump;
+    g.pad[0] = g.pad[1] = g.pad[2] = 0;
+    d.geo[i] = g;
+    d.cshort[i].divv = d.divv[i];
+}
+
 void launch_transport(slgpu_ctx *c, uint32_t iteration)
 {
+    hipLaunchKernelGGL(k_cell_geo, dim3((c->nx + 255) / 256), dim3(256), 0, c->stream, c->d);
     int dev = 0, ncu = 256;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -1093,12 +1175,11 @@ void launch_transport(slgpu_ctx *c, uint32_t iteration)
     const int64_t resident = (int64_t)ncu * 4 * (c->d.precision == SLGPU_MIXED ? SLGPU_WAVES_MIXED : SLGPU_WAVES_FP64);
     const int64_t share = (c->d.npart + resident - 1) / resident;
     const int lanes = share < 1 ? 1 : (share > 64 ? 64 : (int)share);
-    if (c->d.precision == SLGPU_MIXED)
-        hipLaunchKernelGGL(k_transport<true>, dim3((unsigned)blocks), dim3(256),
-                           c->nx * sizeof(double), c->stream, c->d, iteration, lanes);
-    else
-        hipLaunchKernelGGL(k_transport<false>, dim3((unsigned)blocks), dim3(256),
-                           c->nx * sizeof(double), c->stream, c->d, iteration, lanes);
+    const bool extra = c->d.ampfact || c->d.thm_aniso;
+    auto kernel = c->d.precision == SLGPU_MIXED ? (extra ? k_transport<true, true> : k_transport<true, false>)
+                                                : (extra ? k_transport<false, true> : k_transport<false, false>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), c->nx * sizeof(double), c->stream, c->d,
+                       iteration, lanes);
 }
 
 // the transport's group samplers at arbitrary (r, cell), table path or direct search
