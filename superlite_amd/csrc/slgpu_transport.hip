@@ -1139,6 +1139,40 @@ __global__ __launch_bounds__(256) void k_fluxtally(Dev d)
     atomicAdd(&d.num[ig - 1], 1);
 }
 
+// The same for group grids whose edges and bins fit a block's LDS: particles outnumber the bins a
+// thousandfold at 2^20 x 1000, and their atomics on a bin follow each other.  A block bins its share
+// in LDS, searching the edges there, and adds its nonzero bins to the tally.
+// 2^20 particles on 1000 groups: 0.50 ms with every particle's atomics on the tally, 0.09 ms so;
+// 16384 on 250: 24 us, under 10 us so.
+constexpr int FLUX_THREADS = 1024, FLUX_GROUPS = 2300;     // 28 bytes a group, 64 KB of LDS
+__global__ __launch_bounds__(FLUX_THREADS) void k_fluxtally_lds(Dev d)
+{
+    extern __shared__ double s_edge[];
+    const int ng = d.ng;
+    double *lum = s_edge + ng + 1, *dev = lum + ng;
+    int *num = (int *)(dev + ng);
+    for (int g = threadIdx.x; g <= ng; g += FLUX_THREADS) s_edge[g] = d.wl[g];
+    for (int g = threadIdx.x; g < ng; g += FLUX_THREADS) { lum[g] = 0.0; dev[g] = 0.0; num[g] = 0; }
+    __syncthreads();
+    for (int64_t p = (int64_t)blockIdx.x * FLUX_THREADS + threadIdx.x; p < d.npart; p += (int64_t)gridDim.x * FLUX_THREADS) {
+        const int stat = d.pstat[p];
+        const double wl = d.pwl[p], e = d.pe[p];
+        if (stat != 1) continue;
+        const int ig = binsrch(wl, s_edge, ng + 1, false);
+        if (ig < 1) continue;            // NaN wavelength: not binned
+        atomicAdd(&lum[ig - 1], e);
+        atomicAdd(&dev[ig - 1], e * e);
+        atomicAdd(&num[ig - 1], 1);
+    }
+    __syncthreads();
+    for (int g = threadIdx.x; g < ng; g += FLUX_THREADS) {
+        if (num[g] == 0) continue;
+        atomicAdd(&d.lum[g], lum[g]);
+        atomicAdd(&d.dev[g], dev[g]);
+        atomicAdd(&d.num[g], num[g]);
+    }
+}
+
 void launch_sources(slgpu_ctx *c, uint32_t iteration)
 {
     int64_t n = c->d.npart;
@@ -1235,6 +1269,15 @@ void launch_fluxtally(slgpu_ctx *c)
 {
     int64_t n = c->d.npart;
     if (n == 0) return;
+    if (c->ng <= FLUX_GROUPS) {
+        // a block's rounds over its particles take about 1.3 us each, and the bins it flushes 3 ng
+        // atomics of 0.16 ns: the sum is least at this count
+        const double least = sqrt(2.7 * (double)n / c->ng);
+        const int64_t most = std::min<int64_t>(256, (n + FLUX_THREADS - 1) / FLUX_THREADS);
+        const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(most, (int64_t)ceil(least)));
+        hipLaunchKernelGGL(k_fluxtally_lds, dim3(blocks), dim3(FLUX_THREADS), (size_t)28 * c->ng + 8, c->stream, c->d);
+        return;
+    }
     hipLaunchKernelGGL(k_fluxtally, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream,
                        c->d);
 }
