@@ -295,14 +295,28 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
 // chain of additions, 6 clocks each, and the work is to keep everything else off the chain:
 //   - an LDS access takes the pipe as long for 1 lane as for 64, so a block takes RS_ROWS rows,
 //     one per lane of its first wave (one row per block: 37 ns per value with the chip full);
-//   - the other eight waves store the tile before and fetch the tile after meanwhile;
+//   - the other eight waves store the tile before, write the tile after to LDS and request the one
+//     after that meanwhile, under barriers that wait for LDS alone (with __syncthreads() a tile
+//     took a load's and a store's round trip to memory: 12 ns a value instead of 8);
 //   - the chain's LDS reads run 16 values ahead, in two register sets that take turns.
 // The source rows, which have two chains, start first.  400 x 10^4: 0.85 ms for the same chains on
-// global memory, 0.23 ms so (12 ns per value of the longest chain, the two source passes).
+// global memory, 0.16 ms so (8 ns per value of the longest chain, the two source passes).
 constexpr int RS_ROWS = 8, RS_TILE = 256, RS_PITCH = RS_TILE + 2, RS_AHEAD = 16;
 constexpr int RS_THREADS = 576, RS_MOVERS = RS_THREADS - 64;
+typedef __attribute__((address_space(1))) double *RowPtr;     // not a flat access, which counts as one to LDS too
 
-// s and the running sums of the RS_TILE values of buf from s on, in index order
+// A barrier for what the block keeps in LDS.  __syncthreads() also waits for every load and store
+// under way to global memory, which the movers' tiles are meant to overlap.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// s and the running sums of the RS_TILE values of buf from s on, in index order; OUT: the running
+// sums replace the values
+template <bool OUT>
 __device__ __forceinline__ double chain_sum(double *buf, double s)
 {
     double v[RS_AHEAD], w[RS_AHEAD];
@@ -316,7 +330,7 @@ __device__ __forceinline__ double chain_sum(double *buf, double s)
         #pragma unroll
         for (int k = 0; k < RS_AHEAD; ++k) { s = s + v[k]; v[k] = s; }
         #pragma unroll
-        for (int k = 0; k < RS_AHEAD; ++k) buf[j + k] = v[k];
+        for (int k = 0; k < RS_AHEAD; ++k) { if (OUT) buf[j + k] = v[k]; }
         __builtin_amdgcn_sched_barrier(0);
         const int q = j + 2 * RS_AHEAD < RS_TILE ? j + 2 * RS_AHEAD : j;
         #pragma unroll
@@ -325,7 +339,7 @@ __device__ __forceinline__ double chain_sum(double *buf, double s)
         #pragma unroll
         for (int k = 0; k < RS_AHEAD; ++k) { s = s + w[k]; w[k] = s; }
         #pragma unroll
-        for (int k = 0; k < RS_AHEAD; ++k) buf[j + RS_AHEAD + k] = w[k];
+        for (int k = 0; k < RS_AHEAD; ++k) { if (OUT) buf[j + RS_AHEAD + k] = w[k]; }
         __builtin_amdgcn_sched_barrier(0);
     }
     return s;
@@ -334,30 +348,47 @@ __device__ __forceinline__ double chain_sum(double *buf, double s)
 // For the block's rows r: sums of p[r][0..n[r]) / div[r] in index order, on lane r of the first
 // wave; OUT: the running sums replace the row.  nmax: the longest row.
 template <bool OUT>
-__device__ __forceinline__ double rows_sum(double *const *p, const int *n, const double *div, int nmax,
+__device__ __forceinline__ double rows_sum(RowPtr const *p, const int *n, const double *div, int nmax,
                                            double (*buf)[RS_ROWS][RS_PITCH])
 {
     constexpr int PER = RS_ROWS * RS_TILE / RS_MOVERS;
     const int t = threadIdx.x, lt = t - 64, ntile = (nmax + RS_TILE - 1) / RS_TILE;
-    double s = 0.0;
+    double s = 0.0, v[PER];
+    RowPtr row[PER];
+    int len[PER];
+    double dv[PER];
+    if (t >= 64) {
+        #pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int e = lt + q * RS_MOVERS, r = e / RS_TILE, k = e % RS_TILE;
+            row[q] = p[r] + k;
+            len[q] = n[r] - k;
+            dv[q] = div[r];
+            v[q] = len[q] > 0 ? row[q][0] : 0.0;
+        }
+    }
     for (int c = -1; c <= ntile; ++c) {
         if (t >= 64) {
-            double v[PER];
+            // tile c + 1, requested an iteration ago; then tile c + 2 is
             #pragma unroll
             for (int q = 0; q < PER; ++q) {
-                const int e = lt + q * RS_MOVERS, r = e / RS_TILE, j = (c + 1) * RS_TILE + e % RS_TILE;
-                v[q] = j < n[r] ? p[r][j] : 0.0;
+                const int e = lt + q * RS_MOVERS, r = e / RS_TILE, k = e % RS_TILE;
+                if (c + 1 < ntile) buf[(c + 1) % 3][r][k] = OUT ? v[q] / dv[q] : v[q];
             }
             #pragma unroll
             for (int q = 0; q < PER; ++q) {
-                const int e = lt + q * RS_MOVERS, r = e / RS_TILE, k = e % RS_TILE, j = (c - 1) * RS_TILE + k;
-                if (OUT && c > 0 && j < n[r]) p[r][j] = buf[(c - 1) % 3][r][k];
-                if (c < ntile) buf[(c + 1) % 3][r][k] = OUT ? v[q] / div[r] : v[q];
+                const int o = (c + 2) * RS_TILE;
+                v[q] = o < len[q] ? row[q][o] : 0.0;
+            }
+            #pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const int e = lt + q * RS_MOVERS, r = e / RS_TILE, k = e % RS_TILE, o = (c - 1) * RS_TILE;
+                if (OUT && c > 0 && o < len[q]) row[q][o] = buf[(c - 1) % 3][r][k];
             }
         } else if (t < RS_ROWS && c >= 0 && c < ntile) {
-            s = chain_sum(buf[c % 3][t], s);
+            s = chain_sum<OUT>(buf[c % 3][t], s);
         }
-        __syncthreads();
+        lds_barrier();
     }
     return s;
 }
@@ -372,7 +403,7 @@ __global__ __launch_bounds__(256) void k_src_terms(Dev d)
 __global__ __launch_bounds__(RS_THREADS) void k_row_sums(Dev d)
 {
     __shared__ __align__(16) double buf[3][RS_ROWS][RS_PITCH];
-    __shared__ double *p[RS_ROWS];
+    __shared__ RowPtr p[RS_ROWS];
     __shared__ double div[RS_ROWS];
     __shared__ int n[RS_ROWS], s_max;
     const int ng = d.ng, row = (int)blockIdx.y - 1, t = threadIdx.x;
@@ -384,7 +415,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_row_sums(Dev d)
         double *base = row < 0 ? d.srccum : (row == 0 ? d.cumL : (row == 1 ? d.cumR : (row == 2 ? d.cumD : d.cumS + nl)));
         int m = row < 0 ? ng : (nl == 0 ? 0 : (row == 3 ? ng - nl : nl));
         if (l >= d.nx) m = 0;
-        p[t] = base + (size_t)lc * ng;
+        p[t] = (RowPtr)base + (size_t)lc * ng;
         n[t] = m;
         div[t] = 1.0;
         atomicMax(&s_max, m);
