@@ -501,18 +501,53 @@ __device__ __forceinline__ int first_above_from(const double *cum, int from, int
     return lo >= n ? n : first_above(cum, lo, lo + step <= n ? lo + step - 1 : n - 1, r);
 }
 
-// Exact bucket maps of the five group samplers: one block per (cell, table), which searches the
-// row in LDS (S; rows past the CU's LDS are searched in global memory), each thread a stretch
-// of 16 buckets.  The answers of a stretch rise, so each search starts from the one before.
-// They change hands in LDS: the entries are then made in bucket order, where neighbouring lanes
-// load the same groups' opacities and store side by side.  400 x 10^4: 200 us, against 640 us
-// with two full searches per bucket on global memory; random LDS reads and the gathers bound it.
+// inclusive running maximum over the block of both 16-bit halves
+__device__ __forceinline__ uint32_t max16(uint32_t a, uint32_t b)
+{
+    const uint32_t lo = max(a & 0xffffu, b & 0xffffu), hi = max(a >> 16, b >> 16);
+    return hi << 16 | lo;
+}
+
+__device__ __forceinline__ uint32_t block_scan_max16(uint32_t v, uint32_t *sh)
+{
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    #pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t u = __shfl_up(v, off, 64);
+        if (lane >= off) v = max16(v, u);
+    }
+    if (lane == 63) sh[w] = v;
+    __syncthreads();
+    for (int k = 0; k < w; ++k) v = max16(v, sh[k]);
+    __syncthreads();
+    return v;
+}
+
+// place of a bucket's answer in LDS: a thread's stretch of 16 starts on a bank of its own
+__device__ __forceinline__ int ans_at(int b) { return b + (b >> 4); }
+constexpr size_t BT_ANSWERS = (BT_K + BT_K / 16) * sizeof(uint32_t);
+
+// Exact bucket maps of the five group samplers, one block per (cell, table).
+// A lumped row's answers need no search.  The draw at the lower end of bucket b is b/K (K = 2^14),
+// that at its upper end the double below (b + 1)/K, and the answer is how many running sums c are
+// not above the draw: those with ceil(c K) <= b and with floor(c K) <= b (in the last bucket, whose
+// upper end is 1, also c = 1).  c K is exact.  So the last sum of every ceil(c K) writes its count
+// there, the last of every floor(c K) likewise, and the answers are running maxima.  A row that does
+// not rise throughout (a NaN, see slgpu_sample.h) keeps two searches per bucket.
+// The emission table's draws are scaled and rounded first, so it is searched: the row in LDS (S;
+// rows past the CU's LDS are searched in global memory), each thread a stretch of 16 buckets,
+// whose answers rise, so each search starts from the one before.
+// The answers change hands in LDS: the entries are then made in bucket order, where neighbouring lanes
+// load the same groups' opacities and store side by side.  400 x 10^4: 640 us with two full
+// searches per bucket on global memory, 199 us with searches in LDS that resume, 139 us so;
+// the gathers bound it.
 template <bool S>
 __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
 {
     extern __shared__ double s_row[];
     constexpr int PER = BT_K / 1024;
-    const int ic = blockIdx.x + 1, t = blockIdx.y, ng = d.ng, nep = d.nep, nepg = d.nepg;
+    // the emission tables, which take longest, start first
+    const int ic = blockIdx.x + 1, t = NTAB - 1 - (int)blockIdx.y, ng = d.ng, nep = d.nep, nepg = d.nepg;
     uint32_t *row = d.btab + ((size_t)t * d.nx + (ic - 1)) * BT_K;
     const bool emit = t == TAB_E;
     const int nlump = d.cell[ic - 1].nlump;
@@ -523,35 +558,56 @@ __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
     }
     const double *cum = emit ? d.emitcum + (size_t)(ic - 1) * ng : L.cum;
     const double *ep = d.emitprob + (size_t)(ic - 1) * nep;
-    const int n = emit ? ng : L.cnt;
-    __shared__ int s_nan;
-    if (threadIdx.x == 0) s_nan = 0;
-    __syncthreads();
-    for (int k = threadIdx.x; k < n; k += 1024) {
-        const double v = cum[k];
-        if constexpr (S) s_row[k] = v;
-        if (v != v) s_nan = 1;
+    const int n = emit ? ng : L.cnt, b0 = threadIdx.x * PER;
+    uint32_t *s_ans = reinterpret_cast<uint32_t *>(s_row);
+    __shared__ int s_bad;
+    __shared__ uint32_t s_max[NW];
+    if (threadIdx.x == 0) s_bad = 0;
+    if (!emit) {
+        #pragma unroll
+        for (int k = 0; k < PER; ++k) s_ans[ans_at(threadIdx.x + k * 1024)] = 0u;
     }
-    if constexpr (S) {
-        if (emit)
+    __syncthreads();
+    if (emit) {
+        for (int k = threadIdx.x; k < n; k += 1024) {
+            const double v = cum[k];
+            if constexpr (S) s_row[k] = v;
+            if (v != v) s_bad = 1;
+        }
+        if constexpr (S) {
             for (int k = threadIdx.x; k < nep; k += 1024) s_row[ng + k] = ep[k];
-        cum = s_row;
-        ep = s_row + ng;
+            cum = s_row;
+            ep = s_row + ng;
+        }
+    } else {
+        uint16_t *s_half = reinterpret_cast<uint16_t *>(s_row);      // low half: lower ends, high: upper
+        auto bucket = [](double c, bool up) {                          // BT_K: past the last bucket
+            const double v = c * (double)BT_K;
+            if (!(v > 0.0)) return 0;
+            if (v > (double)BT_K) return BT_K;
+            const int f = (int)v;
+            return up ? f + (v > (double)f) : (f < BT_K ? f : BT_K - 1);
+        };
+        for (int k = threadIdx.x; k < n; k += 1024) {
+            const double v = cum[k], w = k + 1 < n ? cum[k + 1] : INFINITY;
+            if (!(v <= w)) s_bad = 1;
+            const int cv = bucket(v, true), fv = bucket(v, false);
+            if (cv < BT_K && (k + 1 == n || bucket(w, true) != cv)) s_half[2 * ans_at(cv)] = (uint16_t)(k + 1);
+            if (fv < BT_K && (k + 1 == n || bucket(w, false) != fv)) s_half[2 * ans_at(fv) + 1] = (uint16_t)(k + 1);
+        }
     }
     __syncthreads();
-    // a row with a NaN (see slgpu_sample.h) keeps two searches of the whole row per bucket
-    const bool whole = s_nan != 0;
-    const double cg = d.capemgrey[ic - 1];
-    const int b0 = threadIdx.x * PER;
+    const bool bad = s_bad != 0;
     uint32_t ans[PER];
-    int at = 0;
-    #pragma unroll
-    for (int k = 0; k < 2 * PER; ++k) {
-        const double r = k & 1 ? bt_hi(b0 + k / 2) : bt_lo(b0 + k / 2);
-        int v;
-        if (emit) {
-            const double r1 = r * cg;
-            if (k == 0 || whole) {
+    if (emit) {
+        // a row with a NaN (see slgpu_sample.h) keeps two searches of the whole row per bucket
+        const double cg = d.capemgrey[ic - 1];
+        int at = 0;
+        #pragma unroll
+        for (int k = 0; k < 2 * PER; ++k) {
+            const double r1 = (k & 1 ? bt_hi(b0 + k / 2) : bt_lo(b0 + k / 2)) * cg;
+            int v;
+            if (k == 0 || bad) {
                 v = emitgroup_search(d, r1, ep, cum);
             } else {
                 // the bin index and the place in the bin resume at the answer before
@@ -560,16 +616,35 @@ __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
                 const int ig = iep * nepg + 1, igp1 = ig + nepg - 1 < ng ? ig + nepg - 1 : ng;
                 v = first_above_from(cum, (ig > at ? ig : at) - 1, igp1 - 1, r1) + 1;
             }
-        } else {
-            v = k == 0 || whole ? first_above(cum, 0, n, r) : first_above_from(cum, at, n, r);
+            at = v;
+            ans[k / 2] = k & 1 ? ans[k / 2] | (uint32_t)v << 15 : (uint32_t)v;
         }
-        at = v;
-        ans[k / 2] = k & 1 ? ans[k / 2] | (uint32_t)v << 15 : (uint32_t)v;
+    } else if (bad) {
+        #pragma unroll 1
+        for (int k = 0; k < PER; ++k) {
+            const int b = threadIdx.x + k * 1024;
+            const uint32_t lo = (uint32_t)first_above(cum, 0, n, bt_lo(b));
+            s_ans[ans_at(b)] = lo | (uint32_t)first_above(cum, 0, n, bt_hi(b)) << 16;
+        }
+        __syncthreads();
+        #pragma unroll
+        for (int k = 0; k < PER; ++k) { const uint32_t e = s_ans[ans_at(b0 + k)]; ans[k] = (e & 0xffffu) | e >> 16 << 15; }
+    } else {
+        uint32_t m = 0u;
+        #pragma unroll
+        for (int k = 0; k < PER; ++k) { m = max16(m, s_ans[ans_at(b0 + k)]); ans[k] = m; }
+        // what the threads before have reached
+        uint32_t before = __shfl_up(block_scan_max16(m, s_max), 1, 64);
+        if ((threadIdx.x & 63) == 0) {
+            before = 0u;
+            for (int k = 0; k < (int)(threadIdx.x >> 6); ++k) before = max16(before, s_max[k]);
+        }
+        #pragma unroll
+        for (int k = 0; k < PER; ++k) { const uint32_t e = max16(ans[k], before); ans[k] = (e & 0xffffu) | e >> 16 << 15; }
     }
     __syncthreads();
-    uint32_t *s_ans = reinterpret_cast<uint32_t *>(s_row);
     #pragma unroll
-    for (int k = 0; k < PER; ++k) s_ans[b0 + k] = ans[k];
+    for (int k = 0; k < PER; ++k) s_ans[ans_at(b0 + k)] = ans[k];
     __syncthreads();
     // a pure bucket's group and its destination's flags: the cell lc that receives the particle
     // (none past the outer face: it escapes) and the group a Doppler event shifts it to
@@ -581,7 +656,7 @@ __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
     #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int b = threadIdx.x + k * 1024;
-        uint32_t e = s_ans[b];
+        uint32_t e = s_ans[ans_at(b)];
         const int lo = (int)(e & 0x7fffu), hi = (int)(e >> 15);
         const bool pure = emit ? lo == hi : (lo < n ? lo : n - 1) == (hi < n ? hi : n - 1);
         const int g = !pure ? 0 : (emit ? lo : lump_group(d, L, ic, lo));
@@ -607,7 +682,7 @@ void launch_ddmc_tables(slgpu_ctx *c)
         hipLaunchKernelGGL(k_emitprob<true>, dim3(c->nx), dim3(256), rows, c->stream, c->d);
     else
         hipLaunchKernelGGL(k_emitprob<false>, dim3(c->nx), dim3(256), 0, c->stream, c->d);
-    const size_t lds = (size_t)(c->ng + c->d.nep) * sizeof(double), answers = BT_K * sizeof(uint32_t);
+    const size_t lds = (size_t)(c->ng + c->d.nep) * sizeof(double), answers = BT_ANSWERS;
     if (lds <= 160000)
         hipLaunchKernelGGL(k_bucket_tables<true>, dim3(c->nx, NTAB), dim3(1024), lds > answers ? lds : answers,
                            c->stream, c->d);
