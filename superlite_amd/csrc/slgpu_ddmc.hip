@@ -239,7 +239,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     }
     if (nl_eff == 0) return;
 
-    // pass 3: lump order and cumulative sampling weights
+    // pass 3: lump order
     int *gorder = d.gorder + (size_t)(l - 1) * ng;
     int baseL = 0, baseU = nl_eff;
     for (int g0 = 1; g0 <= ng; g0 += NT) {
@@ -256,39 +256,51 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         baseL += tl;
         baseU += tu;
     }
-    __syncthreads();
-    // a face or Doppler channel with zero total opacity is never chosen (its event
-    // probability is 0); its row is kept finite (all zero) so every row is monotone
-    const double hL = o1 > 0.0 ? 1.0 / o1 : 0.0, hR = o2 > 0.0 ? 1.0 / o2 : 0.0;
-    const double hD = c_doplump > 0.0 ? 1.0 / c_doplump : 0.0;
-    const double d2s = 1.0 / (1.0 - c_emitlump);
-    double *cL = d.cumL + (size_t)(l - 1) * ng, *cR = d.cumR + (size_t)(l - 1) * ng;
-    double *cD = d.cumD + (size_t)(l - 1) * ng, *cS = d.cumS + (size_t)(l - 1) * ng;
-    // the rows' terms; k_row_sums turns them into running sums
-    for (int p = threadIdx.x; p < nl_eff; p += NT) {
-        // the Doppler scan runs ascending for redshift, descending for blueshift
-        const int pd = divv >= 0 ? p : nl_eff - 1 - p;
-        const int g = gorder[p], gd = gorder[pd];
-        const double sp = spec[g - 1];
-        double tD = 0.0;
-        cL[p] = i > 1 ? sp * resleak(d, i, g, -1) * speclump * hL : 0.0;
-        cR[p] = sp * resleak(d, i, g, +1) * speclump * hR;
-        if (divv >= 0) {
-            if (gd != ng && !(CAPC(gd + 1, l) * dist >= d.taulump))
-                tD = dopspeccalc(tinv, d.wlinv, gd) * divv / (3 * PC_C) * speclump * hD;
-        } else {
-            if (gd != 1 && !(CAPC(gd - 1, l) * dist >= d.taulump))
-                tD = -(dopspeccalc(tinv, d.wlinv, gd - 1) * divv / (3 * PC_C) * speclump * hD);
-        }
-        cD[p] = tD;
-    }
-    for (int p = nl_eff + threadIdx.x; p < ng; p += NT) {
-        const int g = gorder[p];
-        cS[p] = spec[g - 1] * CAPE(g, l) * cgi * d2s;     // diffusion11.f90:574-581
-    }
 }
 
-// The running sums of the cells' sampling rows (the four lumped rows of k_leakage) and of their source
+// The terms of the running sums, one thread per (cell, position): the four lumped rows', in the order
+// k_leakage left, and the source spectrum's (interior_source.f90:69-75).  At the end of k_leakage
+// they had its 400 blocks alone, which leave half of the CUs half empty, and its register limit:
+// 400 x 10^4, both and the source terms 153 us together, 103 + 49 us so, the preparation 644 -> 625 us.
+__global__ __launch_bounds__(256) void k_row_terms(Dev d)
+{
+    const int ng = d.ng, nx = d.nx;
+    const int p = blockIdx.x * 256 + threadIdx.x, i = blockIdx.y + 1, l = i;
+    if (p >= ng) return;
+    const size_t row = (size_t)(l - 1) * ng;
+    d.srccum[row + p] = specintv_g(1.0 / d.radtemp[l - 1], d.wlinv, p + 1);
+    const CellDDMC cc = d.cell[l - 1];
+    if (cc.nlump == 0) return;
+    const int g = d.gorder[row + p];
+    const double *spec = d.specarr + row;
+    if (p >= cc.nlump) {
+        const double d2s = 1.0 / (1.0 - cc.emitlump);
+        d.cumS[row + p] = spec[g - 1] * CAPE(g, l) * cc.emgreyinv * d2s;     // diffusion11.f90:574-581
+        return;
+    }
+    // a face or Doppler channel with zero total opacity is never chosen (its event
+    // probability is 0); its row is kept finite (all zero) so every row is monotone
+    const double o1 = d.opaclump[(size_t)(l - 1) * 11], o2 = d.opaclump[(size_t)(l - 1) * 11 + 1];
+    const double hL = o1 > 0.0 ? 1.0 / o1 : 0.0, hR = o2 > 0.0 ? 1.0 / o2 : 0.0;
+    const double hD = cc.doplump > 0.0 ? 1.0 / cc.doplump : 0.0;
+    const double dist = DX(i), tinv = d.tempinv[l - 1], divv = d.divv[l - 1], speclump = cc.speclump;
+    // the Doppler scan runs ascending for redshift, descending for blueshift
+    const int gd = divv >= 0 ? g : d.gorder[row + cc.nlump - 1 - p];
+    const double sp = spec[g - 1];
+    double tD = 0.0;
+    d.cumL[row + p] = i > 1 ? sp * resleak(d, i, g, -1) * speclump * hL : 0.0;
+    d.cumR[row + p] = sp * resleak(d, i, g, +1) * speclump * hR;
+    if (divv >= 0) {
+        if (gd != ng && !(CAPC(gd + 1, l) * dist >= d.taulump))
+            tD = dopspeccalc(tinv, d.wlinv, gd) * divv / (3 * PC_C) * speclump * hD;
+    } else {
+        if (gd != 1 && !(CAPC(gd - 1, l) * dist >= d.taulump))
+            tD = -(dopspeccalc(tinv, d.wlinv, gd - 1) * divv / (3 * PC_C) * speclump * hD);
+    }
+    d.cumD[row + p] = tD;
+}
+
+// The running sums of the cells' sampling rows (the four lumped rows) and of their source
 // spectra, normalised Planck at T_rad (interior_source.f90:69-75, 96-103).  The reference
 // accumulates sequentially, and a sequential sum of nonnegative terms is monotone (a parallel
 // scan is not, by rounding), which the samplers' searches need.  So each row is one lane's
@@ -391,13 +403,6 @@ __device__ __forceinline__ double rows_sum(RowPtr const *p, const int *n, const 
         lds_barrier();
     }
     return s;
-}
-
-// the source spectrum's terms (interior_source.f90:69-75)
-__global__ __launch_bounds__(256) void k_src_terms(Dev d)
-{
-    const int g = blockIdx.x * 256 + threadIdx.x + 1, l = blockIdx.y;
-    if (g <= d.ng) d.srccum[(size_t)l * d.ng + g - 1] = specintv_g(1.0 / d.radtemp[l], d.wlinv, g);
 }
 
 __global__ __launch_bounds__(RS_THREADS) void k_row_sums(Dev d)
@@ -675,7 +680,7 @@ __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
 void launch_ddmc_tables(slgpu_ctx *c)
 {
     hipLaunchKernelGGL(k_leakage, dim3(c->nx), dim3(NT), 0, c->stream, c->d);
-    hipLaunchKernelGGL(k_src_terms, dim3((c->ng + 255) / 256, c->nx), dim3(256), 0, c->stream, c->d);
+    hipLaunchKernelGGL(k_row_terms, dim3((c->ng + 255) / 256, c->nx), dim3(256), 0, c->stream, c->d);
     hipLaunchKernelGGL(k_row_sums, dim3((c->nx + RS_ROWS - 1) / RS_ROWS, 5), dim3(RS_THREADS), 0, c->stream, c->d);
     const size_t rows = (size_t)c->ng * (sizeof(double) + sizeof(float));
     if (rows <= 143000)                            // beside 16 KB of bin sums
