@@ -137,6 +137,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     __shared__ int shi[NW];
     __shared__ double s_emax[NW];
     __shared__ int s_imax[NW];
+    __shared__ __align__(16) int s_cnt[2][NW];
     const int ng = d.ng, nx = d.nx;
     const int i = blockIdx.x + 1, l = i;
     const int icnb1 = i - 1 < 1 ? 1 : i - 1, icnb2 = i + 1 > nx ? nx : i + 1;
@@ -239,22 +240,31 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     }
     if (nl_eff == 0) return;
 
-    // pass 3: lump order
+    // pass 3: lump order.  Ballots count within a wave, the waves' counts meet in LDS (two sets that
+    // take turns, one barrier per 1024 groups), and unlumped places follow from the lumped ones.
     int *gorder = d.gorder + (size_t)(l - 1) * ng;
-    int baseL = 0, baseU = nl_eff;
-    for (int g0 = 1; g0 <= ng; g0 += NT) {
-        const int g = g0 + threadIdx.x;
-        int lump = 0;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int base = 0;                                  // lumped groups so far
+    for (int g0 = 0; g0 < ng; g0 += NT) {
+        const int g = g0 + threadIdx.x + 1;
+        bool lump = false;
         if (g <= ng) {
             const double c = CAPC(g, l);
-            lump = (c * dist >= d.taulump && (sg + c) * dist >= d.tauddmc) ? 1 : 0;
+            lump = c * dist >= d.taulump && (sg + c) * dist >= d.tauddmc;
         }
-        int tl, tu;
-        int pl = block_scan_int(lump, shi, tl);
-        int pu = block_scan_int(g <= ng ? 1 - lump : 0, shi, tu);
-        if (g <= ng) gorder[lump ? baseL + pl - 1 : baseU + pu - 1] = g;
-        baseL += tl;
-        baseU += tu;
+        const unsigned long long m = __ballot(lump);
+        int *cnt = s_cnt[(g0 / NT) & 1];
+        if (lane == 0) cnt[w] = __popcll(m);
+        __syncthreads();
+        int before = base + __popcll(m & ((1ull << lane) - 1ull)), total = 0;
+        #pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            const int v = cnt[k];
+            before += k < w ? v : 0;
+            total += v;
+        }
+        if (g <= ng) gorder[lump ? before : nl_eff + (g - 1 - before)] = g;
+        base += total;
     }
 }
 
