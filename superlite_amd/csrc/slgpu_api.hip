@@ -248,6 +248,7 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
     rc |= dalloc(c, &d.emitcum, cg);
     rc |= dparts(c, {{(void **)&d.emit, nc * 8}, {(void **)&d.radtemp, nc * 8}});
     rc |= dalloc(c, &d.srccum, cg);
+    rc |= dalloc(c, &d.srctot, nc);
     rc |= dalloc(c, &d.cell, nc);
     rc |= dalloc(c, &d.gcapT, cg);
     rc |= dalloc(c, &d.gmpart, (size_t)2 * ((ng + 63) / 64) * nc);

@@ -319,10 +319,11 @@ __global__ __launch_bounds__(256) void k_row_terms(Dev d)
 //     one per lane of its first wave (one row per block: 37 ns per value with the chip full);
 //   - the other eight waves store the tile before, write the tile after to LDS and request the one
 //     after that meanwhile, under barriers that wait for LDS alone (with __syncthreads() a tile
-//     took a load's and a store's round trip to memory: 12 ns a value instead of 8);
+//     took a load's and a store's round trip to memory: the two passes that the source rows had
+//     then 0.23 ms instead of 0.16);
 //   - the chain's LDS reads run 16 values ahead, in two register sets that take turns.
-// The source rows, which have two chains, start first.  400 x 10^4: 0.85 ms for the same chains on
-// global memory, 0.16 ms so (8 ns per value of the longest chain, the two source passes).
+// The source rows, the longest, start first; their totals come from k_emitprob.  400 x 10^4: 0.85 ms
+// for the same chains on global memory, 0.11 ms so (11 ns per value of the longest chain).
 constexpr int RS_ROWS = 8, RS_TILE = 256, RS_PITCH = RS_TILE + 2, RS_AHEAD = 16;
 constexpr int RS_THREADS = 576, RS_MOVERS = RS_THREADS - 64;
 typedef __attribute__((address_space(1))) double *RowPtr;     // not a flat access, which counts as one to LDS too
@@ -432,16 +433,11 @@ __global__ __launch_bounds__(RS_THREADS) void k_row_sums(Dev d)
         if (l >= d.nx) m = 0;
         p[t] = (RowPtr)base + (size_t)lc * ng;
         n[t] = m;
-        div[t] = 1.0;
+        div[t] = row < 0 ? d.srctot[lc] : 1.0;
         atomicMax(&s_max, m);
     }
     __syncthreads();
     if (s_max == 0) return;
-    if (row < 0) {
-        const double s = rows_sum<false>(p, n, div, s_max, buf);
-        if (t < RS_ROWS) div[t] = s;
-        __syncthreads();
-    }
     rows_sum<true>(p, n, div, s_max, buf);
 }
 
@@ -449,20 +445,37 @@ __global__ __launch_bounds__(RS_THREADS) void k_row_sums(Dev d)
 // cumulative sums emitgroup.f:38-50 walks.  A thread adds up a bin, in order; S: the cell's rows
 // pass through LDS both ways, since a wave's bins lie nepg groups apart (400 x 10^4: 87 us with
 // the strided global accesses, 53 us so).
+// The first blocks add up the source spectra, whose running sums are of the normalised terms: a chain
+// as long as k_row_sums' own, which hides behind the bins' blocks here (400 x 10^4: the bins 53 us
+// alone and 59 us with them, k_row_sums 162 us with both chains and 111 us with its own).
 template <bool S>
-__global__ __launch_bounds__(256) void k_emitprob(Dev d)
+__global__ __launch_bounds__(RS_THREADS) void k_emitprob(Dev d)
 {
-    extern __shared__ double s_spec[];                         // ng doubles, then ng floats
+    extern __shared__ __align__(16) double s_spec[];           // ng doubles, then ng floats
     __shared__ double binsum[1024];
     __shared__ double pref[1025];
-    const int ng = d.ng, nep = d.nep, nepg = d.nepg;
-    const int l = blockIdx.x + 1;
+    __shared__ RowPtr p[RS_ROWS];
+    __shared__ int n[RS_ROWS];
+    const int ng = d.ng, nep = d.nep, nepg = d.nepg, nsrc = (d.nx + RS_ROWS - 1) / RS_ROWS;
+    if ((int)blockIdx.x < nsrc) {
+        const int l = blockIdx.x * RS_ROWS + threadIdx.x;
+        if (threadIdx.x < RS_ROWS) {
+            p[threadIdx.x] = (RowPtr)d.srccum + (size_t)(l < d.nx ? l : d.nx - 1) * ng;
+            n[threadIdx.x] = l < d.nx ? ng : 0;
+            binsum[threadIdx.x] = 1.0;                         // no divisor
+        }
+        __syncthreads();
+        const double s = rows_sum<false>(p, n, binsum, ng, reinterpret_cast<double (*)[RS_ROWS][RS_PITCH]>(s_spec));
+        if (threadIdx.x < RS_ROWS && l < d.nx) d.srctot[l] = s;
+        return;
+    }
+    const int l = blockIdx.x - nsrc + 1;
     const double *spec = d.specarr + (size_t)(l - 1) * ng;
     const float *cap = d.capem32 + (size_t)(l - 1) * ng;
     double *cum = d.emitcum + (size_t)(l - 1) * ng, *out = cum;
     if constexpr (S) {
         float *s_cap = reinterpret_cast<float *>(s_spec + ng);
-        for (int g = threadIdx.x; g < ng; g += 256) {
+        for (int g = threadIdx.x; g < ng; g += RS_THREADS) {
             s_spec[g] = spec[g];
             s_cap[g] = cap[g];
         }
@@ -471,7 +484,7 @@ __global__ __launch_bounds__(256) void k_emitprob(Dev d)
         cap = s_cap;
         out = s_spec;
     }
-    for (int b = threadIdx.x; b < nep; b += 256) {
+    for (int b = threadIdx.x; b < nep; b += RS_THREADS) {
         const int g1 = (b + 1) * nepg < ng ? (b + 1) * nepg : ng;
         double s = 0.0;
         for (int g = b * nepg; g < g1; ++g) s = fma(spec[g], (double)cap[g], s);
@@ -488,7 +501,7 @@ __global__ __launch_bounds__(256) void k_emitprob(Dev d)
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < nep; b += 256) {
+    for (int b = threadIdx.x; b < nep; b += RS_THREADS) {
         ep[b] = b < nep - 1 ? pref[b + 1] : d.capemgrey[l - 1];
         const int g1 = (b + 1) * nepg < ng ? (b + 1) * nepg : ng;
         double s = pref[b];
@@ -500,7 +513,7 @@ __global__ __launch_bounds__(256) void k_emitprob(Dev d)
     if constexpr (S) {
         __syncthreads();
         const int n = nep * nepg < ng ? nep * nepg : ng;
-        for (int g = threadIdx.x; g < n; g += 256) cum[g] = s_spec[g];
+        for (int g = threadIdx.x; g < n; g += RS_THREADS) cum[g] = s_spec[g];
     }
 }
 
@@ -691,12 +704,15 @@ void launch_ddmc_tables(slgpu_ctx *c)
 {
     hipLaunchKernelGGL(k_leakage, dim3(c->nx), dim3(NT), 0, c->stream, c->d);
     hipLaunchKernelGGL(k_row_terms, dim3((c->ng + 255) / 256, c->nx), dim3(256), 0, c->stream, c->d);
-    hipLaunchKernelGGL(k_row_sums, dim3((c->nx + RS_ROWS - 1) / RS_ROWS, 5), dim3(RS_THREADS), 0, c->stream, c->d);
     const size_t rows = (size_t)c->ng * (sizeof(double) + sizeof(float));
+    const size_t tiles = sizeof(double) * 3 * RS_ROWS * RS_PITCH;
+    const unsigned rblocks = (c->nx + RS_ROWS - 1) / RS_ROWS;
     if (rows <= 143000)                            // beside 16 KB of bin sums
-        hipLaunchKernelGGL(k_emitprob<true>, dim3(c->nx), dim3(256), rows, c->stream, c->d);
+        hipLaunchKernelGGL(k_emitprob<true>, dim3(rblocks + c->nx), dim3(RS_THREADS), rows > tiles ? rows : tiles,
+                           c->stream, c->d);
     else
-        hipLaunchKernelGGL(k_emitprob<false>, dim3(c->nx), dim3(256), 0, c->stream, c->d);
+        hipLaunchKernelGGL(k_emitprob<false>, dim3(rblocks + c->nx), dim3(RS_THREADS), tiles, c->stream, c->d);
+    hipLaunchKernelGGL(k_row_sums, dim3(rblocks, 5), dim3(RS_THREADS), 0, c->stream, c->d);
     const size_t lds = (size_t)(c->ng + c->d.nep) * sizeof(double), answers = BT_ANSWERS;
     if (lds <= 160000)
         hipLaunchKernelGGL(k_bucket_tables<true>, dim3(c->nx, NTAB), dim3(1024), lds > answers ? lds : answers,

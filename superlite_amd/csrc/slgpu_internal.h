@@ -120,6 +120,7 @@ struct Dev {
     double *emit;               // nc
     double *radtemp;            // nc
     double *srccum;             // nc*ng  cumulative normalised Planck at T_rad
+    double *srctot;             // nc     its total before normalisation
     CellDDMC *cell;             // nc
     DdmcProb *cprob;            // nc     lumped-group step of each cell
     DdmcProb *gprob;            // nc*ng  unlumped step of each (cell, group), group-fastest
