@@ -3,9 +3,9 @@
 // sampling tables that replace the reference's per-event O(ng) linear scans
 // (GRID/emitgroup.f:23-51, TRANSPORT1/diffusion11.f90:289-313, 375-398, 447-460,
 // 489-511, 571-584; SOURCE/interior_source.f90:96-103) by cumulative rows plus exact
-// bucket maps (slgpu_sample.h), so a sampled group usually costs one table load.  One
-// 1024-thread block per cell; groups are swept in chunks of 1024 with block-wide (wave64
-// shuffle) scans carrying the running prefix.
+// bucket maps (slgpu_sample.h), so a sampled group usually costs one table load.  Per cell:
+// lumped sums and lump order (k_leakage), the rows' terms (k_row_terms), emission bins and source
+// totals (k_emitprob), the rows' running sums (k_row_sums), the bucket maps (k_bucket_tables).
 #include "slgpu_device.h"
 #include "slgpu_internal.h"
 #include "slgpu_sample.h"
