@@ -235,6 +235,7 @@ struct slgpu_ctx {
     std::vector<double> h_emit_cache;
     double line_top = 0.0;      // largest lower level of the used lines [1/cm]; 0: no tables
     double hckt_max = 0.0;      // largest hc/kT of the last build's cells
+    double etab_step = 0.0;     // line_step that Dev::etab was filled with for the last build's cells; 0: not
     int opac_flags = 0;         // flags of the last opacity build (its backward uses them)
     std::vector<void *> allocations;
     bool have_eos_data = false, have_eos = false;
@@ -261,6 +262,7 @@ void launch_cell_prep(slgpu_ctx *c, const double *d_natom, const double *d_vol,
                       const double *d_nelec, const double *d_oc, const double *d_ginv,
                       int flags);
 void launch_lines64(slgpu_ctx *c, int64_t n);
+void launch_exp_table(slgpu_ctx *c);
 int line_degree(const slgpu_ctx *c);
 void launch_eos_ndens(slgpu_ctx *c, const double *temp, const double *mass, const double *natom,
                       const double *natomfr, double *ndens);

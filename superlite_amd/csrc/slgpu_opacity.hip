@@ -563,8 +563,8 @@ void launch_cell_prep(slgpu_ctx *c, const double *d_natom, const double *d_vol,
     int n = c->nx * nk;
     hipLaunchKernelGGL(k_cell_prep, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d,
                        d_natom, d_vol, d_nelec, d_oc, d_ginv, flags, g_rgg_scratch(c));
-    if (c->d.line_step > 0.0 && !(flags & SLGPU_NOBB))
-        hipLaunchKernelGGL(k_exp_table, dim3((EXP_ROWS * c->nx + 255) / 256), dim3(256), 0, c->stream, c->d);
+    c->etab_step = 0.0;                            // the cells are other ones
+    if (!(flags & SLGPU_NOBB)) launch_exp_table(c);
     if (!(flags & SLGPU_NOFF))
         hipLaunchKernelGGL(k_ff_table, dim3(c->nx), dim3(128), 0, c->stream, c->d,
                            (const double *)g_rgg_scratch(c));
@@ -579,6 +579,16 @@ double ff_prefactor()
 }
 
 const double *rgg_scratch(slgpu_ctx *c) { return g_rgg_scratch(c); }
+
+// The cells' exponential tables for the present lines' step.  A build fills them; its backward comes
+// here too, since other lines or groups (another step) may have been set in between.
+void launch_exp_table(slgpu_ctx *c)
+{
+    if (c->etab_step == c->d.line_step) return;
+    c->etab_step = c->d.line_step;
+    if (c->d.line_step > 0.0)
+        hipLaunchKernelGGL(k_exp_table, dim3((EXP_ROWS * c->nx + 255) / 256), dim3(256), 0, c->stream, c->d);
+}
 
 void launch_lines64(slgpu_ctx *c, int64_t n)
 {

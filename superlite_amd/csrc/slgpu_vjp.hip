@@ -583,9 +583,12 @@ void launch_opacity_vjp(slgpu_ctx *c, int flags, const double *gc, const double 
             if (mixed)
                 hipLaunchKernelGGL((k_vjp_opacity<true, true, 1, 8>), grid, dim3(512), bb_b + pop_b, c->stream,
                                    c->d, flags, ffc1, rgg);
-            else if (deg == 6) launch_vjp_lines64<6>(c, lds64);
-            else if (deg == 8) launch_vjp_lines64<8>(c, lds64);
-            else launch_vjp_lines64<10>(c, lds64);
+            else {
+                launch_exp_table(c);
+                if (deg == 6) launch_vjp_lines64<6>(c, lds64);
+                else if (deg == 8) launch_vjp_lines64<8>(c, lds64);
+                else launch_vjp_lines64<10>(c, lds64);
+            }
         }
         if (!(flags & SLGPU_NOFF) && c->d.nel > 0)
             hipLaunchKernelGGL((k_vjp_opacity<true, false, 2, 4>), grid, dim3(256), ff_b, c->stream,
