@@ -597,13 +597,19 @@ __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
     }
     __syncthreads();
     if (emit) {
+        // searches that resume need bins whose sums rise, bins that rise and draws that rise
+        if (threadIdx.x == 0 && !(d.capemgrey[ic - 1] >= 0.0)) s_bad = 1;
         for (int k = threadIdx.x; k < n; k += 1024) {
             const double v = cum[k];
             if constexpr (S) s_row[k] = v;
-            if (v != v) s_bad = 1;
+            if (!(v >= (k % nepg != 0 ? cum[k - 1] : v))) s_bad = 1;
+        }
+        for (int k = threadIdx.x; k < nep; k += 1024) {
+            const double v = ep[k];
+            if constexpr (S) s_row[ng + k] = v;
+            if (k < nep - 1 && !(v >= (k > 0 ? ep[k - 1] : v))) s_bad = 1;
         }
         if constexpr (S) {
-            for (int k = threadIdx.x; k < nep; k += 1024) s_row[ng + k] = ep[k];
             cum = s_row;
             ep = s_row + ng;
         }
@@ -628,7 +634,8 @@ __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
     const bool bad = s_bad != 0;
     uint32_t ans[PER];
     if (emit) {
-        // a row with a NaN (see slgpu_sample.h) keeps two searches of the whole row per bucket
+        // a row that does not rise (a NaN, see slgpu_sample.h; negative line strengths) keeps two
+        // searches of the whole row per bucket
         const double cg = d.capemgrey[ic - 1];
         int at = 0;
         #pragma unroll

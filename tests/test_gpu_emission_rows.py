@@ -1,0 +1,43 @@
+"""The emission table's bucket maps where its running sums do not rise: lines of negative strength, which
+the line setter takes, leave groups of negative opacity.  A bucket whose two ends are answered alike by
+the plain search holds that answer; whole numbers, so the comparison is exact.  Rows searched in LDS
+and (ng + nep beyond 20000) in global memory, a bin per group and several groups per bin."""
+import numpy as np
+import pytest
+
+from test_gpu_lines64 import GAS, IZ, II, problem
+
+pytestmark = pytest.mark.gpu
+
+K = 1 << 14
+
+
+@pytest.mark.parametrize("nx,ng,nep", [(2, 60, 8), (3, 500, 22), (2, 3000, 55), (2, 300, 300), (1, 21_000, 145)])
+@pytest.mark.parametrize("negative", [0.1, 0.3])
+def test_falling_rows(tables, nx, ng, nep, negative):
+    from superlite_amd import slgpu as S
+    print("case: falling emission rows", nx, ng, nep, negative, flush=True)
+    wl, lines, st = problem(nx, ng, 3 * ng, 6000.0, ng)
+    sign = np.where(np.random.default_rng(1).random(3 * ng) < negative, -1.0, 1.0)
+    st["mass"][:] = 1.0
+    ctx = S.Context(nx, ng, nep, -(-ng // nep), npartmax=64, seed=5)
+    x = 1e14 * np.arange(nx + 1)
+    ctx.set_grid(x, x / 1.7e6, np.full(nx, 1.7e-6), 4.19 * np.diff(x ** 3), 0.5 * (x[1:] + x[:-1]))
+    ctx.set_groups(wl)
+    ctx.set_ions(IZ, II)
+    ctx.set_tables(*tables)
+    ctx.set_lines(lines[0], (lines[1] * sign).astype(np.float32), *lines[2:])
+    o = ctx.opacity_build(*[st[k] for k in GAS])
+    assert np.any(o["cap"] < 0.0)
+    ctx.ddmc_prep(st["temp"], 1e43)
+    b = np.arange(1, K, dtype=np.float64)                  # bucket 0 starts at a draw of 0, which is refused
+    lo, hi = b / K, np.nextafter((b + 1) / K, 0.0)
+    hi[-1] = 1.0
+    for i in range(1, nx + 1):
+        cell = np.full(K - 1, i, np.int32)
+        want = ctx.sample_groups(4, lo, cell, direct=True)
+        same = want == ctx.sample_groups(4, hi, cell, direct=True)
+        assert same.sum() > K // 3
+        for r in (lo, hi):
+            assert np.array_equal(ctx.sample_groups(4, r, cell)[same], want[same])
+    ctx.close()
