@@ -26,6 +26,7 @@
 // bb line terms are FP32 in short partial sums folded into FP64, like that form's forward; bf, ff,
 // the means and every accumulator stay FP64.  Elements absent from every cell are skipped
 // by the forward's ff sum, so their mass-fraction gradient is returned as 0.
+#include <type_traits>
 #include "slgpu_device.h"
 #include "slgpu_internal.h"
 
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(NWV * 64)
 __attribute__((amdgpu_waves_per_eu(P == 1 ? 6 : 1, 8)))
 void k_vjp_opacity(Dev d, int flags, double ffc1, const double *__restrict__ rgg_tab)
 {
-    using PT = float;              // staged populations: the precision form only
+    using PT = typename std::conditional<M, float, double>::type;
     constexpr bool BB = (P & 1) != 0, FF = (P & 2) != 0;
     constexpr int NT = NWV * 64;
     extern __shared__ double s_acc[];
@@ -271,15 +272,46 @@ void k_vjp_opacity(Dev d, int flags, double ffc1, const double *__restrict__ rgg
                 s0 = pe * t0;
                 s1 = pe * t1;
             } else {
-                for (int l = l0; l < l1; ++l) {
-                    const LineRec r = d.lines[l];
-                    const double o = ocg[(size_t)r.ion * nc];
-                    if (o > 0.0) {
-                        const double base = phi * (double)r.gxs * exp(-((double)r.chilw * hckt)) * expfac;
-                        const double term = base * o;
-                        s0 += term;
-                        s1 += term * (double)r.chilw;
-                        atomicAdd(&s_bb[r.ion * 64 + lane], G * base);
+                // a line's term to the sums; its part of the ion's derivative
+                auto add = [&](const LineRec &r, double o) {
+                    const double base = phi * (double)r.gxs * exp(-((double)r.chilw * hckt)) * expfac;
+                    const double term = base * o;
+                    s0 += term;
+                    s1 += term * (double)r.chilw;
+                    return base;
+                };
+                if constexpr (S) {
+                    LineRec *ln = s_lines[wave];
+                    int cur = -1;
+                    double o = 0.0, sb = 0.0;
+                    for (int base0 = l0; base0 < l1; base0 += 64) {
+                        const int n = l1 - base0 < 64 ? l1 - base0 : 64;
+                        wave_lds_sync();
+                        if (lane < n) ln[lane] = d.lines_ion[base0 + lane];
+                        wave_lds_sync();
+                        // one run of an ion's lines at a time (pad: lines left in the run)
+                        for (int j = 0; j < n;) {
+                            const int ion = __builtin_amdgcn_readfirstlane(ln[j].ion);
+                            int len = __builtin_amdgcn_readfirstlane(ln[j].pad);
+                            len = len < n - j ? len : n - j;
+                            len = len > 1 ? len : 1;                 // always advances
+                            if (ion != cur) {
+                                if (sb != 0.0) atomicAdd(&s_bb[cur * 64 + lane], G * sb);
+                                cur = ion;
+                                sb = 0.0;
+                                o = s_pop[ion * 64 + lane];
+                            }
+                            if (o > 0.0)
+                                for (int t = j; t < j + len; ++t) sb += add(ln[t], o);
+                            j += len;
+                        }
+                    }
+                    if (sb != 0.0) atomicAdd(&s_bb[cur * 64 + lane], G * sb);
+                } else {
+                    for (int l = l0; l < l1; ++l) {
+                        const LineRec r = d.lines[l];
+                        const double o = ocg[(size_t)r.ion * nc];
+                        if (o > 0.0) atomicAdd(&s_bb[r.ion * 64 + lane], G * add(r, o));
                     }
                 }
             }
@@ -569,21 +601,22 @@ void launch_opacity_vjp(slgpu_ctx *c, int flags, const double *gc, const double 
     const bool mixed = c->d.precision == SLGPU_MIXED;
     const size_t acc_b = (size_t)(c->nion + c->d.nel) * 64 * sizeof(double);
     const size_t bb_b = (size_t)c->nion * 64 * sizeof(double), ff_b = (size_t)c->d.nel * 64 * sizeof(double);
-    const size_t pop_b = (size_t)c->nion * 64 * sizeof(float);
-    // The bb lines run in a kernel of their own, ff in another, when the cells' populations (and in
-    // FP64 their exponential tables) fit in LDS beside the accumulators; otherwise both in one
-    // 256-thread kernel, populations unstaged.  Precision form: 8 waves x 2 groups share the
-    // cells' accumulators within 64 KiB.
+    const size_t pop_b = (size_t)c->nion * 64 * (mixed ? sizeof(float) : sizeof(double));
+    // The bb lines run in a kernel of their own, ff in another, when the cells' populations fit in LDS
+    // beside the accumulators: in FP64 together with their exponential tables, otherwise (the precision
+    // form; FP64 without tables) within 64 KiB with the line slots of 8 waves x 2 groups.  Beyond,
+    // both parts run in one 256-thread kernel, populations unstaged.  FP64 without tables, at 250 K: 64 x 1000
+    // groups x 1e5 lines 0.16 ms staged and 0.42 ms unstaged, 400 x 10^4 x 2e6 lines 1.4 and 3.0 ms.
     const size_t lds64 = ((size_t)2 * c->nion + EXP_ROWS) * 64 * sizeof(double);
     const int deg = c->force_unstaged || mixed || lds64 > 163840 ? 0 : line_degree(c);
-    const bool staged = mixed ? !c->force_unstaged && bb_b + pop_b + 8 * 64 * sizeof(LineRec) <= 65536 : deg > 0;
+    const bool staged = deg > 0 || (!c->force_unstaged && bb_b + pop_b + 8 * 64 * sizeof(LineRec) <= 65536);
     dim3 grid((nc + 63) / 64, (ng + VJP_GROUPS - 1) / VJP_GROUPS);
     if (staged) {
         if (!(flags & SLGPU_NOBB) && c->nion > 0) {
-            if (mixed)
-                hipLaunchKernelGGL((k_vjp_opacity<true, true, 1, 8>), grid, dim3(512), bb_b + pop_b, c->stream,
-                                   c->d, flags, ffc1, rgg);
-            else {
+            if (deg == 0) {
+                auto kernel = mixed ? k_vjp_opacity<true, true, 1, 8> : k_vjp_opacity<false, true, 1, 8>;
+                hipLaunchKernelGGL(kernel, grid, dim3(512), bb_b + pop_b, c->stream, c->d, flags, ffc1, rgg);
+            } else {
                 launch_exp_table(c);
                 if (deg == 6) launch_vjp_lines64<6>(c, lds64);
                 else if (deg == 8) launch_vjp_lines64<8>(c, lds64);
