@@ -298,9 +298,12 @@ int slgpu_create(const slgpu_config *cfg, slgpu_ctx **out)
                      {(void **)&c->eos_natom, nc * 8}, {(void **)&c->eos_natomfr, 30 * nc * 8},
                      {(void **)&c->eos_niter, nc * 4}});
     if (!rc) {
-        // inputs of a call: 35 per-cell numbers and two per ion; outputs: up to 20 bytes per (cell,
-        // group) and some hundred per cell.  What does not fit goes straight from the caller's memory.
-        const hipError_t e = c->io.create(std::min((size_t)4 << 20, nc * 167 * 8 + 4096), 20 * cg + 200 * 8 * nc);
+        // inputs of a call: 35 per-cell numbers and two per ion; what does not fit goes straight from the
+        // caller's memory.  Outputs: up to 20 bytes per (cell, group) and some hundred per cell, or the
+        // particles' 49 bytes each (10^6 of them on 4 x 16 groups: 434 ms through a ring sized by the
+        // grid alone, 2.8 ms so).
+        const hipError_t e = c->io.create(std::min((size_t)4 << 20, nc * 167 * 8 + 4096),
+                                          std::max(20 * cg + 200 * 8 * nc, 49 * np));
         if (e != hipSuccess) rc = fail(SLGPU_ENOMEM, std::string("hipHostMalloc: ") + hipGetErrorString(e));
     }
     if (rc) {

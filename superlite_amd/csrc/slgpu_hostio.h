@@ -25,7 +25,8 @@
 
 namespace slgpu {
 
-// The pinned memory of one context: 12 MiB at most, less where its largest output is smaller.
+// The pinned memory of one context, 16 MiB at most: a ring of 12 MiB for outputs, less where its largest
+// output is smaller, and up to 4 MiB of inputs.
 struct HostIO {
     static constexpr int SLOTS = 6;
     static constexpr size_t CHUNK = (size_t)2 << 20;
