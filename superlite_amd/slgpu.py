@@ -266,7 +266,7 @@ class Context:
     def transport(self, iteration, want=True, check=True):
         nc, ng = self.nx, self.ng
         tally = np.zeros(nc) if want else None
-        jrad = np.empty((nc, ng)) if want else None
+        jrad = np.zeros((nc, ng)) if want else None       # returned as it is when a call fails unchecked
         eamp = np.zeros(nc) if want else None
         tot = np.zeros(7)
         ct = np.zeros(10, np.int64)
