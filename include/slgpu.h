@@ -283,11 +283,12 @@ int slgpu_set_unstaged(slgpu_ctx *ctx, int on);
 int slgpu_sample_groups(slgpu_ctx *ctx, int table, int direct, int64_t n, const double *r,
                         const int *cell, int *out_group);
 
-/* accumulated device time per phase in ms, measured with HIP events on the context
- * stream: [0] opacity, [1] ddmc prep, [2] sources, [3] transport, [4] fluxtally,
- * [5] opacity bb+bf+ff kernel alone, [6] transport kernel alone, [7] opacity backward,
- * [8] EOS, [9] EOS backward, [10] opacity backward kernels alone, [11] opacity forward
- * kernels alone (cell prep, bb+bf+ff, transpose, means); n <= 12; reset = 1 zeroes them */
+/* accumulated time per phase in ms, measured with HIP events on the context stream and, past the
+ * last device copy, on the host until the caller's arrays hold the outputs: [0] opacity,
+ * [1] ddmc prep, [2] sources, [3] transport, [4] fluxtally, [5] opacity bb+bf+ff kernel alone,
+ * [6] transport kernel alone, [7] opacity backward, [8] EOS, [9] EOS backward, [10] opacity
+ * backward kernels alone, [11] opacity forward kernels alone (cell prep, bb+bf+ff, transpose,
+ * means); n <= 12; reset = 1 zeroes them */
 int slgpu_timers(slgpu_ctx *ctx, double *ms, int n, int reset);
 
 /* the HIP stream all work of the context is ordered on (hipStream_t) */

@@ -112,7 +112,7 @@ struct PhaseTimer {
         if (e != hipSuccess) return fail(SLGPU_EHIP, std::string("device: ") + hipGetErrorString(e));
         float ms = 0.f;
         hipEventElapsedTime(&ms, c->ev[2 * slot], c->ev[2 * slot + 1]);
-        c->t_ms[slot] += ms;
+        c->t_ms[slot] += ms + out.tail_ms();
         return 0;
     }
 };

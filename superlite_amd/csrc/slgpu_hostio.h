@@ -168,7 +168,7 @@ public:
         gate_.store(made ? made : -1, std::memory_order_release);
     }
 
-    // the last copy is followed by `last` on the stream, which is drained on return
+    // `last` follows the last copy on the stream, which is drained on return
     hipError_t finish(hipEvent_t last)
     {
         hipError_t e = hipSuccess;
@@ -182,6 +182,7 @@ public:
             return e;
         }
         int issued = 0;
+        auto t_last = std::chrono::steady_clock::now();
         for (int k = 0; k < n && e == hipSuccess; ++k) {
             while (issued < n && issued < k + io_.slots && e == hipSuccess) {
                 if (issued >= io_.slots && workers_ > 0) {
@@ -196,14 +197,19 @@ public:
             }
             if (e == hipSuccess) e = hipEventSynchronize(k == n - 1 ? last : io_.ev[k % io_.slots]);
             if (e != hipSuccess) break;
+            t_last = std::chrono::steady_clock::now();
             if (workers_ > 0) ready_.store(k + 1, std::memory_order_release);
             else copy(k, 0, chunks_[k].n);
         }
         if (e != hipSuccess) stop_.store(true, std::memory_order_release);
         else io_.busy = false;
         end();
+        tail_ms_ = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_last).count();
         return e;
     }
+
+    // from `last` until the caller's arrays held everything, which the event does not cover
+    double tail_ms() const { return tail_ms_; }
 
 private:
     struct Item {
@@ -297,6 +303,7 @@ private:
     std::atomic<int> ready_{0}, gate_{0};
     std::atomic<bool> stop_{false};
     int workers_ = 0;
+    double tail_ms_ = 0.0;
 };
 
 }  // namespace slgpu
