@@ -12,6 +12,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <sched.h>
 #include <sys/mman.h>
 #include <unistd.h>
 
@@ -152,8 +153,9 @@ public:
             }
             total += t.n;
         }
-        // a thread per MiB, up to 8: one thread copies 8-10 GB/s
-        workers_ = total < ((size_t)1 << 20) ? 0 : (int)std::min<size_t>(8, total >> 20);
+        // a thread per MiB, up to 8 (one copies 8-10 GB/s), on cores beside the caller's: a rank bound to
+        // one core copies by itself
+        workers_ = (int)std::min<size_t>(std::min(8, spare_cores()), total >> 20);
         if (!workers_) return;
         done_.reset(new std::atomic<int>[chunks_.size()]);
         for (size_t k = 0; k < chunks_.size(); ++k) done_[k].store(0, std::memory_order_relaxed);
@@ -228,6 +230,13 @@ private:
         int seg, nseg;
         size_t n;
     };
+
+    // cores that threads of the caller may run on, less its own
+    static int spare_cores()
+    {
+        cpu_set_t s;
+        return sched_getaffinity(0, sizeof(s), &s) == 0 ? CPU_COUNT(&s) - 1 : 8;
+    }
 
     hipError_t issue(int k, hipEvent_t done)
     {

@@ -4,6 +4,8 @@
 #include "../../superlite_amd/csrc/slgpu_hostio.h"
 
 #include <cstdio>
+#include <dirent.h>
+#include <sched.h>
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned int) { *p = malloc(n); return *p ? hipSuccess : hipErrorOutOfMemory; }
@@ -13,12 +15,28 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned int) { *e = (hipEvent_t)malloc(1); return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t);
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *, const void *) { return hipErrorInvalidValue; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 }
 
-static int failures = 0;
+static int failures = 0, most_threads = 0;
+
+static int threads()
+{
+    int n = 0;
+    DIR *d = opendir("/proc/self/task");
+    while (dirent *e = readdir(d)) n += e->d_name[0] != '.';
+    closedir(d);
+    return n;
+}
+
+hipError_t hipEventSynchronize(hipEvent_t)
+{
+    most_threads = std::max(most_threads, threads());
+    return hipSuccess;
+}
+
 static void check(bool ok, const char *what, size_t n)
 {
     printf("%s %s %zu\n", ok ? "ok" : "FAILED", what, n);
@@ -29,7 +47,16 @@ static void check(bool ok, const char *what, size_t n)
 int main()
 {
     using namespace slgpu;
+    cpu_set_t all;
+    if (sched_getaffinity(0, sizeof(all), &all) != 0) return 98;
+    for (int cores : {CPU_COUNT(&all), std::min(2, CPU_COUNT(&all)), 1})
     for (size_t n : {(size_t)1, (size_t)4096, (size_t)1048575, (size_t)1048576, (size_t)2097153, (size_t)30000001}) {
+        cpu_set_t s;
+        CPU_ZERO(&s);
+        for (int k = 0; k < CPU_SETSIZE && CPU_COUNT(&s) < cores; ++k)
+            if (CPU_ISSET(k, &all)) CPU_SET(k, &s);
+        sched_setaffinity(0, sizeof(s), &s);
+        most_threads = 0;
         HostIO io;
         if (io.create(4096, n) != hipSuccess) return 99;
         std::vector<char> dev(n + 77), a(n, 0), b(77, 0);
@@ -46,6 +73,9 @@ int main()
             // events here are complete before the copies out of the ring begin
             check(out.tail_ms() > 0.0 && out.tail_ms() <= wall, "tail", n);
         }
+        // at most eight threads beside the caller's, each with a MiB to copy and a core to run on
+        const size_t most = std::min<size_t>({8, (n + 77) >> 20, (size_t)CPU_COUNT(&s) - 1});
+        check(most_threads <= 1 + (int)most, "threads", n);
         io.destroy();
     }
     return failures;

@@ -1,6 +1,7 @@
 """The host side of the transfers (slgpu_hostio.h), compiled for the CPU against a HIP runtime of a few
-lines (tests/cpp/hostio_check.cpp): bytes arrive whole, and the time from the last device copy until the
-caller's arrays are filled is reported, which the phase timers add to their events' time."""
+lines (tests/cpp/hostio_check.cpp): bytes arrive whole, the time from the last device copy until the
+caller's arrays are filled is reported, which the phase timers add to their events' time, and the copying
+threads are no more than the cores the process may use beside the caller's."""
 import os
 import shutil
 import subprocess
