@@ -304,9 +304,10 @@ void launch_eos_vjp(slgpu_ctx *c, const double *temp, const double *mass, const 
 // The tables (64 entries per cell, k_exp_table) stand in LDS as rows of the block's 64 cells; k1, k2, r
 // and gxs are the same for the whole wave and come as scalars.  That is 10 FP64 operations
 // and two LDS rows per line and cell, against about 50 for exp() and the reference's product;
-// its error is that of the table entries (2 units in the last place), below the rounding of
-// the product chi h that exp() takes.  P is the Taylor polynomial of degree DEG; the launch
-// picks the smallest whose remainder at the largest |r h| stays under 2^-53.
+// its error is that of the table entries and their products (2-3 units in the last place; exp()
+// takes the product chi h rounded, an error of chi h / 2 units, more from chi h = 5 on).  P is the
+// Taylor polynomial of degree DEG; the launch picks the smallest whose remainder, relative to the
+// exponential at the largest |r h|, stays under 2^-53 (line_degree).
 template <int DEG> __device__ __forceinline__ double exp_poly(double x)
 {
     constexpr double inv[13] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,

@@ -613,13 +613,13 @@ void launch_lines64(slgpu_ctx *c, int64_t n)
 }
 
 // degree of the line sums' polynomial for the last build's cells: the smallest of 6, 8 and 10 whose
-// Taylor remainder x^(n+1)/(n+1)! at the largest x = step/2 hc/kT is under 2^-53; 0 when there
-// are no tables or the cells are too cold for them (exp() per line then)
+// Taylor remainder, relative to exp(-x) at the largest x = step/2 hc/kT (about e^x x^(n+1)/(n+1)!), is
+// under 2^-53; 0 when there are no tables or the cells are too cold for them (exp() per line then)
 int line_degree(const slgpu_ctx *c)
 {
     const double x = 0.5 * c->d.line_step * c->hckt_max;
     if (!(x > 0.0)) return 0;
-    return x <= 0.0177 ? 6 : (x <= 0.069 ? 8 : (x <= 0.176 ? 10 : 0));
+    return x <= 0.0177 ? 6 : (x <= 0.069 ? 8 : (x <= 0.171 ? 10 : 0));
 }
 
 // LDS of k_opacity64: tables, populations and the waves' partial sums
