@@ -1205,10 +1205,14 @@ void launch_transport(slgpu_ctx *c, uint32_t iteration)
     int dev = 0, ncu = 256;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    const int64_t blocks = (int64_t)ncu * 8;
     const int64_t resident = (int64_t)ncu * 4 * (c->d.precision == SLGPU_MIXED ? SLGPU_WAVES_MIXED : SLGPU_WAVES_FP64);
-    const int64_t share = (c->d.npart + resident - 1) / resident;
-    const int lanes = share < 1 ? 1 : (share > 64 ? 64 : (int)share);
+    // Pure IMC: half waves at least.  Its passes cost a wave as much for 1 to 8 lanes as for 64, and less
+    // for 16 to 32 (20 x 300, 3000 steps each, FP64: 300 particles 22 ms alone, 21 by 8, 15 by 16, 13 by
+    // 32 and 14 by 64; 3000 21, 23, 16, 14 and 17; precision form alike).
+    const int64_t share = std::max<int64_t>(c->d.puretran ? 32 : 1, (c->d.npart + resident - 1) / resident);
+    const int lanes = share > 64 ? 64 : (int)share;
+    // no more blocks than take particles: an empty pool's 2048 cost 90 us of queue and flush
+    const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((int64_t)ncu * 8, (c->d.npart + 4 * lanes - 1) / (4 * lanes)));
     const bool extra = c->d.ampfact || c->d.thm_aniso;
     auto kernel = c->d.precision == SLGPU_MIXED ? (extra ? k_transport<true, true> : k_transport<true, false>)
                                                 : (extra ? k_transport<false, true> : k_transport<false, false>);
