@@ -391,7 +391,8 @@ def main():
                      "traffic": measured_traffic(kname, args.workload),
                      "kernel": kname, "kernel_ms": t_kernel * 1e3,
                      "algorithmic_bytes": f"36 B/particle-step + 2x{state_b:.0f} B/particle",
-                     "limiter": "latency and divergence (lanes active, wave waits), not bandwidth"},
+                     "limiter": "latency and divergence (lanes active, wave waits); its gathers' lines beyond L2 "
+                                "move at a copy's rate (traffic over kernel_ms)"},
         "roofline_opacity": {"bound": "exp", "kernel": "k_opacity<true>" if mixed else "k_opacity<false>",
                              "achieved": line_evals / t_opk, "peak": exp_peak,
                              "unit": "line evaluations/s vs measured " +

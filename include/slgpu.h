@@ -268,8 +268,9 @@ int slgpu_eos_vjp(slgpu_ctx *ctx, const double *grad_natom, const double *grad_n
 
 /* Verification hook, no counterpart in the reference: on = 1 makes the context's opacity
  * build and its backward take the kernels they use when the ion populations do not fit in
- * LDS (more than 256 ions for the build in the precision form, 128 in FP64; about 74 and 56
- * for the backward), so tests can compare them with the staged kernels on small inputs.
+ * LDS (more than 256 ions for the build and about 74 for the backward in the precision form; in
+ * FP64 more than 240 for the build, or 128 and 56 where a cell is too cold or a level unsuited
+ * to the exponential tables), so tests can compare them with the staged kernels on small inputs.
  * on = 0 (the default) restores the choice by size. */
 int slgpu_set_unstaged(slgpu_ctx *ctx, int on);
 
