@@ -5,7 +5,8 @@
 // 489-511, 571-584; SOURCE/interior_source.f90:96-103) by cumulative rows plus exact
 // bucket maps (slgpu_sample.h), so a sampled group usually costs one table load.  Per cell:
 // lumped sums and lump order (k_leakage), the rows' terms (k_row_terms), emission bins and source
-// totals (k_emitprob), the rows' running sums (k_row_sums), the bucket maps (k_bucket_tables).
+// totals (k_emitprob), the rows' running sums (k_row_sums), the bucket maps (k_bucket_tables; few
+// cells: k_bucket_search).
 #include "slgpu_device.h"
 #include "slgpu_internal.h"
 #include "slgpu_sample.h"
@@ -707,6 +708,41 @@ __global__ __launch_bounds__(1024) void k_bucket_tables(Dev d)
     }
 }
 
+// The same maps by two plain searches per bucket, a thread per (bucket, cell, table): 64 blocks a map where
+// k_bucket_tables has one, for meshes whose maps leave most CUs without a block there.  The whole
+// preparation, blocks against searches: 2 x 16 groups 62 and 39 us, 20 x 250 72 and 60, 24 x 250 72 and 64,
+// 24 x 4000 158 and 153, 32 x 250 72 and 70, 32 x 4000 161 and 167, 64 x 250 75 and 98: up to 24 cells.
+constexpr int BT_SEARCH_CELLS = 24;
+__global__ __launch_bounds__(256) void k_bucket_search(Dev d)
+{
+    const int b = blockIdx.x * 256 + threadIdx.x, ic = blockIdx.y + 1, t = blockIdx.z;
+    const double rlo = bt_lo(b), rhi = bt_hi(b);
+    int lo, hi, g = 0;
+    if (t == TAB_E) {
+        lo = emitgroup_direct(d, rlo, ic);
+        hi = emitgroup_direct(d, rhi, ic);
+        if (lo == hi) g = lo;
+    } else {
+        const int nlump = d.cell[ic - 1].nlump;
+        const LumpRow L = lump_row(d, t, ic, nlump);
+        if (nlump == 0 || L.cnt <= 0) {
+            d.btab[((size_t)t * d.nx + (ic - 1)) * BT_K + b] = 0u;
+            return;
+        }
+        lo = first_above(L.cum, 0, L.cnt, rlo);
+        hi = first_above(L.cum, 0, L.cnt, rhi);
+        if ((lo < L.cnt ? lo : L.cnt - 1) == (hi < L.cnt ? hi : L.cnt - 1)) g = lump_group(d, L, ic, lo);
+    }
+    uint32_t e = (uint32_t)hi << 15 | (uint32_t)lo;
+    if (g > 0) {
+        const int lc = t == TAB_L ? ic - 1 : (t == TAB_R ? ic + 1 : ic);
+        int g2 = t != TAB_D ? g : (d.divv[ic - 1] >= 0 ? g + 1 : g - 1);
+        g2 = g2 < 1 ? 1 : (g2 > d.ng ? d.ng : g2);
+        e = BT_PURE | (uint32_t)g | (lc >= 1 && lc <= d.nx ? group_flags(d, g2, lc) : 0u);
+    }
+    d.btab[((size_t)t * d.nx + (ic - 1)) * BT_K + b] = e;
+}
+
 void launch_ddmc_tables(slgpu_ctx *c)
 {
     hipLaunchKernelGGL(k_leakage, dim3(c->nx), dim3(NT), 0, c->stream, c->d);
@@ -721,7 +757,9 @@ void launch_ddmc_tables(slgpu_ctx *c)
         hipLaunchKernelGGL(k_emitprob<false>, dim3(rblocks + c->nx), dim3(RS_THREADS), tiles, c->stream, c->d);
     hipLaunchKernelGGL(k_row_sums, dim3(rblocks, 5), dim3(RS_THREADS), 0, c->stream, c->d);
     const size_t lds = (size_t)(c->ng + c->d.nep) * sizeof(double), answers = BT_ANSWERS;
-    if (lds <= 160000)
+    if (c->nx <= BT_SEARCH_CELLS)
+        hipLaunchKernelGGL(k_bucket_search, dim3(BT_K / 256, c->nx, NTAB), dim3(256), 0, c->stream, c->d);
+    else if (lds <= 160000)
         hipLaunchKernelGGL(k_bucket_tables<true>, dim3(c->nx, NTAB), dim3(1024), lds > answers ? lds : answers,
                            c->stream, c->d);
     else

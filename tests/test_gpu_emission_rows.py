@@ -1,7 +1,8 @@
 """The emission table's bucket maps where its running sums do not rise: lines of negative strength, which
 the line setter takes, leave groups of negative opacity.  A bucket whose two ends are answered alike by
-the plain search holds that answer; whole numbers, so the comparison is exact.  Rows searched in LDS
-and (ng + nep beyond 20000) in global memory, a bin per group and several groups per bin."""
+the plain search holds that answer; whole numbers, so the comparison is exact.  Meshes mapped by plain
+searches (up to 24 cells) and by a block per map, rows in LDS and (ng + nep beyond 20000) in global
+memory, a bin per group and several groups per bin."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 K = 1 << 14
 
 
-@pytest.mark.parametrize("nx,ng,nep", [(2, 60, 8), (3, 500, 22), (2, 3000, 55), (2, 300, 300), (1, 21_000, 145)])
+@pytest.mark.parametrize("nx,ng,nep", [(3, 500, 22), (25, 60, 8), (25, 500, 22), (26, 3000, 55), (25, 300, 300),
+                                       (25, 21_000, 145)])
 @pytest.mark.parametrize("negative", [0.1, 0.3])
 def test_falling_rows(tables, nx, ng, nep, negative):
     from superlite_amd import slgpu as S
